@@ -98,6 +98,9 @@ enum oops_table_column {
   OOPS_TABLE_WIDTH = 40
 };
 
+/* vec_ok: rows of Q, K, V, O and dO start 16-byte aligned, rows of the bias need not (an odd number of keys) */
+#define OOPS_VEC_QKV 2
+
 typedef struct oops_attn_geometry {
   int32_t dtype;       /* OOPS_F32 / OOPS_BF16 / OOPS_F16 for Q, K, V, O, dO */
   int32_t bias_dtype;  /* dtype of the bias: the Q dtype or OOPS_F32 */
@@ -106,7 +109,8 @@ typedef struct oops_attn_geometry {
   int32_t num_samples; /* rows of the table */
   int32_t has_bias;    /* 0/1 */
   int32_t has_mask;    /* 0/1 */
-  int32_t vec_ok;      /* 1 when every row of Q/K/V/O/dO/bias starts 16-byte aligned */
+  int32_t vec_ok;      /* 1 when every row of Q/K/V/O/dO/bias starts 16-byte aligned; OOPS_VEC_QKV when
+                          every row but the bias's does; 0 otherwise */
   float scale;         /* multiplies Q.K before the bias is added */
   int32_t phases;      /* backward kernels to run: OR of OOPS_PHASE_*, 0 = all */
   int32_t force_generic; /* testing: 1 skips the specialised fast kernels, 2 keeps them but

@@ -15,6 +15,7 @@ from pathlib import Path
 LIB_PATH = Path(os.environ.get("OOPS_AMD_LIB") or Path(__file__).resolve().parent / "lib" / "liboops_amd.so")
 
 F32, BF16, F16 = 0, 1, 2
+VEC_QKV = 2  # Geometry.vec_ok: every row 16-byte aligned but the bias's
 BIAS_NONE, BIAS_FULL, BIAS_SHARED = 0, 1, 2
 NOALLOC_SCRATCH_BYTES = 32 << 20
 PHASE_DELTA, PHASE_DQ, PHASE_DKV, PHASE_DBIAS = 1, 2, 4, 8

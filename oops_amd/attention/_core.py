@@ -171,12 +171,14 @@ def device_table(table: Sequence[int], device: torch.device) -> tuple[Tensor, Te
     return host, dev
 
 
-def _vec_ok(table: Sequence[int], tensors: Sequence[Optional[Tensor]], bias: Optional[Tensor]) -> bool:
-    """True when every row of every operand starts on a 16-byte boundary."""
+def _vec_ok(table: Sequence[int], tensors: Sequence[Optional[Tensor]], bias: Optional[Tensor]) -> int:
+    """1 when every row of every operand starts on a 16-byte boundary, ``_lib.VEC_QKV`` when only the
+    bias's rows do not (an odd number of keys), else 0."""
 
-    for t in (*tensors, bias):
+    for t in tensors:
         if t is not None and t.data_ptr() % 16:
-            return False
+            return 0
+    aligned = bias is None or bias.data_ptr() % 16 == 0
     width = _lib.TABLE_WIDTH
     q = tensors[0]
     ce = 16 // q.element_size()
@@ -191,14 +193,14 @@ def _vec_ok(table: Sequence[int], tensors: Sequence[Optional[Tensor]], bias: Opt
     for s in range(len(table) // width):
         row = table[s * width : (s + 1) * width]
         if any(int(row[c]) % ce for c in cols):
-            return False
-        if bias is not None and int(row[_lib.T_B_OFF]) >= 0 and any(int(row[c]) % bce for c in bcols):
-            return False
-    return True
+            return 0
+        if aligned and bias is not None and int(row[_lib.T_B_OFF]) >= 0 and any(int(row[c]) % bce for c in bcols):
+            aligned = False
+    return 1 if aligned else _lib.VEC_QKV
 
 
 def _geometry(q: Tensor, bias: Optional[Tensor], mask: Optional[Tensor], table: Sequence[int],
-              num_heads: int, scale: float, vec_ok: bool) -> tuple[_lib.Geometry, tuple]:
+              num_heads: int, scale: float, vec_ok: int) -> tuple[_lib.Geometry, tuple]:
     host, dev = device_table(table, q.device)
     geo = _lib.Geometry()
     geo.dtype = _DTYPE_CODE[q.dtype]
@@ -208,7 +210,7 @@ def _geometry(q: Tensor, bias: Optional[Tensor], mask: Optional[Tensor], table: 
     geo.num_samples = len(table) // _lib.TABLE_WIDTH
     geo.has_bias = int(bias is not None)
     geo.has_mask = int(mask is not None)
-    geo.vec_ok = int(vec_ok)
+    geo.vec_ok = vec_ok
     geo.scale = float(scale)
     geo.phases = _PHASES
     geo.force_generic = _FORCE_GENERIC

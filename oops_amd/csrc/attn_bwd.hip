@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void attn_dq_kernel(BwdArgs a) {
           BT e[BCE];
         } bu;
         bu.u = make_uint4(0, 0, 0, 0);
-        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, k0 + kc, Lk, vec && (k0 + kc + BCE <= Lk));
+        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, k0 + kc, Lk, a.bias_vec);
 #pragma unroll
         for (int i = 0; i < BCE; i += 4) {
           BT* dst = &b_lds[r * BLD + perm32(kc + i)];
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void attn_dkv_kernel(BwdArgs a) {
           BT e[BCE];
         } bu;
         bu.u = make_uint4(0, 0, 0, 0);
-        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, key0, Lk, vec && (key0 + BCE <= Lk));
+        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, key0, Lk, a.bias_vec);
         const int pos = perm32(r);
 #pragma unroll
         for (int e = 0; e < BCE; ++e) bt_lds[(kc + e) * BLD + pos] = bu.e[e];
@@ -751,8 +751,8 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
   const bool fast = backward_fast_ok(geo, plan);
   const int phases = geo.phases == 0 ? 0xF : geo.phases;
   hipError_t err = hipSuccess;
-  // the fragment-major bias copy feeds the fast dQ and dK/dV kernels
-  const bool use_bf = fast && plan.bias_frag && (phases & (OOPS_PHASE_DQ | OOPS_PHASE_DKV));
+  // the fragment-major bias copy feeds every fast kernel
+  const bool use_bf = fast && plan.bias_frag && (phases & (OOPS_PHASE_DQ | OOPS_PHASE_DKV | OOPS_PHASE_DBIAS));
   if (use_bf) {
     err = launch_bias_frag(geo, plan, bias, bias_frag, stream);
     if (err != hipSuccess) return err;

@@ -25,7 +25,8 @@ namespace oops {
 
 using namespace fast;
 
-template <typename T, int DP, bool HAS_BIAS, int R>
+// XW: the bias weight in two terms (see exact_weight).
+template <typename T, int DP, bool HAS_BIAS, int R, bool XW = false>
 __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -102,6 +103,8 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
   }
   Frag ident[2];
   identity_frags<T>(ident, 1.0f / a.scale, lane);
+  Frag ident_low[2];
+  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
 
   // ---- per-thread staging offsets (bytes); the step adds q0 * stride via soffset
   __amdgpu_buffer_rsrc_t q_rsrc[R], do_rsrc[R], l_rsrc[R], d_rsrc[R];
@@ -213,6 +216,10 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
         if constexpr (HAS_BIAS) {
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][0]), ident[0], sacc);
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][1]), ident[1], sacc);
+          if constexpr (XW) {
+            sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][0]), ident_low[0], sacc);
+            sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][1]), ident_low[1], sacc);
+          }
         }
         f32x16 pacc = *reinterpret_cast<const f32x16*>(&ndlt_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16]);
 #pragma unroll
@@ -292,11 +299,18 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
     const int g = g0 + r;
     T* krow = a.dk ? a.dk + S.k_off + g * S.k_sg + h * S.k_sh + (int64_t)key * S.k_si : nullptr;
     T* vrow = a.dv ? a.dv + S.v_off + g * S.v_sg + h * S.v_sh + (int64_t)key * S.v_si : nullptr;
-    const float ks = kvalid[r] ? a.scale : 0.0f, vs = kvalid[r] ? 1.0f : 0.0f;
 #pragma unroll
     for (int t = 0; t < NDT; ++t) {
-      if (krow) store_tile<T>(krow, t * 32, D, g2, dk[r][t], ks);
-      if (vrow) store_tile<T>(vrow, t * 32, D, g2, dv[r][t], vs);
+      if (wave_masked[r]) {
+        // (a select, not a product with 0: a NaN row leaves masked keys' gradients 0)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          dk[r][t][j] = kvalid[r] ? dk[r][t][j] : 0.0f;
+          dv[r][t][j] = kvalid[r] ? dv[r][t][j] : 0.0f;
+        }
+      }
+      if (krow) store_tile<T>(krow, t * 32, D, g2, dk[r][t], a.scale);
+      if (vrow) store_tile<T>(vrow, t * 32, D, g2, dv[r][t], 1.0f);
     }
   }
 }
@@ -313,14 +327,15 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
 // FULL_DBIAS: some sample has a per-group bias whose dBias = dS is written
 // here.  Both only add code that costs registers when compiled in.  FOLD
 // (bf16, bias, at most kFoldTiles key tiles): the key masks are folded into
-// the bias fragments (fold_bias) instead of selected per score.
+// the bias fragments (fold_bias) instead of selected per score.  XW: the bias
+// weight in two terms (see exact_weight).
 // The lean instances (D <= 32, no per-score mask code, no full dBias) start
 // dP from a register tile of -delta instead of zero (one VALU add less per
 // score) and are built for four waves per SIMD, which the extra 16 registers
 // still fit.
 template <int DP, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD>
 constexpr bool kLeanDq = DP == 32 && (!MASKED_TILES || FOLD) && !FULL_DBIAS;
-template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD>
+template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD, bool XW = false>
 __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ? 4 : OOPS_DQ_OCC)) void attn_dq_fast_kernel(
     BwdArgsT<T, T> a) {
   constexpr bool LEAN = kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD>;
@@ -495,6 +510,8 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
   }
   Frag ident[2];
   identity_frags<T>(ident, 1.0f / a.scale, lane);
+  Frag ident_low[2];
+  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
 
   const T* kbase = a.k + S.k_off + g * S.k_sg + h * S.k_sh;
   const T* vbase = a.v + S.v_off + g * S.v_sg + h * S.v_sh;
@@ -637,6 +654,10 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
         const uint4 b1 = FOLD ? fold_bias(bf[t2][1], fm[t2 * 2 + 1]) : bf[t2][1];
         sacc = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
         sacc = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc);
+        if constexpr (XW) {
+          sacc = E::mma(ident_low[0], __builtin_bit_cast(Frag, b0), sacc);
+          sacc = E::mma(ident_low[1], __builtin_bit_cast(Frag, b1), sacc);
+        }
       } else {
         sacc = f32x16{};
       }
@@ -802,21 +823,30 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
   // bias contribution of this (query, key) block, shared by every group
   f32x16 bacc[2];
   {
-    Frag ident[2];
+    Frag ident[2], ident_low[2];
     identity_frags<T>(ident, 1.0f / a.scale, lane);
+    identity_low_frags<T>(ident_low, a.exact_weight ? 1.0f / a.scale : 1.0f, lane);  // (zeros for weight 1)
+    // (from the fragment-major copy, or from the aligned bias rows when there is none)
     const T* brow = a.bias + S.b_off + h * S.b_sh + (int64_t)q_lane * S.b_si;
+    const int qt = qb * 4 + wave;
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
       bacc[t2] = f32x16{};
+      const int kt = kb * 2 + t2;
+      const T* frag = a.bias_frag + s_idx * a.bf_sample_stride + (((int64_t)h * a.bf_nqt + qt) * a.bf_nkt + kt) * 1024;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const int key = k0 + 32 * t2 + 16 * c + g2 * 8;
         uint4 u = make_uint4(0, 0, 0, 0);
-        if (qv) {
+        if (a.bias_frag != nullptr) {
+          if (qt < a.bf_nqt && kt < a.bf_nkt) u = *reinterpret_cast<const uint4*>(frag + c * 512 + lane * 8);
+        } else if (qv) {
           if (key + 8 <= Lk) u = *reinterpret_cast<const uint4*>(brow + key);
           else u = load16(brow, key, Lk, false);
+          u = finite16<T>(u);
         }
-        bacc[t2] = E::mma(ident[c], __builtin_bit_cast(Frag, finite16<T>(u)), bacc[t2]);
+        bacc[t2] = E::mma(ident[c], __builtin_bit_cast(Frag, u), bacc[t2]);
+        if (a.exact_weight) bacc[t2] = E::mma(ident_low[c], __builtin_bit_cast(Frag, u), bacc[t2]);
       }
     }
   }
@@ -1003,7 +1033,8 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
       for (int j = 0; j < 16; j += 4) {
         const int key = k0 + 32 * t2 + kappa(g2, j);
         if (key + 3 < Lk) {
-          *reinterpret_cast<float4*>(row + key) = make_float4(acc[t2][j], acc[t2][j + 1], acc[t2][j + 2], acc[t2][j + 3]);
+          typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));  // (rows of an odd number of keys)
+          *reinterpret_cast<F4*>(row + key) = (F4){acc[t2][j], acc[t2][j + 1], acc[t2][j + 2], acc[t2][j + 3]};
         } else {
           for (int e = 0; e < 4; ++e)
             if (key + e < Lk) row[key + e] = acc[t2][j + e];
@@ -1020,6 +1051,8 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
 #define OOPS_BWD_FAST_INST(T, DP)                                                \
   template __global__ void attn_dkv_fast_kernel<T, DP, true, 1>(BwdArgsT<T, T>);  \
   template __global__ void attn_dkv_fast_kernel<T, DP, true, 2>(BwdArgsT<T, T>);  \
+  template __global__ void attn_dkv_fast_kernel<T, DP, true, 1, true>(BwdArgsT<T, T>); \
+  template __global__ void attn_dq_fast_kernel<T, DP, true, true, false, false, true>(BwdArgsT<T, T>); \
   template __global__ void attn_dkv_fast_kernel<T, DP, false, 1>(BwdArgsT<T, T>); \
   OOPS_DQ_FAST_INST(T, DP, true)                                                 \
   OOPS_DQ_FAST_INST(T, DP, false)                                                \
@@ -1057,7 +1090,7 @@ hipError_t launch_dkv_fast(const oops_attn_geometry& geo, const Plan& plan, cons
     fill_bwd_args(a, geo, plan, L);
     // OOPS_DKV_ROWS=2: two rows per workgroup share each bias fragment (row-shared
     // biases only); it costs a wave of occupancy and measured slower at the headline shape
-    const bool pair = !rest && OOPS_DKV_ROWS == 2 && a.bias != nullptr && !plan.any_full && plan.dkv_tiles_r2 > 0;
+    const bool pair = !rest && !a.exact_weight && OOPS_DKV_ROWS == 2 && a.bias != nullptr && !plan.any_full && plan.dkv_tiles_r2 > 0;
     a.uniform_tiles = pair ? plan.dkv_uniform_r2 : plan.dkv_uniform;
     a.total_tiles = pair ? plan.dkv_tiles_r2 : plan.dkv_tiles;
     if (rest) {
@@ -1067,7 +1100,9 @@ hipError_t launch_dkv_fast(const oops_attn_geometry& geo, const Plan& plan, cons
     }
     if (a.total_tiles == 0) return hipSuccess;
     const dim3 grid((unsigned)xcd_grid(a.total_tiles, xcd_chunk(a.uniform_tiles)));
-    if (pair)
+    if (a.exact_weight)
+      hipLaunchKernelGGL((attn_dkv_fast_kernel<T, DP, true, 1, true>), grid, dim3(256), 0, stream, a);
+    else if (pair)
       hipLaunchKernelGGL((attn_dkv_fast_kernel<T, DP, true, 2>), grid, dim3(256), 0, stream, a);
     else if (a.bias != nullptr)
       hipLaunchKernelGGL((attn_dkv_fast_kernel<T, DP, true, 1>), grid, dim3(256), 0, stream, a);
@@ -1107,7 +1142,10 @@ hipError_t launch_dq_fast(const oops_attn_geometry& geo, const Plan& plan, const
       if (plan.masked_tiles) by_full(has_bias, std::true_type{});
       else by_full(has_bias, std::false_type{});
     };
-    if (a.bias != nullptr) by_mask(std::true_type{});
+    // (an exact weight comes with shared biases only: no full dBias)
+    if (a.exact_weight)
+      hipLaunchKernelGGL((attn_dq_fast_kernel<T, DP, true, true, false, false, true>), grid, dim3(256), 0, stream, a);
+    else if (a.bias != nullptr) by_mask(std::true_type{});
     else by_mask(std::false_type{});
     return hipGetLastError();
   });

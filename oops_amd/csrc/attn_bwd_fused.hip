@@ -372,9 +372,9 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
           o.w += x.w;
         }
         if (dst != nullptr && red_live[it] && live) {
-          const float f = ok[it] ? sc : 0.0f;
-          *reinterpret_cast<uint2*>(dst + off[it] + goff) =
-              make_uint2(pack2<T>(o.x * f, o.y * f), pack2<T>(o.z * f, o.w * f));
+          // (a select, not a product with 0: a NaN row leaves masked keys' gradients 0)
+          const uint2 r = make_uint2(pack2<T>(o.x * sc, o.y * sc), pack2<T>(o.z * sc, o.w * sc));
+          *reinterpret_cast<uint2*>(dst + off[it] + goff) = ok[it] ? r : make_uint2(0u, 0u);
         }
       }
     }
@@ -584,7 +584,8 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
 }  // namespace
 
 bool dkvb_fused_ok(const oops_attn_geometry& geo, const Plan& plan) {
-  return geo.force_generic == 0 && fast_path_ok(geo, plan) && plan.dp == kCompactRow && plan.all_shared &&
+  // (its registers and LDS have no room for the second term of an exact weight)
+  return geo.force_generic == 0 && !exact_weight(geo) && fast_path_ok(geo, plan) && plan.dp == kCompactRow && plan.all_shared &&
          plan.bias_frag && plan.fused_max_len_q <= kFusedMaxLen && (plan.fused_tiles > 0 || plan.fused_long_tiles > 0);
 }
 

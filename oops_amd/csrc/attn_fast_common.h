@@ -99,6 +99,13 @@ __device__ __forceinline__ void identity_frags(typename Elem<T>::Frag (&id)[2], 
   }
 }
 
+// The identity fragments of the part of weight w that its rounding to T drops
+// (w - T(w), itself rounded to T): with both, the weight has twice T's bits.
+template <typename T>
+__device__ __forceinline__ void identity_low_frags(typename Elem<T>::Frag (&id)[2], float w, int lane) {
+  identity_frags<T>(id, w - Elem<T>::to_f((T)w), lane);
+}
+
 // The identity MFMA that adds the bias multiplies every bias element of a
 // 16-key chunk by the zeros of the other keys' columns, so a non-finite bias
 // element (an additive -inf mask) would make the whole chunk NaN.  Bias
@@ -118,6 +125,29 @@ __device__ __forceinline__ uint32_t finite2(uint32_t d) {
 template <typename T>
 __device__ __forceinline__ uint4 finite16(uint4 u) {
   return make_uint4(finite2<T>(u.x), finite2<T>(u.y), finite2<T>(u.z), finite2<T>(u.w));
+}
+
+// The same for biases that would otherwise take the generic kernels, which
+// add the bias in float32 arithmetic: a row whose kept keys all have a -inf
+// bias is a masked row (output 0), and a NaN or +inf bias at a kept key makes
+// its row NaN.  NaN reads as +max here.  In bfloat16 +-max times a weight of
+// at least 1.0625 overflows to +-inf, which gives both.  A float16 maximum
+// stays finite, so finite float16 elements are clamped to +-60000 (a logit
+// difference of 5504 at least remains: the same softmax) and the forward
+// takes a row maximum beyond +-62750 as a marked element's.
+constexpr float kEdgeLogit = 62750.0f * kLog2e;
+template <typename T>
+__device__ __forceinline__ uint32_t edge1(uint32_t b) {
+  constexpr bool kBf = std::is_same_v<T, __bf16>;
+  constexpr uint32_t kExp = kBf ? 0x7F80u : 0x7C00u, kMax = kBf ? 0x7F7Fu : 0x7BFFu;
+  const uint32_t neg = b & 0x8000u, mag = b & 0x7FFFu;
+  if (mag >= kExp) return mag == kExp ? neg | kMax : kMax;
+  return neg | (!kBf && mag > 0x7B53u ? 0x7B53u : mag);  // (0x7B53: 60000)
+}
+template <typename T>
+__device__ __forceinline__ uint4 edge16(uint4 u) {
+  auto two = [](uint32_t d) { return edge1<T>(d & 0xFFFFu) | (edge1<T>(d >> 16) << 16); };
+  return make_uint4(two(u.x), two(u.y), two(u.z), two(u.w));
 }
 
 // Key masks folded into the bias operand of the identity MFMA (bf16, row-

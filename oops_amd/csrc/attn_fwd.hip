@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(FwdArgs a) {
           BT e[BCE];
         } bu;
         bu.u = make_uint4(0, 0, 0, 0);
-        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, k0 + kc, Lk, vec && (k0 + kc + BCE <= Lk));
+        if (q < Lq) bu.u = load16(bbase + (int64_t)q * S.b_si, k0 + kc, Lk, a.bias_vec);
 #pragma unroll
         for (int i = 0; i < BCE; i += 4) {
           // 4 consecutive keys stay contiguous under perm32
@@ -306,7 +306,10 @@ hipError_t launch_forward(const oops_attn_geometry& geo, const Plan& plan, const
     a.num_samples = geo.num_samples;
     a.num_heads = geo.num_heads;
     a.head_size = geo.head_size;
-    a.vec_ok = geo.vec_ok;
+    a.vec_ok = geo.vec_ok != 0;
+    a.bias_vec = geo.vec_ok == 1;
+    a.lazy = 0.0f;
+    a.edge_bias = 0;
     a.scale = geo.scale;
     if (plan.fwd_tiles > 0) {
       hipLaunchKernelGGL((attn_fwd_kernel<T, BT, DP>), dim3((unsigned)plan.fwd_tiles), dim3(256), 0, stream, a);

@@ -47,8 +47,9 @@ constexpr int kRing = 4;  // K/V tile buffers in LDS
 // out-of-range keys; without it the per-score mask code is not compiled
 // (it costs registers even when never executed).  FOLD (bf16, bias, at most
 // kFoldTiles key tiles): the masks are folded into the bias fragments
-// instead of selected per score.
-template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FOLD>
+// instead of selected per score.  XW: the bias weight in two terms
+// (identity_low_frags; see exact_weight).
+template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FOLD, bool XW = false>
 __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -140,6 +141,8 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
   // identity A-fragments carrying the bias weight 1/scale: MFMA c adds bias keys 16c..16c+15
   Frag ident[2];
   identity_frags<T>(ident, 1.0f / a.scale, lane);
+  Frag ident_low[2];
+  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
 
   // ---- fixed per-lane offsets (bytes) of the direct-to-LDS tile loads:
   // wave w fills rows 16w .. 16w+15 of the K and V tiles; lane l writes slot
@@ -251,6 +254,10 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
         const uint4 b1 = FOLD ? fold_bias(r1, fm[t2 * 2 + 1]) : r1;
         sacc[t2] = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
         sacc[t2] = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
+        if constexpr (XW) {
+          sacc[t2] = E::mma(ident_low[0], __builtin_bit_cast(Frag, b0), sacc[t2]);
+          sacc[t2] = E::mma(ident_low[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
+        }
       } else {
         sacc[t2] = f32x16{};
       }
@@ -309,10 +316,11 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
       mc[t2] = fmaxf(x, sacc[t2][15]);
     }
     float mx = max_halves(fmaxf(mc[0], mc[1])) * c1;
-    const bool grow = mx > m_run + kLazyRescale;
+    const bool grow = mx > m_run + a.lazy;
     if (__any(grow)) {
       const float m_new = grow ? mx : m_run;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      // (1 where the max stays: a row with only -inf logits so far has -inf - -inf there)
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
       m_run = m_new;
       neg_m = m_run == kNegInf ? 0.0f : -m_run;
       l_run *= alpha;
@@ -394,7 +402,17 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 
   // ---- epilogue
   const float l_tot = sum_halves(l_run);
-  const float inv = 1.0f / (l_tot == 0.0f ? 1.0f : l_tot);
+  float inv = 1.0f / (l_tot == 0.0f ? 1.0f : l_tot);
+  float lse = l_tot == 0.0f ? 0.0f : (m_run == kNegInf ? 0.0f : m_run) + __log2f(l_tot);
+  if constexpr (HAS_BIAS && std::is_same_v<T, _Float16>) {
+    if (a.edge_bias) {
+      // only -inf biases at the kept keys: a fully masked row; a NaN or +inf one: NaN (see edge16)
+      if (m_run < -kEdgeLogit) lse = inv = 0.0f;
+      uint32_t nan_bits = 0x7FC00000u;
+      asm volatile("" : "+v"(nan_bits));  // (opaque: this file is compiled without NaN semantics)
+      if (m_run > kEdgeLogit) lse = inv = __builtin_bit_cast(float, nan_bits);
+    }
+  }
   if (qv) {
     const int64_t o_row = S.o_off + g * S.o_sg + h * S.o_sh + (int64_t)q_lane * S.o_si;
     T* orow = a.out + o_row;
@@ -410,16 +428,14 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
       store_tile<T>(orow, t * 32, D, g2, o, 1.0f);
       if (lrow) store_tile<T>(lrow, t * 32, D, g2, r, 1.0f);
     }
-    if (g2 == 0 && a.lse != nullptr) {
-      const float m_use = m_run == kNegInf ? 0.0f : m_run;
-      a.lse[S.l_off + ((int64_t)g * H + h) * Lq + q_lane] = l_tot == 0.0f ? 0.0f : m_use + __log2f(l_tot);
-    }
+    if (g2 == 0 && a.lse != nullptr) a.lse[S.l_off + ((int64_t)g * H + h) * Lq + q_lane] = lse;
   }
 }
 
 #define OOPS_FWD_FAST_INST(T, DP)                                                       \
   template __global__ void attn_fwd_fast_kernel<T, DP, true, false, false>(FwdArgsT<T, T>);  \
   template __global__ void attn_fwd_fast_kernel<T, DP, true, true, false>(FwdArgsT<T, T>);   \
+  template __global__ void attn_fwd_fast_kernel<T, DP, true, true, false, true>(FwdArgsT<T, T>); \
   template __global__ void attn_fwd_fast_kernel<T, DP, false, false, false>(FwdArgsT<T, T>); \
   template __global__ void attn_fwd_fast_kernel<T, DP, false, true, false>(FwdArgsT<T, T>);
 OOPS_FWD_FAST_INST(__bf16, 32)
@@ -431,12 +447,47 @@ OOPS_FWD_FAST_INST(_Float16, 64)
 
 bool fold_masks_ok(const Plan& plan) { return plan.max_len_k <= 64 * kFoldTiles; }
 
-bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan) {
+// Bias rows that are not 16-byte aligned (an odd number of keys) reach the
+// fast kernels only through the fragment-major copy, so every sample's bias
+// must be shared by its rows.  The bias weight 1/scale must be large enough
+// that the largest bfloat16 times it is infinite (see edge16).  Measured at
+// 331 residues, 4 heads of 32, masked, bf16, forward and backward: generic
+// kernels 2304 us, this route 325 us; at 127 MSA rows x 277 tokens, 8 heads,
+// float16, forward: 237 and 54 us.
+static bool unaligned_bias_ok(const oops_attn_geometry& geo, const Plan& plan) {
+  const float w = 1.0f / geo.scale;
+  return plan.all_shared && geo.scale > 0.0f && w >= 1.0625f && w <= 16384.0f;
+}
+
+// The generic kernels, which add the bias in float32, served unaligned bias
+// rows before.  So that no such call loses precision by the faster route, the
+// bias weight keeps at least four bits more than the inputs have (relative
+// error up to 2^-12 in bfloat16, 2^-15 in float16): where one rounding to the
+// input dtype does not (head sizes 24 and 48 in bfloat16, 32 in float16),
+// two more identity MFMAs per score tile add the rounding's rest.
+bool exact_weight(const oops_attn_geometry& geo) {
+  if (!bias_unaligned(geo)) return false;
+  const int drop = geo.dtype == OOPS_F16 ? 13 : 16;  // float32 mantissa bits that T does not have
+  const float w = 1.0f / geo.scale;
+  uint32_t u;
+  __builtin_memcpy(&u, &w, 4);
+  u = (u + (1u << (drop - 1)) - 1u + ((u >> drop) & 1u)) & ~((1u << drop) - 1u);  // nearest even
+  float r;
+  __builtin_memcpy(&r, &u, 4);
+  return !(__builtin_fabsf(r - w) <= w * (geo.dtype == OOPS_F16 ? 0x1p-15f : 0x1p-12f));
+}
+
+bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan) {
   if (geo.force_generic == 1) return false;
   if (geo.dtype == OOPS_F32 || plan.dp > 64 || plan.max_len_k > 64 * kMaxKeyTiles || plan.any_pair_mask ||
       !geo.vec_ok || geo.head_size % 8 != 0 || !plan.offsets_32bit)
     return false;
-  return !(geo.has_bias && geo.bias_dtype != geo.dtype);
+  if (geo.has_bias && geo.bias_dtype != geo.dtype) return false;
+  return !bias_unaligned(geo) || unaligned_bias_ok(geo, plan);
+}
+
+bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan) {
+  return fast_geometry_ok(geo, plan) && (!bias_unaligned(geo) || plan.bias_frag);
 }
 
 // attn_bias_frag_kernel: the fragment-major copy of every shared bias.  For
@@ -446,7 +497,10 @@ bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan) {
 // exactly the bias fragments of the fast kernels' identity MFMAs, so a wave
 // reads a fragment with one contiguous 1 KB load instead of 32 rows of
 // 32 bytes (which the L1 serves one row at a time).  One thread per entry.
-template <typename T>
+// ALIGNED: the bias rows start 16-byte aligned; else their elements are read
+// one by one and non-finite ones are marked so that the kernels treat them as
+// the generic ones do (edge16).
+template <typename T, bool ALIGNED>
 __global__ __launch_bounds__(256) void attn_bias_frag_kernel(const T* __restrict__ bias, T* __restrict__ bf,
                                                              const int64_t* table, int num_samples, int H,
                                                              int nqt, int nkt, int64_t sample_stride) {
@@ -469,14 +523,16 @@ __global__ __launch_bounds__(256) void attn_bias_frag_kernel(const T* __restrict
   const int k = kt * 32 + 16 * c + 8 * (lane >> 5);
   if (S.bias_mode == OOPS_BIAS_SHARED && S.b_off >= 0 && q < S.Lq && k < S.Lk) {
     const T* row = bias + S.b_off + h * S.b_sh + (int64_t)q * S.b_si;
-    if (k + 8 <= S.Lk) {
+    if (ALIGNED && k + 8 <= S.Lk) {
       v = *reinterpret_cast<const uint4*>(row + k);
     } else {
       T e[8];
+#pragma unroll
       for (int j = 0; j < 8; ++j) e[j] = k + j < S.Lk ? row[k + j] : (T)0.0f;
       v = __builtin_bit_cast(uint4, e);
     }
-    v = fast::finite16<T>(v);  // (non-finite elements read as +-max: see finite2)
+    // (non-finite elements read as +-max: see finite2)
+    v = ALIGNED ? fast::finite16<T>(v) : fast::edge16<T>(v);
   }
   const int64_t dst = (int64_t)s * sample_stride + ((((int64_t)h * nqt + qt) * nkt + kt) * 2 + c) * 512 + lane * 8;
   *reinterpret_cast<uint4*>(bf + dst) = v;
@@ -486,14 +542,18 @@ hipError_t launch_bias_frag(const oops_attn_geometry& geo, const Plan& plan, con
                             hipStream_t stream) {
   const int64_t n = (int64_t)geo.num_samples * geo.num_heads * plan.bf_nqt * plan.bf_nkt * 128;
   const dim3 grid((unsigned)((n + 255) / 256));
-  if (geo.dtype == OOPS_BF16)
-    hipLaunchKernelGGL(attn_bias_frag_kernel<__bf16>, grid, dim3(256), 0, stream, static_cast<const __bf16*>(bias),
-                       static_cast<__bf16*>(bf), geo.table_device, geo.num_samples, geo.num_heads, plan.bf_nqt,
-                       plan.bf_nkt, plan.bf_sample_stride);
-  else
-    hipLaunchKernelGGL(attn_bias_frag_kernel<_Float16>, grid, dim3(256), 0, stream,
-                       static_cast<const _Float16*>(bias), static_cast<_Float16*>(bf), geo.table_device,
-                       geo.num_samples, geo.num_heads, plan.bf_nqt, plan.bf_nkt, plan.bf_sample_stride);
+  auto go = [&](auto tag, auto aligned) {
+    using T = typename decltype(tag)::type;
+    hipLaunchKernelGGL((attn_bias_frag_kernel<T, decltype(aligned)::value>), grid, dim3(256), 0, stream,
+                       static_cast<const T*>(bias), static_cast<T*>(bf), geo.table_device, geo.num_samples,
+                       geo.num_heads, plan.bf_nqt, plan.bf_nkt, plan.bf_sample_stride);
+  };
+  auto by_align = [&](auto tag) {
+    if (bias_unaligned(geo)) go(tag, std::false_type{});
+    else go(tag, std::true_type{});
+  };
+  if (geo.dtype == OOPS_BF16) by_align(Tag<__bf16>{});
+  else by_align(Tag<_Float16>{});
   return hipGetLastError();
 }
 
@@ -518,8 +578,12 @@ bool launch_forward_fast(const oops_attn_geometry& geo, const Plan& plan, const 
     a.num_samples = geo.num_samples;
     a.num_heads = geo.num_heads;
     a.head_size = geo.head_size;
-    a.vec_ok = geo.vec_ok;
+    a.vec_ok = geo.vec_ok != 0;
+    a.bias_vec = geo.vec_ok == 1;
     a.scale = geo.scale;
+    // (the generic kernels keep the exact maximum: so does the route that replaces them)
+    a.lazy = bias_unaligned(geo) ? 0.0f : kLazyRescale;
+    a.edge_bias = bias_unaligned(geo);
     a.total_tiles = plan.fwd_tiles;
     a.head_group = head_group(geo);
     a.bias_frag = static_cast<const T*>(bias_frag);
@@ -532,6 +596,11 @@ bool launch_forward_fast(const oops_attn_geometry& geo, const Plan& plan, const 
                                                decltype(fold)::value>),
                          grid, dim3(256), 0, stream, a);
     };
+    if (a.bias != nullptr && exact_weight(geo)) {
+      hipLaunchKernelGGL((attn_fwd_fast_kernel<T, DP, true, true, false, true>), grid, dim3(256), 0, stream, a);
+      *err = hipGetLastError();
+      return;
+    }
     auto by_mask = [&](auto has_bias) {
       if constexpr (decltype(has_bias)::value && std::is_same_v<T, __bf16>) {
         if (plan.masked_tiles && fold_masks_ok(plan)) return go(has_bias, std::true_type{}, std::true_type{});

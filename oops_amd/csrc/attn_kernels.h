@@ -23,8 +23,11 @@ struct FwdArgsT {
   int num_samples;
   int num_heads;
   int head_size;
-  int vec_ok;
+  int vec_ok;    // rows of Q, K and V 16-byte aligned
+  int bias_vec;  // rows of the bias 16-byte aligned
   float scale;
+  float lazy;    // fast kernels: log2 slack of the running max (see kLazyRescale)
+  int edge_bias; // fast kernels: bias_frag marks non-finite float16 elements (see edge16)
   const T* bias_frag;        // fragment-major copy of the shared biases, or nullptr
   int64_t bf_sample_stride;  // elements per sample in bias_frag
   int bf_nqt, bf_nkt;        // 32-query / 32-key tiles per head in bias_frag
@@ -61,7 +64,8 @@ struct BwdArgsT {
   int num_samples;
   int num_heads;
   int head_size;
-  int vec_ok;
+  int vec_ok;    // rows of Q, K, V, O and dO 16-byte aligned
+  int bias_vec;  // rows of the bias 16-byte aligned
   int parts;
   int64_t part_groups;  // > 0: per-sample parts, parts_for(G, part_groups, parts) (fast dBias)
   // > 0: a batch split between the fused dK/dV + dBias kernel (samples with Lq <= fused_max_lq) and the
@@ -77,6 +81,7 @@ struct BwdArgsT {
   int64_t bf_sample_stride;
   int bf_nqt, bf_nkt;
   int delta_in_dq;           // fast dQ kernel computes delta (and stores it) instead of reading it
+  int exact_weight;          // fast kernels: the bias weight in two terms
 };
 
 }  // namespace oops
@@ -174,6 +179,12 @@ struct Plan {
 
 // True when the 16-bit fast kernels serve this geometry (forward and backward).
 bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan);
+// fast_path_ok but for how the bias is read: the fragment-major copy may be planned
+bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan);
+// the bias weight of the identity MFMAs takes two terms (see exact_weight in attn_fwd_fast.hip)
+bool exact_weight(const oops_attn_geometry& geo);
+// bias rows that are not 16-byte aligned: only the fragment-major copy can be read
+inline bool bias_unaligned(const oops_attn_geometry& geo) { return geo.has_bias && geo.vec_ok == OOPS_VEC_QKV; }
 // key masks may be folded into the bias fragments (every sample's keys fit the fold table)
 bool fold_masks_ok(const Plan& plan);
 
@@ -234,7 +245,8 @@ inline void fill_bwd_args(BwdArgsT<T, BT>& a, const oops_attn_geometry& geo, con
   a.num_samples = geo.num_samples;
   a.num_heads = geo.num_heads;
   a.head_size = geo.head_size;
-  a.vec_ok = geo.vec_ok;
+  a.vec_ok = geo.vec_ok != 0;
+  a.bias_vec = geo.vec_ok == 1;
   a.parts = plan.parts;
   a.part_groups = 0;
   a.fused_max_lq = 0;
@@ -248,6 +260,7 @@ inline void fill_bwd_args(BwdArgsT<T, BT>& a, const oops_attn_geometry& geo, con
   a.bf_nqt = plan.bf_nqt;
   a.bf_nkt = plan.bf_nkt;
   a.delta_in_dq = 0;
+  a.exact_weight = geo.has_bias && exact_weight(geo);
 }
 
 bool backward_fast_ok(const oops_attn_geometry& geo, const Plan& plan);

@@ -240,7 +240,7 @@ int make_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
   // fragment-major copy of the shared biases for the fast kernels: one slab
   // of H x ceil(Lq/32) x ceil(Lk/32) x 1024 elements per sample (the largest
   // sample's extent, so a kernel finds its slab from the sample index alone)
-  if (geo->has_bias && plan.any_shared && oops::fast_path_ok(*geo, plan)) {
+  if (geo->has_bias && plan.any_shared && oops::fast_geometry_ok(*geo, plan)) {
     const int64_t nqt = cdiv(plan.max_len_q, 32), nkt = cdiv(plan.max_len_k, 32);
     const int64_t stride = H * nqt * nkt * 1024;
     const size_t bytes = (size_t)stride * (size_t)geo->num_samples * 2;
@@ -279,6 +279,22 @@ size_t parts_bytes(const oops::Plan& plan) {
 size_t workspace_bytes(const oops::Plan& plan) {
   return align256(sizeof(float) * (size_t)plan.lse_extent) + pack_bytes(plan) + compact_bytes(plan) +
          parts_bytes(plan) + align256(plan.bf_bytes);
+}
+
+// The plan of a forward call.  With unaligned bias rows the fast kernel needs
+// the bias copied by a launch of its own, which a small call does not repay:
+// the generic kernel walks a 32-key tile in about 3.3 us, so up to nine of
+// them (with up to three workgroups per CU at a time) end before the host has
+// enqueued the next call.  Measured back to back, generic against fast: 23.7
+// and 27.0 us at 127 residues, 30.2 and 34.8 at 32 MSA rows x 201 tokens, but
+// 40.3 and 27.4 at 151 residues, 42.1 and 34.7 at 385 single tokens.
+int make_forward_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
+  if (int rc = make_plan(geo, plan)) return rc;
+  if (oops::bias_unaligned(*geo) && cdiv(plan.max_len_k, 32) * cdiv(plan.fwd_tiles, 768) <= 9) {
+    plan.bias_frag = false;
+    plan.bf_bytes = 0;
+  }
+  return OOPS_OK;
 }
 
 size_t forward_workspace_bytes(const oops::Plan& plan) { return align256(plan.bf_bytes); }
@@ -404,7 +420,7 @@ const char* oops_last_error(void) { return g_last_error.c_str(); }
 
 size_t oops_attn_forward_workspace_bytes(const oops_attn_geometry* geo) {
   oops::Plan plan;
-  if (make_plan(geo, plan)) return 0;
+  if (make_forward_plan(geo, plan)) return 0;
   return forward_workspace_bytes(plan);
 }
 
@@ -413,7 +429,7 @@ int oops_attn_forward(const oops_attn_geometry* geo, const void* q, const void* 
                       size_t ws_bytes, void* stream) {
   g_last_error.clear();
   oops::Plan plan;
-  if (int rc = make_plan(geo, plan)) return rc;
+  if (int rc = make_forward_plan(geo, plan)) return rc;
   if (int rc = check_forward_pointers(geo, q, k, v, mask, bias, out)) return rc;
   if (int rc = check_workspace(workspace, ws_bytes, forward_workspace_bytes(plan))) return rc;
   return run_forward(geo, plan, q, k, v, mask, bias, out, out_lo, lse, workspace, stream);
@@ -424,7 +440,7 @@ int oops_attn_forward_noalloc(const oops_attn_geometry* geo, const void* q, cons
                               void* stream) {
   g_last_error.clear();
   oops::Plan plan;
-  if (int rc = make_plan(geo, plan)) return rc;
+  if (int rc = make_forward_plan(geo, plan)) return rc;
   size_t need = forward_workspace_bytes(plan);
   if (need > kNoAllocScratchBytes) {
     // The fragment-major bias copy is the only scratch the forward uses, and
