@@ -775,10 +775,21 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
     auto check = [&]() {
       if (err == hipSuccess) err = hipGetLastError();
     };
-    const bool need_dq = dq != nullptr || (a.dbias != nullptr && plan.any_full);
+    const bool f32 = attn_f32_ok(geo, plan);
+    // float32: the shared dBias comes from the dQ kernel (all phases run, or none of it is wanted)
+    const bool both = (phases & OOPS_PHASE_DQ) && (phases & OOPS_PHASE_DBIAS) && a.dbias != nullptr;
+    const bool f32_fused = f32 && plan.f32_fused && both;
+    const bool f32_direct = f32 && plan.f32_direct;
+    const bool need_dq = dq != nullptr || (a.dbias != nullptr && (plan.any_full || f32_fused || f32_direct));
     const bool run_dq = (phases & OOPS_PHASE_DQ) && need_dq && plan.fwd_tiles > 0;
     // the fast dQ kernel computes delta itself when it runs first
-    const bool fused_delta = fast && run_dq;
+    const bool fused_delta = (fast || f32) && run_dq;
+    auto launch_f32 = [&](int phase) {
+      if constexpr (std::is_same_v<T, float>) {
+        a.delta_in_dq = 1;
+        if (err == hipSuccess) err = launch_backward_f32(plan, a, phase, stream);
+      }
+    };
     if ((phases & OOPS_PHASE_DELTA) && !fused_delta) {
       a.uniform_tiles = plan.delta_uniform;
       hipLaunchKernelGGL((attn_delta_kernel<T, BT, DP>), dim3((unsigned)plan.delta_tiles), block, 0, stream, a);
@@ -787,6 +798,8 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
     if (run_dq) {
       if (fast) {
         if (err == hipSuccess) err = launch_dq_fast(geo, plan, L, fused_delta, stream);
+      } else if (f32) {
+        launch_f32(f32_fused ? OOPS_PHASE_DQ | OOPS_PHASE_DBIAS : OOPS_PHASE_DQ);
       } else {
         a.uniform_tiles = plan.fwd_uniform;
         hipLaunchKernelGGL((attn_dq_kernel<T, BT, DP>), dim3((unsigned)plan.fwd_tiles), block, 0, stream, a);
@@ -822,17 +835,23 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
     if ((phases & OOPS_PHASE_DKV) && (dk != nullptr || dv != nullptr) && plan.dkv_tiles > 0) {
       if (fast) {
         if (err == hipSuccess) err = launch_dkv_fast(geo, plan, L, stream);
+      } else if (f32) {
+        launch_f32(OOPS_PHASE_DKV);
       } else {
         a.uniform_tiles = plan.dkv_uniform;
         hipLaunchKernelGGL((attn_dkv_kernel<T, BT, DP>), dim3((unsigned)plan.dkv_tiles), block, 0, stream, a);
         check();
       }
     }
-    if ((phases & OOPS_PHASE_DBIAS) && a.dbias != nullptr && plan.any_shared && plan.sbias_tiles > 0) {
-      if (fast) {
+    if ((phases & OOPS_PHASE_DBIAS) && a.dbias != nullptr && plan.any_shared && plan.sbias_tiles > 0 && !f32_direct) {
+      if (f32_fused) {
+        a.parts = plan.f32_parts;
+      } else if (fast) {
         if (err == hipSuccess) err = launch_dbias_fast(geo, plan, L, stream);
         a.parts = plan.fast_parts;
         a.part_groups = plan.fast_part_groups;
+      } else if (f32) {
+        launch_f32(OOPS_PHASE_DBIAS);
       } else {
         a.uniform_tiles = plan.sbias_uniform;
         hipLaunchKernelGGL((attn_dbias_shared_kernel<T, BT, DP>), dim3((unsigned)plan.sbias_tiles), block, 0,

@@ -311,6 +311,12 @@ hipError_t launch_forward(const oops_attn_geometry& geo, const Plan& plan, const
     a.lazy = 0.0f;
     a.edge_bias = 0;
     a.scale = geo.scale;
+    if constexpr (std::is_same_v<T, float>) {
+      if (plan.fwd_tiles > 0 && attn_f32_ok(geo, plan)) {
+        err = launch_forward_f32(geo, plan, a, stream);
+        return;
+      }
+    }
     if (plan.fwd_tiles > 0) {
       hipLaunchKernelGGL((attn_fwd_kernel<T, BT, DP>), dim3((unsigned)plan.fwd_tiles), dim3(256), 0, stream, a);
       err = hipGetLastError();

@@ -82,6 +82,7 @@ struct BwdArgsT {
   int bf_nqt, bf_nkt;
   int delta_in_dq;           // fast dQ kernel computes delta (and stores it) instead of reading it
   int exact_weight;          // fast kernels: the bias weight in two terms
+  int direct_dbias;          // float32 dQ kernel: shared biases have one group, dBias = dS is written there
 };
 
 }  // namespace oops
@@ -166,9 +167,15 @@ struct Plan {
   int64_t fused_long_uniform = 0;
   bool fused_split = false;                      // some samples too long for it: separate kernels for those
   int64_t dkv_rest_tiles = 0, fast_sbias_rest_tiles = 0;  // the separate kernels' tiles of those samples
+  // float32: dQ + shared dBias in one kernel (128-query blocks x group ranges), or written by the dQ kernel
+  // because every shared bias has a single group
+  bool f32_fused = false, f32_direct = false;
+  int f32_parts = 1;
+  int64_t f32_tiles = 0, f32_uniform = 0;
   bool any_pair_mask = false;                    // a mask that depends on the query
   bool masked_tiles = false;                     // some 64-key tile has masked or out-of-range keys
   bool offsets_32bit = true;                     // every per-(group, head) K/V/bias block < 2 GiB
+  bool q_offsets_32bit = true;                   // the same for Q/O/dO
   int64_t max_len_q = 0, max_len_k = 0;
   // fragment-major copy of the shared biases for the fast kernels (see attn_bias_frag_kernel)
   bool bias_frag = false;
@@ -261,7 +268,16 @@ inline void fill_bwd_args(BwdArgsT<T, BT>& a, const oops_attn_geometry& geo, con
   a.bf_nkt = plan.bf_nkt;
   a.delta_in_dq = 0;
   a.exact_weight = geo.has_bias && exact_weight(geo);
+  a.direct_dbias = 0;
 }
+
+// float32 kernels (attn_f32.hip); phase: OOPS_PHASE_DQ (with a.delta_in_dq also delta), _DKV, _DBIAS, or _DQ | _DBIAS
+// where dqb_f32_ok (plan.f32_fused)
+bool dqb_f32_ok(const oops_attn_geometry& geo, const Plan& plan);
+bool attn_f32_ok(const oops_attn_geometry& geo, const Plan& plan);
+hipError_t launch_forward_f32(const oops_attn_geometry& geo, const Plan& plan, FwdArgsT<float, float>& a,
+                              hipStream_t stream);
+hipError_t launch_backward_f32(const Plan& plan, BwdArgsT<float, float> a, int phase, hipStream_t stream);
 
 bool backward_fast_ok(const oops_attn_geometry& geo, const Plan& plan);
 // rest: only the samples of a split batch that the fused dK/dV + dBias kernel does not serve

@@ -32,6 +32,7 @@ SOURCES = (
     "attn_bwd.hip",
     "attn_bwd_fast.hip",
     "attn_bwd_fused.hip",
+    "attn_f32.hip",
     "gate.hip",
     "trimul.hip",
     "trimul_f32.hip",

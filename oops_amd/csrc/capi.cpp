@@ -39,6 +39,10 @@ constexpr size_t kMaxBiasFragBytes = size_t(1) << 30;
 #endif
 constexpr int64_t kTargetFusedBlocks = OOPS_FUSED_BLOCKS;  // three rounds of one workgroup per CU on 256 CUs
 constexpr int64_t kMinFusedPartGroups = 16;
+#ifndef OOPS_F32_BLOCKS
+#define OOPS_F32_BLOCKS 512
+#endif
+constexpr int64_t kTargetF32Blocks = OOPS_F32_BLOCKS;  // float32 dQ + dBias: two resident workgroups per CU
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -123,6 +127,8 @@ int make_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
       const int64_t kspan = (S.Lk * std::max(S.k_si, S.v_si) + geo->head_size) * elt;
       const int64_t bspan = (S.Lq * std::max<int64_t>(S.b_si, 0) + S.Lk) * elt;
       if (kspan >= lim || bspan >= lim) plan.offsets_32bit = false;
+      const int64_t qspan = (S.Lq * std::max({S.q_si, S.o_si, S.do_si}) + geo->head_size) * elt;
+      if (qspan >= lim) plan.q_offsets_32bit = false;
     }
     if (geo->has_bias && S.b_off >= 0) {
       if (S.bias_mode == OOPS_BIAS_FULL) plan.any_full = true;
@@ -254,6 +260,25 @@ int make_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
     }
   }
   plan.fused_ok = oops::dkvb_fused_ok(*geo, plan);
+  if (geo->dtype == OOPS_F32 && plan.any_shared) {
+    int64_t blocks = 0, first = -1, max_groups = 0;
+    bool uniform = true;
+    for (int s = 0; s < geo->num_samples; ++s) {
+      const Sample& S = tab[s];
+      const int64_t c = H * cdiv(S.Lq, 128);
+      blocks += c;
+      track(c, first, uniform);
+      if (S.bias_mode == OOPS_BIAS_SHARED) max_groups = std::max(max_groups, S.G);
+    }
+    plan.f32_direct = max_groups == 1 && oops::attn_f32_ok(*geo, plan);
+    plan.f32_fused = oops::dqb_f32_ok(*geo, plan);
+    if (plan.f32_fused) {
+      // two workgroups per CU; a part writes a float32 slab of the whole bias, so no more than that
+      plan.f32_parts = (int)std::min<int64_t>({std::max<int64_t>(kTargetF32Blocks / blocks, 1), kMaxParts, min_shared_groups});
+      plan.f32_tiles = blocks * plan.f32_parts;
+      plan.f32_uniform = uniform ? first * plan.f32_parts : 0;
+    }
+  }
   return OOPS_OK;
 }
 
@@ -272,7 +297,7 @@ size_t compact_bytes(const oops::Plan& plan) {
 }
 
 size_t parts_bytes(const oops::Plan& plan) {
-  const int parts = std::max({plan.parts, plan.fast_parts, plan.fused_parts});
+  const int parts = std::max({plan.parts, plan.fast_parts, plan.fused_parts, plan.f32_parts});
   return plan.any_shared && parts > 1 ? align256(sizeof(float) * (size_t)parts * plan.dbias_extent) : 0;
 }
 
