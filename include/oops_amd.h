@@ -236,6 +236,21 @@ typedef struct oops_row_norm_geometry {
 
 int oops_layer_norm_rows_forward(const oops_row_norm_geometry* geo, const void* x, const float* weight,
                                  const float* bias, void* y, float* mean, float* rstd, void* stream);
+/* The same for a pair of n x n cells (geo->rows = n * n) whose normalized rows
+ * sit on an n_pad x n_pad grid: cell i * n + j is row i * n_pad + j of y or
+ * grad_y (the forward writes the other rows of y as zeros).  x, grad_x, mean
+ * and rstd keep the n * n rows.  The forward also writes the grid's float32
+ * mask, mask_pad [n_pad * n_pad]: mask [n * n] (NULL: ones) at the cells, zero
+ * elsewhere.  16-bit rows, widths and strides multiples of
+ * 8 up to 512, 16-byte aligned pointers, n at least four rows per 64 lanes (16
+ * at 128 channels, 32 at 64); OOPS_EINVAL otherwise.  No counterpart in the
+ * reference, whose kernels mask unaligned tiles. */
+int oops_layer_norm_pair_forward(const oops_row_norm_geometry* geo, int64_t n, int64_t n_pad, const void* x,
+                                 const float* weight, const float* bias, const float* mask, void* y, float* mask_pad,
+                                 float* mean, float* rstd, void* stream);
+int oops_layer_norm_pair_backward(const oops_row_norm_geometry* geo, int64_t n, int64_t n_pad, const void* x,
+                                  const float* weight, const float* mean, const float* rstd, const void* grad_y,
+                                  void* grad_x, float* grad_weight_parts, float* grad_bias_parts, void* stream);
 /* Rows of float32 weight/bias gradient partials the backward writes (sum them). */
 size_t oops_layer_norm_rows_parts(const oops_row_norm_geometry* geo);
 /* grad_x (rows of x_row) from grad_y (rows of y_row); weight/bias gradient
@@ -322,6 +337,16 @@ int oops_trimul_output_backward(const oops_trimul_geometry* geo, const void* nor
                                 const void* pair_normalized, const void* output_weight, const void* gate_weight,
                                 const float* output_bias, const float* gate_bias, const void* grad_out,
                                 void* grad_value, void* grad_gate, void* stream);
+/* The same on a padded pair: geo describes the n_pad x n_pad grid (one group),
+ * out and grad_out hold the n x n cells; grad_value and grad_gate are zero at
+ * the other rows.  16-bit, C a multiple of 8, c_row and h_row <= 128. */
+int oops_trimul_output_pair_forward(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                                    const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                    const float* output_bias, const float* gate_bias, void* out, void* stream);
+int oops_trimul_output_pair_backward(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                                     const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                     const float* output_bias, const float* gate_bias, const void* grad_out,
+                                     void* grad_value, void* grad_gate, void* stream);
 
 /* ---- float32 partial sums -------------------------------------------------
  *

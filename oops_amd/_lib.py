@@ -20,7 +20,7 @@ BIAS_NONE, BIAS_FULL, BIAS_SHARED = 0, 1, 2
 NOALLOC_SCRATCH_BYTES = 32 << 20
 PHASE_DELTA, PHASE_DQ, PHASE_DKV, PHASE_DBIAS = 1, 2, 4, 8
 TABLE_WIDTH = 40
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 # geometry table columns (enum oops_table_column)
 (
@@ -47,6 +47,8 @@ EXPORTED_SYMBOLS = (
     "oops_gate_multiply_forward",
     "oops_gate_multiply_backward",
     "oops_layer_norm_rows_forward",
+    "oops_layer_norm_pair_forward",
+    "oops_layer_norm_pair_backward",
     "oops_layer_norm_rows_parts",
     "oops_layer_norm_rows_backward",
     "oops_layer_norm_rows_backward_workspace_bytes",
@@ -60,6 +62,8 @@ EXPORTED_SYMBOLS = (
     "oops_trimul_output_norm_backward",
     "oops_trimul_output_forward",
     "oops_trimul_output_backward",
+    "oops_trimul_output_pair_forward",
+    "oops_trimul_output_pair_backward",
     "oops_trimul_output_grad_parts",
     "oops_trimul_output_grad_products",
     "oops_sum_partials_workspace_bytes",
@@ -194,6 +198,11 @@ def load() -> ctypes.CDLL:
         lib.oops_layer_norm_rows_parts.restype = sz
         lib.oops_layer_norm_rows_backward.argtypes = [rg, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_layer_norm_rows_backward.restype = i32
+        i64 = ctypes.c_int64
+        lib.oops_layer_norm_pair_forward.argtypes = [rg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_layer_norm_pair_forward.restype = i32
+        lib.oops_layer_norm_pair_backward.argtypes = [rg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_layer_norm_pair_backward.restype = i32
         lib.oops_layer_norm_rows_backward_workspace_bytes.argtypes = [rg]
         lib.oops_layer_norm_rows_backward_workspace_bytes.restype = sz
         lib.oops_layer_norm_rows_backward_affine.argtypes = [rg, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
@@ -217,7 +226,10 @@ def load() -> ctypes.CDLL:
         lib.oops_trimul_output_forward.restype = i32
         lib.oops_trimul_output_backward.argtypes = [tg, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_trimul_output_backward.restype = i32
-        i64 = ctypes.c_int64
+        lib.oops_trimul_output_pair_forward.argtypes = [tg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_trimul_output_pair_forward.restype = i32
+        lib.oops_trimul_output_pair_backward.argtypes = [tg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_trimul_output_pair_backward.restype = i32
         lib.oops_trimul_output_grad_parts.argtypes = [tg]
         lib.oops_trimul_output_grad_parts.restype = sz
         lib.oops_trimul_output_grad_products.argtypes = [tg, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, vp]

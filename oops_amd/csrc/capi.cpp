@@ -439,7 +439,7 @@ int run_forward(const oops_attn_geometry* geo, const oops::Plan& plan, const voi
 
 extern "C" {
 
-int oops_abi_version(void) { return 6; }
+int oops_abi_version(void) { return 7; }
 
 const char* oops_last_error(void) { return g_last_error.c_str(); }
 
@@ -564,6 +564,35 @@ int oops_layer_norm_rows_forward(const oops_row_norm_geometry* geo, const void* 
   return gate_launch_result(oops::launch_layer_norm_rows_forward(*geo, x, weight, bias, y, mean, rstd,
                                                                  static_cast<hipStream_t>(stream)),
                             "row LayerNorm forward");
+}
+
+int oops_layer_norm_pair_forward(const oops_row_norm_geometry* geo, int64_t n, int64_t n_pad, const void* x,
+                                 const float* weight, const float* bias, const float* mask, void* y, float* mask_pad,
+                                 float* mean, float* rstd, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_row_norm(geo)) return rc;
+  if (!x || !y || !mask_pad || !mean || !rstd)
+    return fail(OOPS_EINVAL, "x, y, mask_pad, mean and rstd must be non-NULL");
+  if (!oops::layer_norm_pair_ok(*geo, n, n_pad, x, y, nullptr))
+    return fail(OOPS_EINVAL, "not a padded pair that is served (sides %lld and %lld)", n, n_pad);
+  return gate_launch_result(oops::launch_layer_norm_pair_forward(*geo, n, n_pad, x, weight, bias, mask, y, mask_pad, mean,
+                                                                 rstd, static_cast<hipStream_t>(stream)),
+                            "pair LayerNorm forward");
+}
+
+int oops_layer_norm_pair_backward(const oops_row_norm_geometry* geo, int64_t n, int64_t n_pad, const void* x,
+                                  const float* weight, const float* mean, const float* rstd, const void* grad_y,
+                                  void* grad_x, float* grad_weight_parts, float* grad_bias_parts, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_row_norm(geo)) return rc;
+  if (!x || !mean || !rstd || !grad_y || !grad_x)
+    return fail(OOPS_EINVAL, "x, mean, rstd, grad_y and grad_x must be non-NULL");
+  if (!oops::layer_norm_pair_ok(*geo, n, n_pad, x, grad_y, grad_x))
+    return fail(OOPS_EINVAL, "not a padded pair that is served (sides %lld and %lld)", n, n_pad);
+  return gate_launch_result(oops::launch_layer_norm_pair_backward(*geo, n, n_pad, x, weight, mean, rstd, grad_y, grad_x,
+                                                                  grad_weight_parts, grad_bias_parts,
+                                                                  static_cast<hipStream_t>(stream)),
+                            "pair LayerNorm backward");
 }
 
 size_t oops_layer_norm_rows_parts(const oops_row_norm_geometry* geo) {
@@ -721,6 +750,48 @@ int oops_trimul_output_forward(const oops_trimul_geometry* geo, const void* norm
                                                        output_bias, gate_bias, out, nullptr, nullptr, nullptr,
                                                        static_cast<hipStream_t>(stream)),
                             "triangle multiplication output");
+}
+
+static bool output_pair_ok(const oops_trimul_geometry& g, int64_t n, int64_t n_pad) {
+  return oops::trimul_output_w_ok(g) && g.groups == 1 && n > 0 && n_pad > n && g.positions == n_pad * n_pad &&
+         n_pad * n_pad * (int64_t)g.c_row * 2 < (int64_t(1) << 31);
+}
+
+int oops_trimul_output_pair_forward(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                                    const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                    const float* output_bias, const float* gate_bias, void* out, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_trimul(geo)) return rc;
+  if (!normalized || !pair_normalized || !output_weight || !gate_weight || !out)
+    return fail(OOPS_EINVAL, "normalized, pair_normalized, both weights and out must be non-NULL");
+  if (!aligned16(normalized) || !aligned16(pair_normalized) || !aligned16(output_weight) || !aligned16(gate_weight) ||
+      !aligned16(out))
+    return fail(OOPS_EINVAL, "operands must be 16-byte aligned");
+  if (!output_pair_ok(*geo, n, n_pad))
+    return fail(OOPS_EINVAL, "not a padded pair that is served (sides %lld and %lld)", n, n_pad);
+  return gate_launch_result(oops::launch_trimul_output(*geo, normalized, pair_normalized, output_weight, gate_weight,
+                                                       output_bias, gate_bias, out, nullptr, nullptr, nullptr,
+                                                       static_cast<hipStream_t>(stream), n),
+                            "triangle multiplication output");
+}
+
+int oops_trimul_output_pair_backward(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                                     const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                     const float* output_bias, const float* gate_bias, const void* grad_out,
+                                     void* grad_value, void* grad_gate, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_trimul(geo)) return rc;
+  if (!normalized || !pair_normalized || !output_weight || !gate_weight || !grad_out || !grad_value || !grad_gate)
+    return fail(OOPS_EINVAL, "operands and both gradients must be non-NULL");
+  if (!aligned16(normalized) || !aligned16(pair_normalized) || !aligned16(output_weight) || !aligned16(gate_weight) ||
+      !aligned16(grad_out) || !aligned16(grad_value) || !aligned16(grad_gate))
+    return fail(OOPS_EINVAL, "operands must be 16-byte aligned");
+  if (!output_pair_ok(*geo, n, n_pad))
+    return fail(OOPS_EINVAL, "not a padded pair that is served (sides %lld and %lld)", n, n_pad);
+  return gate_launch_result(oops::launch_trimul_output(*geo, normalized, pair_normalized, output_weight, gate_weight,
+                                                       output_bias, gate_bias, nullptr, grad_out, grad_value, grad_gate,
+                                                       static_cast<hipStream_t>(stream), n),
+                            "triangle multiplication output backward");
 }
 
 int oops_trimul_output_backward(const oops_trimul_geometry* geo, const void* normalized,

@@ -34,6 +34,7 @@
 // v_permlane32_swap so each lane stores 16 consecutive channels of its token.
 // The backward recomputes both projections and writes the two gradients.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "attn_fast_common.h"
@@ -105,7 +106,17 @@ struct RowNormArgs {
   int64_t rows, x_row, y_row;
   int width, lpr;
   float eps;
+  int n, pad;  // PAD: x rows are the cells of an n x n pair, y (dy) rows those of an (n + pad) x (n + pad) one
+  const float* mask;  // PAD, forward: the pair's mask (or nullptr: ones) goes to mask_pad, zero past the pair
+  float* mask_pad;
 };
+
+// Padded pairs: a 16-bit pair whose side n is no multiple of 8 runs on a side
+// n + pad that is one.  Only the input LayerNorm (cell i n + j of the pair is
+// row i (n + pad) + j of xn, the other rows zero) and the output projection
+// (the reverse) know both sides; everything between them works on the padded
+// one with a zero mask there, so that factor rows, GEMM operands and norm
+// tiles are 16-byte aligned.
 
 template <typename T, int CH, bool VEC>
 __device__ __forceinline__ void load_chunks(const T* row, bool valid, int width, int lpr, int sub, float (&x)[CH][8]) {
@@ -159,7 +170,7 @@ __device__ __forceinline__ float group_sum(float s, int lpr) {
 #define OOPS_ROW_U 4
 #endif
 constexpr int kRowU = OOPS_ROW_U;
-template <typename T, int CH>
+template <typename T, int CH, bool PAD>
 __device__ __forceinline__ void row_norm_forward_pipelined(const RowNormArgs& a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lpr = a.lpr, rpw = 64 / lpr;
@@ -198,8 +209,10 @@ __device__ __forceinline__ void row_norm_forward_pipelined(const RowNormArgs& a)
       for (int c = 0; c < CH; ++c) cur[u][c] = raw[u][c];
     load_group(base + gstep, raw);  // the next group (out of range past the rows: no request)
     const int n = group_rows(base);
-    const __amdgpu_buffer_rsrc_t yr =
-        make_rsrc(static_cast<T*>(a.y) + base * a.y_row, (uint32_t)((int64_t)n * a.y_row * 2));
+    // PAD: the group's first cell is (i0, j0); a group is shorter than a pair row, so it crosses at most one
+    const uint32_t i0 = PAD ? (uint32_t)base / (uint32_t)a.n : 0u, j0 = PAD ? (uint32_t)base - i0 * (uint32_t)a.n : 0u;
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(static_cast<T*>(a.y) + (base + (PAD ? (int64_t)i0 * a.pad : 0)) * a.y_row,
+                                                (uint32_t)((int64_t)(n + (PAD ? a.pad : 0)) * a.y_row * 2));
     const __amdgpu_buffer_rsrc_t mr = make_rsrc(a.mean + base, (uint32_t)(n * 4));
     const __amdgpu_buffer_rsrc_t sr = make_rsrc(a.rstd + base, (uint32_t)(n * 4));
 #pragma unroll
@@ -231,19 +244,36 @@ __device__ __forceinline__ void row_norm_forward_pipelined(const RowNormArgs& a)
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = col + e < W ? (x[c][e] - mean) * rstd * wv[c][e] + bv[c][e] : 0.f;
-        buffer_store16(yr, r < n && col < a.y_row ? (uint32_t)((r * a.y_row + col) * 2) : kOut, pack8<T>(o));
+        const int yo = PAD && j0 + r >= (uint32_t)a.n ? r + a.pad : r;
+        buffer_store16(yr, r < n && col < a.y_row ? (uint32_t)((yo * a.y_row + col) * 2) : kOut, pack8<T>(o));
       }
       const uint32_t so = r < n && sub == 0 ? (uint32_t)(r * 4) : kOut;
       buffer_store4(mr, so, mean);
       buffer_store4(sr, so, rstd);
+      if constexpr (PAD) {
+        if (r < n && sub == 0) {
+          const int64_t row = base + r;
+          a.mask_pad[row + (int64_t)(i0 + (j0 + r >= (uint32_t)a.n)) * a.pad] = a.mask != nullptr ? a.mask[row] : 1.0f;
+        }
+      }
+    }
+  }
+  if constexpr (PAD) {
+    // the padding rows: the ends of the n pair rows, then the last pad pair rows
+    const int64_t ends = (int64_t)a.n * a.pad, all = ends + (int64_t)a.pad * (a.n + a.pad);
+    for (int64_t k = ((int64_t)blockIdx.x * 4 + wave) * rpw + rw; k < all; k += (int64_t)gridDim.x * 4 * rpw) {
+      const int64_t row = k < ends ? (k / a.pad + 1) * a.n + k : (int64_t)a.n * a.n + k;
+      if (sub * 8 < a.y_row) *reinterpret_cast<uint4*>(static_cast<T*>(a.y) + row * a.y_row + sub * 8) = make_uint4(0, 0, 0, 0);
+      if (sub == 0) a.mask_pad[row] = 0.0f;
     }
   }
 }
 
-template <typename T, int CH, bool VEC>
+template <typename T, int CH, bool VEC, bool PAD = false>
 __global__ __launch_bounds__(256) void row_norm_forward_kernel(RowNormArgs a) {
+  static_assert(!PAD || (VEC && sizeof(T) == 2 && CH == 1), "padded pairs: one 16-byte chunk per lane");
   if constexpr (VEC && sizeof(T) == 2 && CH <= 2) {
-    row_norm_forward_pipelined<T, CH>(a);
+    row_norm_forward_pipelined<T, CH, PAD>(a);
     return;
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -302,7 +332,7 @@ __global__ __launch_bounds__(256) void row_norm_forward_kernel(RowNormArgs a) {
   }
 }
 
-template <typename T, int CH, bool VEC>
+template <typename T, int CH, bool VEC, bool PAD = false>
 __global__ __launch_bounds__(256) void row_norm_backward_kernel(RowNormArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lpr = a.lpr, rpw = 64 / lpr;
@@ -323,7 +353,8 @@ __global__ __launch_bounds__(256) void row_norm_backward_kernel(RowNormArgs a) {
     const int64_t rr = rv ? row : 0;
     float x[CH][8], g[CH][8];
     load_chunks<T, CH, VEC>(static_cast<const T*>(a.x) + rr * a.x_row, rv, W, lpr, sub, x);
-    load_chunks<T, CH, VEC>(static_cast<const T*>(a.dy) + rr * a.y_row, rv, W, lpr, sub, g);
+    const int64_t dr = PAD ? rr + (int64_t)((uint32_t)rr / (uint32_t)a.n) * a.pad : rr;
+    load_chunks<T, CH, VEC>(static_cast<const T*>(a.dy) + dr * a.y_row, rv, W, lpr, sub, g);
     const float mean = rv ? a.mean[rr] : 0.f, rstd = rv ? a.rstd[rr] : 0.f;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -1553,6 +1584,7 @@ struct OutArgs {
   int64_t rows, c_row, h_row, tiles;
   int C, cblocks;
   int tpw;  // W-resident form: token tiles per workgroup
+  int n, pad;  // PAD: out / grad_out rows are the cells of an n x n pair, the other rows of the padded one
 };
 
 constexpr int kOM = 128;  // tokens per workgroup
@@ -1777,7 +1809,7 @@ __global__ __launch_bounds__(256) void trimul_output_kernel(OutArgs a) {
 #ifndef OOPS_OUTPUT_WGS
 #define OOPS_OUTPUT_WGS 512
 #endif
-template <typename T, bool BWD>
+template <typename T, bool BWD, bool PAD>
 __global__ __launch_bounds__(256, 2) void trimul_output_w_kernel(OutArgs a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -1853,16 +1885,28 @@ __global__ __launch_bounds__(256, 2) void trimul_output_w_kernel(OutArgs a) {
     const int nrows = (int)(left < kOM ? left : kOM);
     const bool rv = wave * 32 + lq < nrows;
     const uint32_t row_lane = (uint32_t)(wave * 32 + lq);
+    // the lane's row of out / grad_out, counted from row u0 (PAD: from the start of the tile's first pair row)
+    int64_t u0 = r0, u_rows = nrows;
+    uint32_t u_lane = row_lane;
+    bool uv = rv;
+    if constexpr (PAD) {
+      const uint32_t np = (uint32_t)(a.n + a.pad), p0 = (uint32_t)r0, i0 = p0 / np, p = p0 + row_lane, i = p / np, j = p - i * np;
+      u0 = (int64_t)i0 * a.n;
+      u_rows = (int64_t)a.n * a.n - u0;
+      u_lane = (i - i0) * (uint32_t)a.n + j;
+      uv = rv && i < (uint32_t)a.n && j < (uint32_t)a.n;
+      if (u_rows < 0) u_rows = 0;
+    }
     // BWD: grad_out of the lane's 16 post-swap channels n .. n + 15 of each tile t
     uint4 gin[2][2];
     if constexpr (BWD) {
-      const __amdgpu_buffer_rsrc_t gr = make_rsrc(static_cast<const T*>(a.gout) + r0 * C, (uint32_t)((int64_t)nrows * C * 2));
+      const __amdgpu_buffer_rsrc_t gr = make_rsrc(static_cast<const T*>(a.gout) + u0 * C, (uint32_t)(u_rows * C * 2));
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
           const int n = c0 + 32 * t + 16 * g2 + 8 * hh;
-          gin[t][hh] = buffer_load16(gr, rv && n < C ? (row_lane * C + n) * 2 : kOut);
+          gin[t][hh] = buffer_load16(gr, uv && n < C ? (u_lane * C + n) * 2 : kOut);
         }
       // keeps these loads ahead of the MFMAs (the compiler would sink them to their first use)
       asm volatile("" ::: "memory");
@@ -1892,8 +1936,8 @@ __global__ __launch_bounds__(256, 2) void trimul_output_w_kernel(OutArgs a) {
     // ---- epilogue: lane (lq, g2) of tile t holds channels c0 + 32t + 8q + 4g2 + i of its token
     const int cr = (int)a.c_row;
     const __amdgpu_buffer_rsrc_t o0 = make_rsrc(
-        BWD ? static_cast<void*>(static_cast<T*>(a.gval) + r0 * cr) : static_cast<void*>(static_cast<T*>(a.out) + r0 * C),
-        (uint32_t)((int64_t)nrows * (BWD ? cr : C) * 2));
+        BWD ? static_cast<void*>(static_cast<T*>(a.gval) + r0 * cr) : static_cast<void*>(static_cast<T*>(a.out) + u0 * C),
+        BWD ? (uint32_t)((int64_t)nrows * cr * 2) : (uint32_t)(u_rows * C * 2));
     const __amdgpu_buffer_rsrc_t o1 =
         make_rsrc(BWD ? static_cast<T*>(a.ggate) + r0 * cr : nullptr, BWD ? (uint32_t)((int64_t)nrows * cr * 2) : 0u);
 #pragma unroll
@@ -1921,9 +1965,9 @@ __global__ __launch_bounds__(256, 2) void trimul_output_w_kernel(OutArgs a) {
         }
         uint4 lo, hi;
         trade16(p, lo, hi);
-        const uint32_t off = rv && n < C ? (row_lane * C + n) * 2 : kOut;
+        const uint32_t off = uv && n < C ? (u_lane * C + n) * 2 : kOut;
         buffer_store16(o0, off, lo);
-        buffer_store16(o0, rv && n + 8 < C ? off + 16 : kOut, hi);
+        buffer_store16(o0, uv && n + 8 < C ? off + 16 : kOut, hi);
       } else {
         const uint4 lo = gin[t][0], hi = gin[t][1];
         const auto y0 = __builtin_amdgcn_permlane32_swap(lo.x, lo.z, false, false);
@@ -2214,6 +2258,51 @@ hipError_t run_rows(const oops_row_norm_geometry& g, bool backward, RowNormArgs&
 }
 }  // namespace
 
+// The LayerNorms of a padded pair (n x n cells, n_pad x n_pad rows of y or
+// grad_y): 16-bit rows of at most 512 channels in the vector layout.
+bool layer_norm_pair_ok(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x, const void* y,
+                        const void* dx) {
+  const void* ptrs[] = {x, y, dx};
+  const RowPlan pl = row_plan(g, true, ptrs, 3);
+  // (a wave's group of kRowU sets of 64 / lpr rows may cross one pair row, not two)
+  return g.dtype != OOPS_F32 && pl.vec && pl.ch == 1 && n >= kRowU * (64 / pl.lpr) && n_pad > n && g.rows == n * n &&
+         n_pad * n_pad < (int64_t(1) << 31);
+}
+hipError_t launch_layer_norm_pair_forward(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x,
+                                          const float* weight, const float* bias, const float* mask, void* y,
+                                          float* mask_pad, float* mean, float* rstd, hipStream_t stream) {
+  RowNormArgs a{};
+  a.x = x, a.w = weight, a.b = bias, a.y = y, a.mean = mean, a.rstd = rstd, a.mask = mask, a.mask_pad = mask_pad;
+  a.rows = g.rows, a.x_row = g.x_row, a.y_row = g.y_row, a.width = g.width, a.eps = g.eps;
+  a.n = (int)n, a.pad = (int)(n_pad - n);
+  const void* ptrs[] = {x, y};
+  const RowPlan pl = row_plan(g, false, ptrs, 2);
+  a.lpr = pl.lpr;
+  return by_half(g.dtype, [&](auto tag) -> hipError_t {
+    using T = decltype(tag);
+    hipLaunchKernelGGL((row_norm_forward_kernel<T, 1, true, true>), dim3(pl.blocks), dim3(256), 0, stream, a);
+    return hipGetLastError();
+  });
+}
+hipError_t launch_layer_norm_pair_backward(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x,
+                                           const float* weight, const float* mean, const float* rstd,
+                                           const void* grad_y, void* grad_x, float* grad_weight_parts,
+                                           float* grad_bias_parts, hipStream_t stream) {
+  RowNormArgs a{};
+  a.x = x, a.w = weight, a.mean = const_cast<float*>(mean), a.rstd = const_cast<float*>(rstd);
+  a.dy = grad_y, a.dx = grad_x, a.dw = grad_weight_parts, a.db = grad_bias_parts;
+  a.rows = g.rows, a.x_row = g.x_row, a.y_row = g.y_row, a.width = g.width, a.eps = g.eps;
+  a.n = (int)n, a.pad = (int)(n_pad - n);
+  const void* ptrs[] = {x, grad_y, grad_x};
+  const RowPlan pl = row_plan(g, true, ptrs, 3);
+  a.lpr = pl.lpr;
+  return by_half(g.dtype, [&](auto tag) -> hipError_t {
+    using T = decltype(tag);
+    hipLaunchKernelGGL((row_norm_backward_kernel<T, 1, true, true>), dim3(pl.blocks), dim3(256), 0, stream, a);
+    return hipGetLastError();
+  });
+}
+
 hipError_t launch_layer_norm_rows_forward(const oops_row_norm_geometry& g, const void* x, const float* weight,
                                           const float* bias, void* y, float* mean, float* rstd, hipStream_t stream) {
   RowNormArgs a{};
@@ -2431,10 +2520,15 @@ hipError_t launch_trimul_output_norm_backward(const oops_trimul_geometry& g, con
   return run_out_norm(g, a, true, stream);
 }
 
+// the W-resident gated output kernel serves these widths
+bool trimul_output_w_ok(const oops_trimul_geometry& g) {
+  return g.dtype != OOPS_F32 && g.h_row <= 2 * kOK && g.c_row <= 2 * kOK && g.channels % 8 == 0;
+}
+
 hipError_t launch_trimul_output(const oops_trimul_geometry& g, const void* normalized, const void* pair_normalized,
                                 const void* output_weight, const void* gate_weight, const float* output_bias,
                                 const float* gate_bias, void* out, const void* grad_out, void* grad_value,
-                                void* grad_gate, hipStream_t stream) {
+                                void* grad_gate, hipStream_t stream, int64_t n) {
   if (g.dtype == OOPS_F32)
     return launch_trimul_output_f32(g, normalized, pair_normalized, output_weight, gate_weight, output_bias,
                                     gate_bias, out, grad_out, grad_value, grad_gate, stream);
@@ -2446,7 +2540,7 @@ hipError_t launch_trimul_output(const oops_trimul_geometry& g, const void* norma
   const int64_t tiles = (a.rows + kOM - 1) / kOM * a.cblocks;
   if (tiles == 0) return hipSuccess;
   const bool bwd = grad_out != nullptr;
-  if (g.h_row <= 2 * kOK && g.c_row <= 2 * kOK && g.channels % 8 == 0) {
+  if (trimul_output_w_ok(g)) {
     const int64_t tiles_m = (a.rows + kOM - 1) / kOM;
     const int64_t runs = std::max<int64_t>(1, OOPS_OUTPUT_WGS / a.cblocks);
     a.tpw = (int)((tiles_m + runs - 1) / runs);
@@ -2454,10 +2548,14 @@ hipError_t launch_trimul_output(const oops_trimul_geometry& g, const void* norma
     const dim3 wgrid((unsigned)xcd_grid(a.tiles, 0));
     return by_half(g.dtype, [&](auto tag) -> hipError_t {
       using T = decltype(tag);
-      if (bwd)
-        hipLaunchKernelGGL((trimul_output_w_kernel<T, true>), wgrid, dim3(256), 0, stream, a);
-      else
-        hipLaunchKernelGGL((trimul_output_w_kernel<T, false>), wgrid, dim3(256), 0, stream, a);
+      auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, wgrid, dim3(256), 0, stream, a); };
+      if (n > 0) {
+        a.n = (int)n;
+        a.pad = (int)(std::llround(std::sqrt((double)g.positions)) - n);
+        bwd ? go(trimul_output_w_kernel<T, true, true>) : go(trimul_output_w_kernel<T, false, true>);
+      } else {
+        bwd ? go(trimul_output_w_kernel<T, true, false>) : go(trimul_output_w_kernel<T, false, false>);
+      }
       return hipGetLastError();
     });
   }

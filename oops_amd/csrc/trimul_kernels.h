@@ -33,7 +33,19 @@ int64_t trimul_output_norm_parts(const oops_trimul_geometry& g);
 hipError_t launch_trimul_output(const oops_trimul_geometry& g, const void* normalized, const void* pair_normalized,
                                 const void* output_weight, const void* gate_weight, const float* output_bias,
                                 const float* gate_bias, void* out, const void* grad_out, void* grad_value,
-                                void* grad_gate, hipStream_t stream);
+                                void* grad_gate, hipStream_t stream, int64_t n = 0);
+bool trimul_output_w_ok(const oops_trimul_geometry& g);
+
+// padded pairs (n x n cells on an n_pad x n_pad grid; n in launch_trimul_output)
+bool layer_norm_pair_ok(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x, const void* y,
+                        const void* dx);
+hipError_t launch_layer_norm_pair_forward(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x,
+                                          const float* weight, const float* bias, const float* mask, void* y,
+                                          float* mask_pad, float* mean, float* rstd, hipStream_t stream);
+hipError_t launch_layer_norm_pair_backward(const oops_row_norm_geometry& g, int64_t n, int64_t n_pad, const void* x,
+                                           const float* weight, const float* mean, const float* rstd,
+                                           const void* grad_y, void* grad_x, float* grad_weight_parts,
+                                           float* grad_bias_parts, hipStream_t stream);
 
 // the output projection's gradient products for C = H = 128, 16-bit (oops_trimul_output_grad_products)
 bool trimul_output_grad_supported(const oops_trimul_geometry& g);

@@ -24,6 +24,7 @@ contraction.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import List, Literal, Optional, Sequence, Tuple
 
 import torch
@@ -248,6 +249,8 @@ def _long_k_partials(a: Tensor, b: Tensor) -> Tensor:
     chunks = min(64, k // 1024)
     if chunks < 2:
         return a.float().mm(b.float())[None]
+    # (a chunk count that divides K saves the remainder's products and their concatenation)
+    chunks = next((c for c in range(chunks, chunks // 2, -1) if k % c == 0), chunks)
     main = k // chunks * chunks
     step = main // chunks
     a_c = a[:, :main].unflatten(1, (chunks, step)).transpose(0, 1)  # (chunks, M, step), strided view
@@ -329,6 +332,44 @@ def _contract(factors: Tensor, out: Tensor, blocks, direction: str, grad: bool =
             out[1, :, :, cells].copy_(d_right.view(G, H, n * n))
 
 
+# below this side the host's time covers either way's GPU time (padded against plain kernels, bf16, C = H = 128,
+# mask and biases: forward 141 and 139 us at 101 residues, 140 and 210 at 301, 245 and 506 at 509; forward +
+# backward 997 and 1909 us at 509)
+PAD_MIN_SIDE = 96
+
+
+def _padded_side(n: int, grouped: Tensor, hidden: int) -> int:
+    """The side on which an ``n x n`` 16-bit pair is worked: ``n`` rounded up to a multiple of 8, so that
+    factor rows, contraction operands and norm tiles are 16-byte aligned, where the kernels that know both
+    sides serve the widths; else ``n``."""
+
+    c = grouped.shape[2]
+    if (n % 8 == 0 or n < PAD_MIN_SIDE or grouped.shape[0] != 1 or grouped.dtype not in _KERNEL_DTYPES or c % 8
+            or c > 128 or c < 32 or hidden not in (32, 64, 128) or n > 2048):  # fmt: skip
+        return n
+    return _round8(n)
+
+
+def _sides(pair: Tensor, blocks: List[int]) -> Tuple[int, int]:
+    """(n, padded side) of a padded pair, or (0, 0): a single block larger than the pair's cells."""
+
+    if len(blocks) != 2 or blocks[1] * blocks[1] == pair.shape[1]:
+        return 0, 0
+    return math.isqrt(pair.shape[1]), blocks[1]
+
+
+def _aligned(t: Tensor) -> Tensor:
+    """``t`` (contiguous) on a 16-byte boundary, which the padded-pair kernels need."""
+
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _cells(pair: Tensor, blocks: List[int]) -> int:
+    """Pair cells per group the pipeline works on (those of the padded side)."""
+
+    return blocks[1] * blocks[1] if len(blocks) == 2 else pair.shape[1]
+
+
 def _pairs(blocks: List[int]):
     return [(blocks[i], blocks[i + 1]) for i in range(0, len(blocks), 2)]
 
@@ -345,27 +386,41 @@ def _small_views(small: Tensor, spans: List[int]) -> List[Optional[Tensor]]:
 
 def _forward_impl(pair: Tensor, mask: Optional[Tensor], w_cat: Tensor, wo: Tensor, wog: Tensor, small: Tensor,
                   spans: List[int], blocks: List[int], direction: str, eps_in: float, eps_out: float):
-    """Forward on prepared operands: pair (G, P, C); float32 mask (G, P); w_cat [4H][c_row]; wo [C][h_row];
+    """Forward on prepared operands: pair (G, P, C); float32 mask (G, P); a padded pair's blocks are (0, side); w_cat [4H][c_row]; wo [C][h_row];
     wog [C][c_row]; the float32 biases and LayerNorm affines in ``small`` (``spans``).  Returns (out, xn,
-    mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out); all but ``out`` are kept for the backward."""
+    mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out, a padded pair's mask or empty); all but ``out``
+    are kept for the backward."""
 
     b_cat, bo, bog, in_w, in_b, on_w, on_b = _small_views(small, spans)
     lib = _lib.load()
-    G, P, C = pair.shape
+    G, rows, C = pair.shape
     H = w_cat.shape[0] // 4
+    n, side = _sides(pair, blocks)
+    P = _cells(pair, blocks)
     R = G * P
     dtype, dev = pair.dtype, pair.device
     geo = _geometry(pair, H, mask is not None, eps_out)
+    geo.positions = P
     cp, hp = geo.c_row, geo.h_row
     stream = _stream(dev)
     with torch.cuda.device(dev):
         xn = torch.empty(R, cp, dtype=dtype, device=dev)
-        mean_in = torch.empty(R, dtype=torch.float32, device=dev)
+        mean_in = torch.empty(G * rows, dtype=torch.float32, device=dev)
         rstd_in = torch.empty_like(mean_in)
-        rg = _row_geometry(dtype, R, C, C, cp, eps_in)
-        _lib.check(lib.oops_layer_norm_rows_forward(ctypes.byref(rg), _ptr(pair), _ptr(in_w), _ptr(in_b), _ptr(xn),
-                                                    _ptr(mean_in), _ptr(rstd_in), stream),
-                   "triangle_multiplication input LayerNorm")  # fmt: skip
+        rg = _row_geometry(dtype, G * rows, C, C, cp, eps_in)
+        mask_pad = torch.empty(R if n else 0, dtype=torch.float32, device=dev)
+        if n:
+            pair = _aligned(pair)
+            _lib.check(lib.oops_layer_norm_pair_forward(ctypes.byref(rg), n, side, _ptr(pair), _ptr(in_w), _ptr(in_b),
+                                                        _ptr(mask), _ptr(xn), _ptr(mask_pad), _ptr(mean_in),
+                                                        _ptr(rstd_in), stream),
+                       "triangle_multiplication input LayerNorm")  # fmt: skip
+            mask = mask_pad
+            geo.has_mask = 1
+        else:
+            _lib.check(lib.oops_layer_norm_rows_forward(ctypes.byref(rg), _ptr(pair), _ptr(in_w), _ptr(in_b), _ptr(xn),
+                                                        _ptr(mean_in), _ptr(rstd_in), stream),
+                       "triangle_multiplication input LayerNorm")  # fmt: skip
         factors = torch.empty(2, G, H, P, dtype=dtype, device=dev)
         _lib.check(lib.oops_trimul_factors_forward(ctypes.byref(geo), _ptr(xn), _ptr(w_cat), _ptr(b_cat),
                                                    _ptr(mask), _ptr(factors), stream),
@@ -378,11 +433,12 @@ def _forward_impl(pair: Tensor, mask: Optional[Tensor], w_cat: Tensor, wo: Tenso
         _lib.check(lib.oops_trimul_output_norm_forward(ctypes.byref(geo), _ptr(combined), _ptr(on_w), _ptr(on_b),
                                                        _ptr(nrm), _ptr(mean_out), _ptr(rstd_out), stream),
                    "triangle_multiplication output LayerNorm")  # fmt: skip
-        out = torch.empty(G, P, C, dtype=dtype, device=dev)
-        _lib.check(lib.oops_trimul_output_forward(ctypes.byref(geo), _ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog),
-                                                  _ptr(bo), _ptr(bog), _ptr(out), stream),
+        out = torch.empty(G, rows, C, dtype=dtype, device=dev)
+        ptrs = (_ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog), _ptr(bo), _ptr(bog), _ptr(out), stream)
+        _lib.check(lib.oops_trimul_output_pair_forward(ctypes.byref(geo), n, side, *ptrs) if n else
+                   lib.oops_trimul_output_forward(ctypes.byref(geo), *ptrs),
                    "triangle_multiplication output")  # fmt: skip
-    return out, xn, mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out
+    return out, xn, mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out, mask_pad
 
 
 @torch.library.custom_op("oops_amd::trimul_forward", mutates_args=(), device_types="cuda")
@@ -398,25 +454,27 @@ def trimul_forward(
     direction: str,
     eps_in: float,
     eps_out: float,
-) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
+) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     return _forward_impl(pair, mask, w_cat, wo, wog, small, spans, blocks, direction, eps_in, eps_out)
 
 
 @trimul_forward.register_fake
 def _(pair, mask, w_cat, wo, wog, small, spans, blocks, direction, eps_in, eps_out):
-    G, P, C = pair.shape
+    G, rows, C = pair.shape
     H = w_cat.shape[0] // 4
+    P = _cells(pair, blocks)
     R = G * P
     f32 = dict(dtype=torch.float32, device=pair.device)
-    return (pair.new_empty(G, P, C), pair.new_empty(R, w_cat.shape[1]), pair.new_empty(R, **f32),
-            pair.new_empty(R, **f32), pair.new_empty(2, G, H, P), pair.new_empty(G, H, P),
-            pair.new_empty(R, wo.shape[1]), pair.new_empty(R, **f32), pair.new_empty(R, **f32))  # fmt: skip
+    return (pair.new_empty(G, rows, C), pair.new_empty(R, w_cat.shape[1]), pair.new_empty(G * rows, **f32),
+            pair.new_empty(G * rows, **f32), pair.new_empty(2, G, H, P), pair.new_empty(G, H, P),
+            pair.new_empty(R, wo.shape[1]), pair.new_empty(R, **f32), pair.new_empty(R, **f32),
+            pair.new_empty(R if len(blocks) == 2 and P != rows else 0, **f32))  # fmt: skip
 
 
 def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Tensor, wo: Tensor, wog: Tensor,
                    small: Tensor, spans: List[int], xn: Tensor, mean_in: Tensor, rstd_in: Tensor, factors: Tensor,
-                   combined: Tensor, nrm: Tensor, mean_out: Tensor, rstd_out: Tensor, blocks: List[int],
-                   direction: str, eps_in: float, eps_out: float, need_mask: bool):  # fmt: skip
+                   combined: Tensor, nrm: Tensor, mean_out: Tensor, rstd_out: Tensor, mask_pad: Tensor,
+                   blocks: List[int], direction: str, eps_in: float, eps_out: float, need_mask: bool):  # fmt: skip
     """Gradients of the prepared operands: (pair, mask, w_cat, wo, wog, small); the mask gradient is empty
     when not needed."""
 
@@ -424,14 +482,22 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
     d_small = torch.empty_like(small)
     d_views = _small_views(d_small, spans)
     lib = _lib.load()
-    G, P, C = pair.shape
+    G, rows, C = pair.shape
     H = factors.shape[2]
+    n, side = _sides(pair, blocks)
+    P = _cells(pair, blocks)
     R = G * P
     dtype, dev = pair.dtype, pair.device
+    want_mask = mask is not None and need_mask
+    if n:
+        mask = mask_pad
     geo = _geometry(pair, H, mask is not None, eps_out)
+    geo.positions = P
     cp, hp = geo.c_row, geo.h_row
     stream = _stream(dev)
     dout = dout.resolve_neg().to(dtype).contiguous()
+    if n:
+        pair, dout = _aligned(pair), _aligned(dout)
 
     def empty():  # a fresh tensor per absent gradient: custom-op outputs may not alias
         return pair.new_empty(0, dtype=torch.float32)
@@ -439,9 +505,10 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
     with torch.cuda.device(dev):
         g_val = torch.empty(R, cp, dtype=dtype, device=dev)
         g_gate = torch.empty(R, cp, dtype=dtype, device=dev)
-        _lib.check(lib.oops_trimul_output_backward(ctypes.byref(geo), _ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog),
-                                                   _ptr(bo), _ptr(bog), _ptr(dout), _ptr(g_val), _ptr(g_gate),
-                                                   stream),
+        ptrs = (_ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog), _ptr(bo), _ptr(bog), _ptr(dout), _ptr(g_val), _ptr(g_gate),
+                stream)  # fmt: skip
+        _lib.check(lib.oops_trimul_output_pair_backward(ctypes.byref(geo), n, side, *ptrs) if n else
+                   lib.oops_trimul_output_backward(ctypes.byref(geo), *ptrs),
                    "triangle_multiplication output backward")  # fmt: skip
         gv, gg = g_val[:, :C], g_gate[:, :C]
         # every float32 partial (K-chunk products, per-workgroup sums) is summed by one launch at the end
@@ -483,7 +550,6 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
         d_factors = torch.empty_like(factors)
         _contract(factors, d_factors, _pairs(blocks), direction, grad=True, grad_out=d_comb)
         d_proj = torch.empty(4 * H, R, dtype=dtype, device=dev)
-        want_mask = mask is not None and need_mask
         mparts = torch.empty(lib.oops_trimul_mask_parts(ctypes.byref(geo)), R, dtype=torch.float32,
                              device=dev) if want_mask else None  # fmt: skip
         bparts = torch.empty(lib.oops_trimul_bias_parts(ctypes.byref(geo)), 4 * H, dtype=torch.float32, device=dev)
@@ -496,18 +562,21 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
         if b_cat is not None:
             sums.add(bparts, out=d_views[0])
 
-        d_pair = torch.empty(G, P, C, dtype=dtype, device=dev)
-        rg = _row_geometry(dtype, R, C, C, C, eps_in)
+        d_pair = torch.empty(G, rows, C, dtype=dtype, device=dev)
+        rg = _row_geometry(dtype, G * rows, C, C, C, eps_in)
         in_parts = torch.empty(2, lib.oops_layer_norm_rows_parts(ctypes.byref(rg)), C, dtype=torch.float32,
                                device=dev)  # fmt: skip
-        _lib.check(lib.oops_layer_norm_rows_backward(ctypes.byref(rg), _ptr(pair), _ptr(in_w), _ptr(mean_in),
-                                                     _ptr(rstd_in), _ptr(d_xn), _ptr(d_pair), _ptr(in_parts[0]),
-                                                     _ptr(in_parts[1]), stream),
+        ptrs = (_ptr(pair), _ptr(in_w), _ptr(mean_in), _ptr(rstd_in), _ptr(d_xn), _ptr(d_pair), _ptr(in_parts[0]),
+                _ptr(in_parts[1]), stream)  # fmt: skip
+        _lib.check(lib.oops_layer_norm_pair_backward(ctypes.byref(rg), n, side, *ptrs) if n else
+                   lib.oops_layer_norm_rows_backward(ctypes.byref(rg), *ptrs),
                    "triangle_multiplication input LayerNorm backward")  # fmt: skip
         d_mask = sums.add(mparts).view(G, P) if want_mask else empty()
         for i, parts in ((3, in_parts[0]), (4, in_parts[1]), (5, on_parts[0]), (6, on_parts[1])):
             sums.add(parts, out=d_views[i])
         sums.run(stream)
+        if want_mask and n:  # the pair's cells of the padded gradient
+            d_mask = d_mask.view(side, side)[:n, :n].reshape(G, rows)
     # projection gradients padded back to the operands' 16-byte rows
     if cp != C:
         d_wog, d_wcat = F.pad(d_wog, (0, cp - C)), F.pad(d_wcat, (0, cp - C))
@@ -534,6 +603,7 @@ def trimul_backward(
     nrm: Tensor,
     mean_out: Tensor,
     rstd_out: Tensor,
+    mask_pad: Tensor,
     blocks: List[int],
     direction: str,
     eps_in: float,
@@ -541,24 +611,24 @@ def trimul_backward(
     need_mask: bool,
 ) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     return _backward_impl(dout, pair, mask, w_cat, wo, wog, small, spans, xn, mean_in, rstd_in, factors, combined,
-                          nrm, mean_out, rstd_out, blocks, direction, eps_in, eps_out, need_mask)  # fmt: skip
+                          nrm, mean_out, rstd_out, mask_pad, blocks, direction, eps_in, eps_out, need_mask)  # fmt: skip
 
 
 @trimul_backward.register_fake
 def _(dout, pair, mask, w_cat, wo, wog, small, spans, xn, mean_in, rstd_in, factors, combined, nrm, mean_out,
-      rstd_out, blocks, direction, eps_in, eps_out, need_mask):  # fmt: skip
-    G, P, C = pair.shape
-    d_mask = pair.new_empty(G, P, dtype=torch.float32) if mask is not None and need_mask else pair.new_empty(
+      rstd_out, mask_pad, blocks, direction, eps_in, eps_out, need_mask):  # fmt: skip
+    G, rows, C = pair.shape
+    d_mask = pair.new_empty(G, rows, dtype=torch.float32) if mask is not None and need_mask else pair.new_empty(
         0, dtype=torch.float32)
-    return (pair.new_empty(G, P, C), d_mask, torch.empty_like(w_cat), torch.empty_like(wo), torch.empty_like(wog),
+    return (pair.new_empty(G, rows, C), d_mask, torch.empty_like(w_cat), torch.empty_like(wo), torch.empty_like(wog),
             torch.empty_like(small))  # fmt: skip
 
 
 def _save(ctx, inputs, output):
     pair, mask, w_cat, wo, wog, small, spans, blocks, direction, eps_in, eps_out = inputs
-    _out, xn, mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out = output
+    _out, xn, mean_in, rstd_in, factors, combined, nrm, mean_out, rstd_out, mask_pad = output
     ctx.save_for_backward(pair, mask, w_cat, wo, wog, small, xn, mean_in, rstd_in, factors, combined, nrm,
-                          mean_out, rstd_out)  # fmt: skip
+                          mean_out, rstd_out, mask_pad)  # fmt: skip
     ctx.args = (spans, blocks, direction, eps_in, eps_out)
     ctx.has_mask = mask is not None
     ctx.set_materialize_grads(False)  # no zero-filled gradients for the saved intermediates
@@ -645,6 +715,10 @@ def _run(grouped: Tensor, mask: Optional[Tensor], blocks, direction, weights, bi
     on their exact float32 MFMA counterparts (csrc/trimul_f32.hip), the contraction as library GEMMs."""
 
     _admit(grouped, weights, biases)
+    if len(blocks) == 1:
+        n = blocks[0][1]
+        side = _padded_side(n, grouped, weights[2].shape[0])
+        blocks = [(0, side)]
     flat = [v for block in blocks for v in block]
     operands = _prepare(grouped, mask, weights, biases)
     args = (*operands, flat, direction, float(eps_in), float(eps_out))
