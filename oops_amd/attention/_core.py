@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 from collections import OrderedDict
 from typing import List, Optional, Sequence, Tuple
 
@@ -162,7 +163,7 @@ def device_table(table: Sequence[int], device: torch.device) -> tuple[Tensor, Te
     launch on another stream may still read it.
     """
 
-    key = (device.index, tuple(map(int, table)))
+    key = (device.index, table if type(table) is tuple else tuple(map(int, table)))
     host, dev, streams = _TABLES.get(key, torch.cuda.is_current_stream_capturing())
     raw = _stream(device)
     if raw not in streams:
@@ -178,48 +179,76 @@ def _vec_ok(table: Sequence[int], tensors: Sequence[Optional[Tensor]], bias: Opt
     for t in tensors:
         if t is not None and t.data_ptr() % 16:
             return 0
-    aligned = bias is None or bias.data_ptr() % 16 == 0
+    rows, bias_rows = _rows_aligned(
+        tuple(table), 16 // tensors[0].element_size(), 0 if bias is None else 16 // bias.element_size()
+    )
+    if not rows:
+        return 0
+    return 1 if bias is None or (bias_rows and bias.data_ptr() % 16 == 0) else _lib.VEC_QKV
+
+
+@functools.lru_cache(maxsize=512)
+def _rows_aligned(table: Tuple[int, ...], ce: int, bce: int) -> Tuple[bool, bool]:
+    """Whether every offset and stride of q, k, v and dO is a multiple of ``ce`` elements, and every one of
+    the biases (``bce`` 0: there is none) of ``bce``."""
+
+    aligned = True
     width = _lib.TABLE_WIDTH
-    q = tensors[0]
-    ce = 16 // q.element_size()
     cols = (
         _lib.T_Q_OFF, _lib.T_Q_SG, _lib.T_Q_SH, _lib.T_Q_SI,
         _lib.T_K_OFF, _lib.T_K_SG, _lib.T_K_SH, _lib.T_K_SI,
         _lib.T_V_OFF, _lib.T_V_SG, _lib.T_V_SH, _lib.T_V_SI,
         _lib.T_DO_OFF, _lib.T_DO_SG, _lib.T_DO_SH, _lib.T_DO_SI,
     )  # fmt: skip
-    bce = 16 // bias.element_size() if bias is not None else 1
     bcols = (_lib.T_B_OFF, _lib.T_B_SG, _lib.T_B_SH, _lib.T_B_SI)
     for s in range(len(table) // width):
         row = table[s * width : (s + 1) * width]
         if any(int(row[c]) % ce for c in cols):
-            return 0
-        if aligned and bias is not None and int(row[_lib.T_B_OFF]) >= 0 and any(int(row[c]) % bce for c in bcols):
+            return False, False
+        if aligned and bce and int(row[_lib.T_B_OFF]) >= 0 and any(int(row[c]) % bce for c in bcols):
             aligned = False
-    return 1 if aligned else _lib.VEC_QKV
+    return True, aligned
 
 
 def _geometry(q: Tensor, bias: Optional[Tensor], mask: Optional[Tensor], table: Sequence[int],
-              num_heads: int, scale: float, vec_ok: int) -> tuple[_lib.Geometry, tuple]:
+              num_heads: int, scale: float, vec_ok: int) -> tuple[_lib.Geometry, tuple, tuple]:
+    """The launch geometry, its values, and the table copies it points to."""
+
     host, dev = device_table(table, q.device)
-    geo = _lib.Geometry()
-    geo.dtype = _DTYPE_CODE[q.dtype]
-    geo.bias_dtype = _DTYPE_CODE[bias.dtype] if bias is not None else geo.dtype
-    geo.num_heads = num_heads
-    geo.head_size = q.shape[-1]
-    geo.num_samples = len(table) // _lib.TABLE_WIDTH
-    geo.has_bias = int(bias is not None)
-    geo.has_mask = int(mask is not None)
-    geo.vec_ok = vec_ok
-    geo.scale = float(scale)
-    geo.phases = _PHASES
-    geo.force_generic = _FORCE_GENERIC
-    geo.table_host = host.data_ptr()
-    geo.table_device = dev.data_ptr()
-    return geo, (host, dev)
+    dtype = _DTYPE_CODE[q.dtype]
+    args = (dtype, dtype if bias is None else _DTYPE_CODE[bias.dtype], num_heads, q.shape[-1],
+            len(table) // _lib.TABLE_WIDTH, int(bias is not None), int(mask is not None), vec_ok, float(scale),
+            _PHASES, _FORCE_GENERIC)  # fmt: skip
+    return _geometry_struct(args, host.data_ptr(), dev.data_ptr()), args, (host, dev)
 
 
-def _remap_dout(table: List[int], out: Tensor, dout: Tensor, num_heads: int) -> Optional[List[int]]:
+@functools.lru_cache(maxsize=1024)
+def _geometry_struct(args: tuple, table_host: int, table_device: int) -> _lib.Geometry:
+    """The launch geometry (cached: the library only reads it; it holds these values and nothing else)."""
+
+    return _lib.Geometry(*args, table_host, table_device)
+
+
+@functools.lru_cache(maxsize=1024)
+def _workspace_sizes(lib, table: tuple, args: tuple) -> Tuple[int, int]:
+    """(forward, backward) workspace bytes of a geometry, from the table's values."""
+
+    host = (ctypes.c_int64 * len(table))(*table)
+    address = ctypes.addressof(host)
+    geo = _lib.Geometry(*args, address, address)  # (sizing reads the host table only)
+    return lib.oops_attn_forward_workspace_bytes(ctypes.byref(geo)), lib.oops_attn_backward_workspace_bytes(
+        ctypes.byref(geo)
+    )
+
+
+def _remap_dout(table: Sequence[int], out: Tensor, dout: Tensor, num_heads: int) -> Optional[List[int]]:
+    new = _remap_strides(tuple(table), out.shape, out.stride(), dout.shape, dout.stride(), num_heads)
+    return None if new is None else list(new)
+
+
+@functools.lru_cache(maxsize=512)
+def _remap_strides(table: Tuple[int, ...], sizes: Sequence[int], ost: Sequence[int], dout_sizes: Sequence[int],
+                   dst: Sequence[int], num_heads: int) -> Optional[Tuple[int, ...]]:
     """``table`` with its dO columns rewritten for ``dout``'s strides, or None.
 
     The rows address the output (dense in some dimension order) as
@@ -230,10 +259,9 @@ def _remap_dout(table: List[int], out: Tensor, dout: Tensor, num_heads: int) -> 
     None when that does not hold or dO's last dimension is not unit-stride.
     """
 
-    if dout.shape != out.shape or out.dim() == 0 or (dout.size(-1) > 1 and dout.stride(-1) != 1):
+    if dout_sizes != sizes or not sizes or (sizes[-1] > 1 and dst[-1] != 1):
         return None
-    sizes, ost, dst = out.shape, out.stride(), dout.stride()
-    order = sorted((d for d in range(out.dim()) if sizes[d] > 1), key=lambda d: -ost[d])
+    order = sorted((d for d in range(len(sizes)) if sizes[d] > 1), key=lambda d: -ost[d])
     expect = 1
     for d in reversed(order):  # dense, non-overlapping over the non-trivial dims
         if ost[d] != expect:
@@ -273,7 +301,7 @@ def _remap_dout(table: List[int], out: Tensor, dout: Tensor, num_heads: int) -> 
         if any(span[k] >= sizes[d] for k, d in enumerate(order)):
             return None
         new[s * width + _lib.T_DO_OFF : s * width + _lib.T_DO_OFF + 4] = cols
-    return new
+    return tuple(new)
 
 
 def _ptr(t: Optional[Tensor]) -> Optional[int]:
@@ -303,9 +331,10 @@ def _forward_impl(q: Tensor, k: Tensor, v: Tensor, mask: Optional[Tensor], bias:
     out = torch.empty_strided(q.size(), q.stride(), dtype=q.dtype, device=q.device)
     out_lo = _residual_like(out, save_residual)
     lse = torch.empty(lse_numel, dtype=torch.float32, device=q.device)
+    table = tuple(table)
     vec = _vec_ok(table, (q, k, v, out), bias)
-    geo, keep = _geometry(q, bias, mask, table, num_heads, scale, vec)
-    ws_bytes = lib.oops_attn_forward_workspace_bytes(ctypes.byref(geo))
+    geo, args, keep = _geometry(q, bias, mask, table, num_heads, scale, vec)
+    ws_bytes = _workspace_sizes(lib, table, args)[0]
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with _on_device(q.device):
         rc = lib.oops_attn_forward(
@@ -353,13 +382,14 @@ def _backward_impl(dout: Tensor, q: Tensor, k: Tensor, v: Tensor, mask: Optional
     """The backward launch: (dq, dk, dv, float32 dbias)."""
 
     lib = _lib.load()
+    table = tuple(table)
     dout = dout.resolve_neg().resolve_conj()
     if dout.dtype != out.dtype:
         dout = dout.to(out.dtype)
     if dout.stride() != out.stride():
         # the kernels read dO through its own table columns: re-express them
         # for dO's strides, or copy dO into the output's layout
-        remapped = _remap_dout(table, out, dout, num_heads)
+        remapped = _remap_strides(table, out.shape, out.stride(), dout.shape, dout.stride(), num_heads)
         if remapped is None:
             dout = torch.empty_strided(out.size(), out.stride(), dtype=out.dtype, device=out.device).copy_(dout)
         else:
@@ -378,8 +408,8 @@ def _backward_impl(dout: Tensor, q: Tensor, k: Tensor, v: Tensor, mask: Optional
         else q.new_empty(0, dtype=torch.float32)
     )
     vec = _vec_ok(table, (q, k, v, out, dout), bias)
-    geo, keep = _geometry(q, bias, mask, table, num_heads, scale, vec)
-    ws_bytes = lib.oops_attn_backward_workspace_bytes(ctypes.byref(geo))
+    geo, args, keep = _geometry(q, bias, mask, table, num_heads, scale, vec)
+    ws_bytes = _workspace_sizes(lib, table, args)[1]
     if ws_bytes == 0:
         _lib.check(1, "attention backward workspace sizing")
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
@@ -548,7 +578,7 @@ def attend(q, k, v, mask, bias, table, num_heads, scale, lse_numel) -> Tensor:
         t is not None and t.requires_grad for t in (q, k, v, bias)
     )
     if needs_custom_op(q):
-        out, _, _ = attention_forward(q, k, v, mask, bias, table, num_heads, scale, lse_numel, save)
+        out, _, _ = attention_forward(q, k, v, mask, bias, list(table), num_heads, scale, lse_numel, save)
     elif save:
         out = _EagerAttention.apply(q, k, v, mask, bias, table, num_heads, scale, lse_numel)
     else:

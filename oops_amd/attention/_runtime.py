@@ -58,16 +58,17 @@ def needs_custom_op(tensor) -> bool:
     return torch.compiler.is_compiling() or type(tensor) is not torch.Tensor or _get_current_dispatch_mode() is not None
 
 
-def without_second_derivative(grads, ctx, grad_output):
+def without_second_derivative(grads, ctx, grad_output, differentiable: bool = False):
     """Gradients that a kernel computed have no derivatives of their own.  When a backward runs under
-    ``create_graph=True`` and ``grad_output`` or any tensor ``ctx`` saved is differentiable, the non-None ``grads`` come back as outputs of an autograd node that raises if it
+    ``create_graph=True`` and ``grad_output`` or any tensor ``ctx`` saved is differentiable (or the caller says
+    that an input it did not save is: ``differentiable``), the non-None ``grads`` come back as outputs of an autograd node that raises if it
     is differentiated, so a second derivative fails loudly instead of silently missing these terms.
     (The custom-op path raises the same way: its backward operator has no autograd formula.)"""
 
     if not torch.is_grad_enabled():  # (an ordinary backward: the saved tensors are not unpacked)
         return grads
     inputs = (grad_output, *ctx.saved_tensors)
-    if not any(isinstance(t, torch.Tensor) and t.requires_grad for t in inputs):
+    if not differentiable and not any(isinstance(t, torch.Tensor) and t.requires_grad for t in inputs):
         return grads
     present = [g for g in grads if g is not None]
     if not present:

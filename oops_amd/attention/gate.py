@@ -22,6 +22,7 @@ does this module.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -30,7 +31,14 @@ from torch.nn import functional as F
 
 from .. import _lib
 from .._errors import unsupported
-from ._runtime import forward_mode_active, is_nested, require_no_forward_mode, require_same_device
+from ._core import _on_device, _stream
+from ._runtime import (
+    forward_mode_active,
+    is_nested,
+    needs_custom_op,
+    require_no_forward_mode,
+    require_same_device,
+)
 from .pair_bias import pair_bias_attention
 
 _OPERATOR = "gate_attention_output"
@@ -41,26 +49,29 @@ _DTYPE_CODE = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16
 
 
 def _gate_geometry(att5: Tensor, single_rows: Optional[Tensor], weight: Optional[Tensor]) -> _lib.GateGeometry:
-    b, s, t, h, d = att5.shape
+    return _geometry_struct(
+        _DTYPE_CODE[att5.dtype], att5.shape, att5.stride(), 0 if single_rows is None else single_rows.shape[1],
+        0 if single_rows is None else single_rows.stride(0), 0 if weight is None else weight.stride(0),
+    )  # fmt: skip
+
+
+@functools.lru_cache(maxsize=256)
+def _geometry_struct(dtype: int, shape, strides, channels: int, s_row: int, w_row: int) -> _lib.GateGeometry:
+    """The launch geometry (cached: the library only reads it)."""
+
+    b, s, t, h, d = shape
     g = _lib.GateGeometry()
-    g.dtype = _DTYPE_CODE[att5.dtype]
-    g.heads, g.width = h, d
-    g.channels = single_rows.shape[1] if single_rows is not None else 0
+    g.dtype, g.heads, g.width, g.channels = dtype, h, d, channels
     g.rows = b * s * t
     g.tokens = max(t, 1)
     g.groups = max(s, 1)
-    g.a_sb, g.a_sg, g.a_st, g.a_sh, g.a_sd = att5.stride()
-    g.s_row = single_rows.stride(0) if single_rows is not None else 0
-    g.w_row = weight.stride(0) if weight is not None else 0
+    g.a_sb, g.a_sg, g.a_st, g.a_sh, g.a_sd = strides
+    g.s_row, g.w_row = s_row, w_row
     return g
 
 
 def _ptr(t: Optional[Tensor]) -> Optional[int]:
     return None if t is None or t.numel() == 0 else t.data_ptr()
-
-
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _fused_ok(att5: Tensor, single_rows: Tensor, weight: Tensor) -> bool:
@@ -75,15 +86,14 @@ def _fused_ok(att5: Tensor, single_rows: Tensor, weight: Tensor) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in (att5, single_rows, weight))
 
 
-@torch.library.custom_op("oops_amd::gate_forward", mutates_args=(), device_types="cuda")
-def gate_forward(attention: Tensor, single: Tensor, weight: Tensor, save_logits: bool) -> Tuple[Tensor, Tensor]:
+def _forward_impl(attention: Tensor, single: Tensor, weight: Tensor, save_logits: bool) -> Tuple[Tensor, Tensor]:
     """(gated, logits) for attention ``(B, S, Q, H, D)`` (any strides), single ``(rows, C)``, weight ``(H*D, C)``."""
 
     lib = _lib.load()
     rows = single.shape[0]
     n = weight.shape[0]
     gated = torch.empty(rows, n, dtype=attention.dtype, device=attention.device)
-    with torch.cuda.device(attention.device):
+    with _on_device(attention.device):
         if _fused_ok(attention, single, weight):
             logits = torch.empty_like(gated) if save_logits else gated.new_empty(0)
             geo = _gate_geometry(attention, single, weight)
@@ -104,14 +114,18 @@ def gate_forward(attention: Tensor, single: Tensor, weight: Tensor, save_logits:
     return gated, logits
 
 
+@torch.library.custom_op("oops_amd::gate_forward", mutates_args=(), device_types="cuda")
+def gate_forward(attention: Tensor, single: Tensor, weight: Tensor, save_logits: bool) -> Tuple[Tensor, Tensor]:
+    return _forward_impl(attention, single, weight, save_logits)
+
+
 @gate_forward.register_fake
 def _(attention, single, weight, save_logits):
     gated = attention.new_empty(single.shape[0], weight.shape[0])
     return gated, (torch.empty_like(gated) if save_logits else gated.new_empty(0))
 
 
-@torch.library.custom_op("oops_amd::gate_backward", mutates_args=(), device_types="cuda")
-def gate_backward(
+def _backward_impl(
     grad: Tensor, attention: Tensor, logits: Tensor, need_attention: bool, need_logits: bool
 ) -> Tuple[Tensor, Tensor]:
     """(grad_attention, grad_logits), each ``(rows, H*D)`` or empty when not needed."""
@@ -122,13 +136,20 @@ def gate_backward(
     grad_logits = torch.empty_like(logits) if need_logits else logits.new_empty(0)
     if need_attention or need_logits:
         geo = _gate_geometry(attention, None, None)
-        with torch.cuda.device(attention.device):
+        with _on_device(attention.device):
             rc = lib.oops_gate_multiply_backward(
                 ctypes.byref(geo), _ptr(attention), _ptr(logits), _ptr(grad), _ptr(grad_attention),
                 _ptr(grad_logits), _stream(attention.device),
             )
         _lib.check(rc, "gate multiply backward")
     return grad_attention, grad_logits
+
+
+@torch.library.custom_op("oops_amd::gate_backward", mutates_args=(), device_types="cuda")
+def gate_backward(
+    grad: Tensor, attention: Tensor, logits: Tensor, need_attention: bool, need_logits: bool
+) -> Tuple[Tensor, Tensor]:
+    return _backward_impl(grad, attention, logits, need_attention, need_logits)
 
 
 @gate_backward.register_fake
@@ -203,12 +224,18 @@ def _setup_context(ctx, inputs, output):
 
 
 def _backward(ctx, grad_gated, _grad_logits):
+    return _grads(ctx, grad_gated, gate_backward)
+
+
+def _grads(ctx, grad_gated, backward):
+    """Gradients of (attention, single, weight, save_logits)."""
+
     if grad_gated is None:
         return None, None, None, None
     attention, single, weight, logits = ctx.saved_tensors
     need_att, need_single, need_weight = ctx.needs_input_grad[:3]
     need_logits = need_single or need_weight
-    ga, gl = gate_backward(grad_gated, attention, logits, need_att, need_logits)
+    ga, gl = backward(grad_gated, attention, logits, need_att, need_logits)
     if torch.is_grad_enabled():
         # differentiable backward: kernel values, derivatives of the composed form
         gate = torch.sigmoid(F.linear(single, weight) if need_logits else logits)
@@ -224,6 +251,22 @@ def _backward(ctx, grad_gated, _grad_logits):
 
 
 torch.library.register_autograd("oops_amd::gate_forward", _backward, setup_context=_setup_context)
+
+
+class _EagerGate(torch.autograd.Function):
+    """The same implementations as the custom ops, for eager calls: autograd calls the backward directly
+    instead of through the operator dispatcher.  Traced code takes the custom ops."""
+
+    @staticmethod
+    def forward(ctx, attention, single, weight):
+        gated, logits = _forward_impl(attention, single, weight, True)
+        ctx.save_for_backward(attention, single, weight, logits)
+        ctx.set_materialize_grads(False)
+        return gated
+
+    @staticmethod
+    def backward(ctx, grad_gated):
+        return _grads(ctx, grad_gated, _backward_impl)[:3]
 
 
 # ----------------------------------------------------------------- front-end
@@ -304,7 +347,12 @@ def _gate_values(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, dtype: to
     if weight.stride(1) != 1:
         weight = weight.contiguous()
     needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (att_qhd, single_rows, weight))
-    gated, _ = gate_forward(att5, single_rows, weight, needs_grad)
+    if needs_custom_op(att5):
+        gated, _ = gate_forward(att5, single_rows, weight, needs_grad)
+    elif needs_grad:
+        gated = _EagerGate.apply(att5, single_rows, weight)
+    else:
+        gated, _ = _forward_impl(att5, single_rows, weight, False)
     return gated.view(*att_qhd.shape[:-2], att_qhd.shape[-2] * att_qhd.shape[-1])
 
 

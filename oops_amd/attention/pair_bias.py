@@ -21,6 +21,7 @@ expand backward sums the gradient to the bias's own shape.
 
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
@@ -29,7 +30,7 @@ from torch import Tensor
 from .. import _lib
 from .._errors import unsupported
 from . import _core
-from ._runtime import is_nested, require_no_forward_mode, require_same_device
+from ._runtime import is_nested, needs_custom_op, require_no_forward_mode, require_same_device
 from .pair_bias_nested import nested_pair_bias_attention
 
 _OPERATOR = "pair_bias_attention"
@@ -247,6 +248,36 @@ def _supported(query, key, value, mask, pair_bias) -> bool:
     return True
 
 
+@functools.lru_cache(maxsize=512)
+def _grouped_table(sizes, q_st, k_st, v_st, bias, mask) -> tuple:
+    """The geometry table, one row per batch element: sizes (batch, samples, heads, queries, keys), the
+    operands' strides, ``bias`` its (samples or 1, strides) and ``mask`` its (samples or 1, whether it depends
+    on the query, strides), or None."""
+
+    batch, samples, num_heads, len_q, len_k = sizes
+    table = []
+    for b in range(batch):
+        qs, ks, vs = ((b * st[0], st[1], st[2], st[3]) for st in (q_st, k_st, v_st))
+        bias_cols = dbias_cols = None
+        mode = _lib.BIAS_NONE
+        if bias is not None:
+            bias_samples, *st = bias
+            shared = bias_samples == 1
+            bias_cols = (b * st[0], 0 if shared else st[1], st[2], st[3])
+            per_b = bias_samples * num_heads * len_q * len_k
+            dbias_cols = (b * per_b, 0 if shared else num_heads * len_q * len_k, len_q * len_k, len_k)
+            mode = _lib.BIAS_SHARED if shared else _lib.BIAS_FULL
+        mask_cols = None
+        if mask is not None:
+            mask_samples, pair_mask, *ms = mask
+            mask_cols = (b * ms[0], 0 if mask_samples == 1 else ms[1], ms[2] if pair_mask else 0)
+        table += _core.table_row(
+            groups=samples, len_q=len_q, len_k=len_k, q=qs, k=ks, v=vs, bias=bias_cols, dbias=dbias_cols,
+            bias_mode=mode, mask=mask_cols, lse_off=b * samples * num_heads * len_q,
+        )
+    return tuple(table)
+
+
 def _grouped(query, key, value, mask, pair_bias, scale):
     """Rank-4 ``(S, H, Q, D)`` or rank-5 ``(B, S, H, Q, D)`` call."""
 
@@ -290,29 +321,12 @@ def _grouped(query, key, value, mask, pair_bias, scale):
             bias = bias.expand(target).contiguous()
     scale = head_size**-0.5 if scale is None else float(scale)
 
-    table = []
-    for b in range(batch):
-        qs = (b * query.stride(0), query.stride(1), query.stride(2), query.stride(3))
-        ks = (b * key.stride(0), key.stride(1), key.stride(2), key.stride(3))
-        vs = (b * value.stride(0), value.stride(1), value.stride(2), value.stride(3))
-        bias_cols = dbias_cols = None
-        mode = _lib.BIAS_NONE
-        if bias is not None:
-            shared = bias.shape[1] == 1
-            st = bias.stride()
-            bias_cols = (b * st[0], 0 if shared else st[1], st[2], st[3])
-            per_b = bias.shape[1] * num_heads * len_q * len_k
-            dbias_cols = (b * per_b, 0 if shared else num_heads * len_q * len_k, len_q * len_k, len_k)
-            mode = _lib.BIAS_SHARED if shared else _lib.BIAS_FULL
-        mask_cols = None
-        if mask is not None:
-            ms = mask.stride()
-            m_sg = 0 if mask.shape[1] == 1 else ms[1]
-            mask_cols = (b * ms[0], m_sg, ms[2] if pair_mask else 0)
-        table += _core.table_row(
-            groups=samples, len_q=len_q, len_k=len_k, q=qs, k=ks, v=vs, bias=bias_cols, dbias=dbias_cols,
-            bias_mode=mode, mask=mask_cols, lse_off=b * samples * num_heads * len_q,
-        )
+    table_of = _grouped_table.__wrapped__ if needs_custom_op(query) else _grouped_table
+    table = table_of(
+        (batch, samples, num_heads, len_q, len_k), query.stride(), key.stride(), value.stride(),
+        None if bias is None else (bias.shape[1], *bias.stride()),
+        None if mask is None else (mask.shape[1], pair_mask, *mask.stride()),
+    )  # fmt: skip
     out = _core.attend(query, key, value, mask, bias, table, num_heads, scale, batch * samples * num_heads * len_q)
     return out.squeeze(0) if rank == 4 else out
 

@@ -10,7 +10,7 @@ The compute runs in the gfx950 HIP library through ``_core``.
 
 from __future__ import annotations
 
-from math import prod
+import functools
 from typing import Optional
 
 import torch
@@ -19,7 +19,7 @@ from torch import Tensor
 from .. import _lib
 from .._errors import unsupported
 from . import _core
-from ._runtime import is_nested, require_no_forward_mode, require_same_device
+from ._runtime import is_nested, needs_custom_op, require_no_forward_mode, require_same_device
 
 _OPERATOR = "triangle_attention"
 
@@ -116,6 +116,32 @@ def pair_orientation(tensor: Tensor) -> Optional[bool]:
     return None
 
 
+@functools.lru_cache(maxsize=512)
+def _dense_table(sizes, q_st, k_st, v_st, bias, mask_st) -> tuple:
+    """The geometry table of a dense call, one row per batch element: sizes (batch, rows, cols, heads), the
+    operands' strides, ``bias`` its (rows or 1, strides) and ``mask_st`` the mask's strides, or None."""
+
+    batch, rows, cols, num_heads = sizes
+    table = []
+    for b in range(batch):
+        qs, ks, vs = ((b * st[0], st[1], st[3], st[2]) for st in (q_st, k_st, v_st))
+        bias_cols = dbias_cols = None
+        mode = _lib.BIAS_NONE
+        if bias is not None:
+            bias_groups, *st = bias
+            shared = bias_groups == 1
+            bias_cols = (b * st[0], 0 if shared else st[1], st[2], st[3])
+            per_b = bias_groups * num_heads * cols * cols
+            dbias_cols = (b * per_b, 0 if shared else num_heads * cols * cols, cols * cols, cols)
+            mode = _lib.BIAS_SHARED if shared else _lib.BIAS_FULL
+        mask_cols = None if mask_st is None else (b * mask_st[0], mask_st[1], 0)
+        table += _core.table_row(
+            groups=rows, len_q=cols, len_k=cols, q=qs, k=ks, v=vs, bias=bias_cols, dbias=dbias_cols,
+            bias_mode=mode, mask=mask_cols, lse_off=b * rows * num_heads * cols,
+        )
+    return tuple(table)
+
+
 def _describe(t) -> Optional[str]:
     return None if t is None else f"{tuple(t.shape)} {t.dtype} {t.device}"
 
@@ -177,28 +203,12 @@ def _dense(query, key, value, mask, triangle_bias, scale):
         triangle_bias = triangle_bias.contiguous()
     scale = head_size**-0.5 if scale is None else float(scale)
 
-    table = []
-    bias_groups = 0 if triangle_bias is None else triangle_bias.shape[1]
-    for b in range(batch):
-        qs = (b * query.stride(0), query.stride(1), query.stride(3), query.stride(2))
-        ks = (b * key.stride(0), key.stride(1), key.stride(3), key.stride(2))
-        vs = (b * value.stride(0), value.stride(1), value.stride(3), value.stride(2))
-        bias_cols = dbias_cols = None
-        mode = _lib.BIAS_NONE
-        if triangle_bias is not None:
-            shared = bias_groups == 1
-            st = triangle_bias.stride()
-            bias_cols = (b * st[0], 0 if shared else st[1], st[2], st[3])
-            per_b = bias_groups * num_heads * cols * cols
-            dbias_cols = (b * per_b, 0 if shared else num_heads * cols * cols, cols * cols, cols)
-            mode = _lib.BIAS_SHARED if shared else _lib.BIAS_FULL
-        mask_cols = None
-        if mask is not None:
-            mask_cols = (b * mask.stride(0), mask.stride(1), 0)
-        table += _core.table_row(
-            groups=rows, len_q=cols, len_k=cols, q=qs, k=ks, v=vs, bias=bias_cols, dbias=dbias_cols,
-            bias_mode=mode, mask=mask_cols, lse_off=b * rows * num_heads * cols,
-        )
+    table_of = _dense_table.__wrapped__ if needs_custom_op(query) else _dense_table
+    table = table_of(
+        (batch, rows, cols, num_heads), query.stride(), key.stride(), value.stride(),
+        None if triangle_bias is None else (triangle_bias.shape[1], *triangle_bias.stride()),
+        None if mask is None else mask.stride(),
+    )  # fmt: skip
     out = _core.attend(
         query, key, value, mask, triangle_bias, table, num_heads, scale, batch * rows * num_heads * cols
     )

@@ -23,6 +23,7 @@ contraction.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 from typing import List, Literal, Optional, Sequence, Tuple
@@ -34,6 +35,7 @@ from torch.nn import functional as F
 from .. import _lib
 from .._errors import unsupported
 from .._partials import PartialSums
+from ..attention._core import _on_device, _stream
 from ..attention._runtime import (
     is_nested,
     needs_custom_op,
@@ -233,10 +235,6 @@ def _ptr(t: Optional[Tensor]) -> Optional[int]:
     return None if t is None or t.numel() == 0 else t.data_ptr()
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
 def _long_k_partials(a: Tensor, b: Tensor) -> Tensor:
     """float32 partial products of ``a (M, K) @ b (K, N)`` for a long K (weight gradients over every pair
     cell), (parts, M, N): their sum is the product.
@@ -293,7 +291,7 @@ def _contract(factors: Tensor, out: Tensor, blocks, direction: str, grad: bool =
 
     G, H = factors.shape[1], factors.shape[2]
     whole = len(blocks) == 1 and blocks[0][1] ** 2 == factors.shape[3]
-    with torch.autocast("cuda", enabled=False):
+    with torch.autocast("cuda", enabled=False) if torch.is_autocast_enabled("cuda") else contextlib.nullcontext():
         if whole and not grad:
             n = blocks[0][1]
             left, right = factors[0].view(G * H, n, n), factors[1].view(G * H, n, n)
@@ -403,7 +401,7 @@ def _forward_impl(pair: Tensor, mask: Optional[Tensor], w_cat: Tensor, wo: Tenso
     geo.positions = P
     cp, hp = geo.c_row, geo.h_row
     stream = _stream(dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         xn = torch.empty(R, cp, dtype=dtype, device=dev)
         mean_in = torch.empty(G * rows, dtype=torch.float32, device=dev)
         rstd_in = torch.empty_like(mean_in)
@@ -502,7 +500,7 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
     def empty():  # a fresh tensor per absent gradient: custom-op outputs may not alias
         return pair.new_empty(0, dtype=torch.float32)
 
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g_val = torch.empty(R, cp, dtype=dtype, device=dev)
         g_gate = torch.empty(R, cp, dtype=dtype, device=dev)
         ptrs = (_ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog), _ptr(bo), _ptr(bog), _ptr(dout), _ptr(g_val), _ptr(g_gate),
@@ -665,17 +663,51 @@ trimul_forward.register_autograd(_backward, setup_context=_setup_context)
 class _EagerTrimul(torch.autograd.Function):
     """The same implementations as the custom ops, for eager calls: autograd
     calls the backward directly instead of through the operator dispatcher.
-    Traced code (torch.compile), fake and subclass tensors take the custom ops."""
+    Traced code (torch.compile), fake and subclass tensors take the custom ops.
+    The caller's parameters are its inputs, prepared inside, so that neither
+    the concatenations and conversions nor their gradients are autograd nodes
+    (some twenty, half of the operator's host time)."""
 
     @staticmethod
-    def forward(ctx, *inputs):
+    def forward(ctx, grouped, mask, blocks, direction, eps_in, eps_out, *params):
+        operands = _prepare(grouped, mask, params[:10], params[10:])
+        inputs = (*operands, blocks, direction, eps_in, eps_out)
         output = _forward_impl(*inputs)
         _save(ctx, inputs, output)
+        ctx.mask_dtype = None if mask is None else mask.dtype
+        ctx.param_dtypes = [None if p is None else p.dtype for p in params]
         return output[0]
 
     @staticmethod
     def backward(ctx, dout):
-        return without_second_derivative(_grads(ctx, dout, _backward_impl), ctx, dout)
+        if dout is None:
+            return (None,) * (6 + len(ctx.param_dtypes))
+        pair, mask, w_cat, wo, wog, small, *rest = ctx.saved_tensors
+        spans, blocks, direction, eps_in, eps_out = ctx.args
+        need = ctx.needs_input_grad
+        need_mask = bool(need[1])
+        d_pair, d_mask, d_wcat, d_wo, d_wog, d_small = _backward_impl(
+            dout, pair, mask, w_cat, wo, wog, small, spans, *rest, blocks, direction, eps_in, eps_out, need_mask
+        )
+        C, H = pair.shape[2], w_cat.shape[0] // 4
+        grads = [None] * 16  # in the order of the operator's weights, then biases
+        for i, index in enumerate((2, 3, 4, 5)):
+            grads[index] = d_wcat[i * H : (i + 1) * H, :C]
+        grads[8], grads[9] = d_wo[:, :H], d_wog[:, :C]
+        views = {d_small.dtype: d_small}  # one conversion per parameter dtype
+        for start, (index, width) in zip(spans[::2], (((10, 11, 12, 13), H), ((14,), C), ((15,), C), ((0,), C), ((1,), C),
+                                                      ((6,), H), ((7,), H))):  # fmt: skip
+            for j, k in enumerate(index):
+                dtype = ctx.param_dtypes[k]
+                if start < 0 or dtype is None:
+                    continue
+                if dtype not in views:
+                    views[dtype] = d_small.to(dtype)
+                grads[k] = views[dtype][start + j * width : start + (j + 1) * width]
+        grads = [g if n else None for g, n in zip(grads, need[6:])]
+        d_mask = d_mask.to(ctx.mask_dtype) if need_mask else None
+        out = (d_pair if need[0] else None, d_mask, None, None, None, None, *grads)
+        return without_second_derivative(out, ctx, dout, differentiable=True)
 
 
 def _prepare(grouped: Tensor, mask: Optional[Tensor], weights, biases):
@@ -720,13 +752,12 @@ def _run(grouped: Tensor, mask: Optional[Tensor], blocks, direction, weights, bi
         side = _padded_side(n, grouped, weights[2].shape[0])
         blocks = [(0, side)]
     flat = [v for block in blocks for v in block]
-    operands = _prepare(grouped, mask, weights, biases)
-    args = (*operands, flat, direction, float(eps_in), float(eps_out))
+    rest = (flat, direction, float(eps_in), float(eps_out))
     if needs_custom_op(grouped):
-        return trimul_forward(*args)[0]
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in operands[:6]):
-        return _EagerTrimul.apply(*args)
-    return _forward_impl(*args)[0]
+        return trimul_forward(*_prepare(grouped, mask, weights, biases), *rest)[0]
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (grouped, mask, *weights, *biases)):
+        return _EagerTrimul.apply(grouped, mask, *rest, *weights, *biases)
+    return _forward_impl(*_prepare(grouped, mask, weights, biases), *rest)[0]
 
 
 # ----------------------------------------------------------------- nested
