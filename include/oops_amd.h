@@ -216,6 +216,33 @@ int oops_gate_multiply_forward(const oops_gate_geometry* geo, const void* attent
 int oops_gate_multiply_backward(const oops_gate_geometry* geo, const void* attention, const void* logits,
                                 const void* grad, void* grad_attention, void* grad_logits, void* stream);
 
+/* The whole stage in one pass over its rows (16-bit dtypes; C, D and O multiples of 8, C, H*D and O at most
+ * 256, a_sd = 1, 16-byte aligned rows, attention values within 2 GiB):
+ *   forward: out [rows][O] = gated . Wo^T, Wo [O][H*D] (row stride wo_row); logits kept unless NULL.
+ *   backward: from grad [rows][O] (the gradient of out) the attention and logit gradients of
+ *     oops_gate_multiply_backward applied to grad . Wo, and float32 partials of Wo's gradient
+ *     grad^T . gated, [parts][O][H*D] with parts = oops_linear_grad_parts(dtype, rows, O, H*D).
+ * Both round where the separate calls do.  oops_gate_stage_supported is 1 when they serve these operands.
+ * They replace the same reference launches together with the output projection's GEMMs
+ * (oops/attention/gate/composed.py:31-53). */
+int oops_gate_stage_supported(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row,
+                              const void* single, const void* weight, const void* attention,
+                              const void* output_weight);
+int oops_gate_stage_forward(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row, const void* single,
+                            const void* weight, const void* attention, const void* output_weight, void* out,
+                            void* logits, void* stream);
+int oops_gate_stage_backward(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row, const void* grad,
+                             const void* attention, const void* logits, const void* output_weight,
+                             void* grad_attention, void* grad_logits, float* g_parts, void* stream);
+
+/* Gradient products of a linear layer over many rows in one pass (16-bit; k and n multiples of 8 and at most
+ * 256, 16-byte aligned rows): d [rows][n] = x . w (x [rows][k], w [k][n]) and float32 partials
+ * [parts][k][n] of x^T . y (y [rows][n]).  parts = oops_linear_grad_parts (0: not served). */
+size_t oops_linear_grad_parts(int32_t dtype, int64_t rows, int64_t k, int64_t n);
+int oops_linear_grad_products(int32_t dtype, int64_t rows, int64_t k, int64_t n, const void* x, int64_t x_row,
+                              const void* w, int64_t w_row, const void* y, int64_t y_row, void* d, int64_t d_row,
+                              float* g_parts, void* stream);
+
 /* ---- row LayerNorm: y = (x - mean) * rstd * weight + bias over `width` ----
  *
  * Replaces the reference's layer_norm forward/backward kernels

@@ -46,6 +46,11 @@ EXPORTED_SYMBOLS = (
     "oops_gate_projection_forward",
     "oops_gate_multiply_forward",
     "oops_gate_multiply_backward",
+    "oops_gate_stage_supported",
+    "oops_gate_stage_forward",
+    "oops_gate_stage_backward",
+    "oops_linear_grad_parts",
+    "oops_linear_grad_products",
     "oops_layer_norm_rows_forward",
     "oops_layer_norm_pair_forward",
     "oops_layer_norm_pair_backward",
@@ -172,7 +177,7 @@ def load() -> ctypes.CDLL:
         import torch  # noqa: F401
 
         lib = ctypes.CDLL(os.fspath(LIB_PATH))
-        vp, sz, i32 = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int
+        vp, sz, i32, i64 = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int64
         geo = ctypes.POINTER(Geometry)
         lib.oops_attn_forward.argtypes = [geo, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
         lib.oops_attn_forward.restype = i32
@@ -191,6 +196,16 @@ def load() -> ctypes.CDLL:
         lib.oops_gate_multiply_forward.restype = i32
         lib.oops_gate_multiply_backward.argtypes = [gg, vp, vp, vp, vp, vp, vp]
         lib.oops_gate_multiply_backward.restype = i32
+        lib.oops_gate_stage_supported.argtypes = [gg, i64, i64, vp, vp, vp, vp]
+        lib.oops_gate_stage_supported.restype = i32
+        lib.oops_gate_stage_forward.argtypes = [gg, i64, i64, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_gate_stage_forward.restype = i32
+        lib.oops_gate_stage_backward.argtypes = [gg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_gate_stage_backward.restype = i32
+        lib.oops_linear_grad_parts.argtypes = [i32, i64, i64, i64]
+        lib.oops_linear_grad_parts.restype = sz
+        lib.oops_linear_grad_products.argtypes = [i32, i64, i64, i64, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp]
+        lib.oops_linear_grad_products.restype = i32
         rg = ctypes.POINTER(RowNormGeometry)
         lib.oops_layer_norm_rows_forward.argtypes = [rg, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_layer_norm_rows_forward.restype = i32
@@ -198,7 +213,6 @@ def load() -> ctypes.CDLL:
         lib.oops_layer_norm_rows_parts.restype = sz
         lib.oops_layer_norm_rows_backward.argtypes = [rg, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_layer_norm_rows_backward.restype = i32
-        i64 = ctypes.c_int64
         lib.oops_layer_norm_pair_forward.argtypes = [rg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_layer_norm_pair_forward.restype = i32
         lib.oops_layer_norm_pair_backward.argtypes = [rg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp]

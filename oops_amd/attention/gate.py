@@ -7,12 +7,14 @@ oops/attention/pair_bias/gated_pair_bias_attention.py:33-126):
     out = linear(round(sigmoid(linear(single, gate_weight))) * attention_flat, output_weight)
 
 ``attention`` is head-major ``(*prefix, H, Q, D)``; its ``(Q, H, D)`` view is
-read in place through its strides (no transposed copy).  On the GPU the gate
-projection, the sigmoid and the product run in one HIP kernel for 16-bit
-operands (MFMA, the logits kept for the backward); other dtypes and layouts
-compute the logits with ``F.linear`` and apply the gate with the HIP
-elementwise kernel.  The output projection and the ``single``/``gate_weight``
-gradients are plain GEMMs, as in the reference
+read in place through its strides (no transposed copy).  On the GPU an eager
+16-bit call of at most 256 channels on each side runs as one HIP kernel
+forward and two backward (``_EagerStage``: every tensor is read and written
+once).  Wider 16-bit operands and traced code run the gate projection, the
+sigmoid and the product in one HIP kernel (MFMA, the logits kept for the
+backward); other dtypes and layouts compute the logits with ``F.linear`` and
+apply the gate with the HIP elementwise kernel; the output projection and the
+``single``/``gate_weight`` gradients are then plain GEMMs, as in the reference
 (gate/triton/generic.py:265-327, gate/composed.py:31-53).  Where the reference
 composes Torch operations instead of launching its kernel (CPU tensors,
 mixed dtypes outside autocast, forward-mode AD, functorch transforms), so
@@ -31,6 +33,7 @@ from torch.nn import functional as F
 
 from .. import _lib
 from .._errors import unsupported
+from .._partials import PartialSums
 from ._core import _on_device, _stream
 from ._runtime import (
     forward_mode_active,
@@ -322,38 +325,149 @@ def _kernel_eligible(att_qhd: Tensor, single: Tensor, gate_weight: Tensor) -> Tu
     return ok, dtype
 
 
+# ----------------------------------------------------------------- the whole stage
+
+
+def _stage_ok(att5: Tensor, single_rows: Tensor, weight: Tensor, out_weight: Tensor) -> bool:
+    """The one-pass kernels serve these operands (gate_stage_ok in gate_stage.hip)."""
+
+    if att5.dtype == torch.float32 or out_weight.dtype != att5.dtype:
+        return False
+    if not single_rows.shape[0] or out_weight.stride(1) != 1 or out_weight.is_neg():
+        return False
+    geo = _gate_geometry(att5, single_rows, weight)
+    return bool(_lib.load().oops_gate_stage_supported(
+        ctypes.byref(geo), out_weight.shape[0], out_weight.stride(0), _ptr(single_rows), _ptr(weight), _ptr(att5),
+        _ptr(out_weight)))  # fmt: skip
+
+
+def _stage_forward(att5: Tensor, single_rows: Tensor, weight: Tensor, out_weight: Tensor, save_logits: bool):
+    """(out (rows, O), logits (rows, H*D) or None)."""
+
+    rows, dev = single_rows.shape[0], att5.device
+    out = torch.empty(rows, out_weight.shape[0], dtype=att5.dtype, device=dev)
+    logits = torch.empty(rows, weight.shape[0], dtype=att5.dtype, device=dev) if save_logits else None
+    with _on_device(dev):
+        rc = _lib.load().oops_gate_stage_forward(
+            ctypes.byref(_gate_geometry(att5, single_rows, weight)), out_weight.shape[0], out_weight.stride(0),
+            _ptr(single_rows), _ptr(weight), _ptr(att5), _ptr(out_weight), _ptr(out), _ptr(logits), _stream(dev),
+        )  # fmt: skip
+    _lib.check(rc, "gated output stage")
+    return out, logits
+
+
+class _EagerStage(torch.autograd.Function):
+    """The stage for eager 16-bit calls: one kernel forward, two backward.  The gated rows are not kept; the
+    backward rebuilds them from the logits."""
+
+    @staticmethod
+    def forward(ctx, att5, single_rows, weight, out_weight):
+        out, logits = _stage_forward(att5, single_rows, weight, out_weight, True)
+        ctx.save_for_backward(att5, single_rows, weight, out_weight, logits)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        att5, single, weight, out_weight, logits = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            # differentiable backward: through the separate operators (aliases keep the operands' own
+            # dependences on each other out of these gradients)
+            inputs = [t.view_as(t) for t in (att5, single, weight, out_weight)]
+            out = _OutputProjection.apply(_EagerGate.apply(*inputs[:3]), inputs[3])
+            wanted = [t for t, n in zip(inputs, need) if n]
+            grads = iter(torch.autograd.grad(out, wanted, grad, create_graph=True))
+            return tuple(next(grads) if n else None for n in need)
+        need_att, need_single, need_weight, need_out = need
+        need_logits = need_single or need_weight
+        lib, dev = _lib.load(), att5.device
+        rows, channels = single.shape
+        width, out_channels = weight.shape[0], out_weight.shape[0]
+        grad = grad.resolve_neg().contiguous()
+        if grad.data_ptr() % 16:
+            grad = grad.clone()
+        sums = PartialSums()
+        grad_att = grad_logits = grad_single = grad_weight = grad_out = None
+        with _on_device(dev):
+            stream = _stream(dev)
+            code = _DTYPE_CODE[att5.dtype]
+            if need_att and need_logits and need_out:
+                geo = _gate_geometry(att5, single, weight)
+                grad_att, grad_logits = torch.empty_like(logits), torch.empty_like(logits)
+                parts = torch.empty(lib.oops_linear_grad_parts(code, rows, out_channels, width), out_channels, width,
+                                    dtype=torch.float32, device=dev)  # fmt: skip
+                _lib.check(lib.oops_gate_stage_backward(
+                    ctypes.byref(geo), out_channels, out_weight.stride(0), _ptr(grad), _ptr(att5), _ptr(logits),
+                    _ptr(out_weight), _ptr(grad_att), _ptr(grad_logits), _ptr(parts), stream),
+                    "gated output stage backward")  # fmt: skip
+                grad_out = sums.add(parts, grad.dtype)
+            else:
+                if need_att or need_logits:
+                    grad_att, grad_logits = _backward_impl(grad @ out_weight, att5, logits, need_att, need_logits)
+                if need_out:
+                    gated = torch.empty_like(logits)
+                    _lib.check(lib.oops_gate_multiply_forward(
+                        ctypes.byref(_gate_geometry(att5, None, None)), _ptr(att5), _ptr(logits), _ptr(gated), stream),
+                        "gate multiply")  # fmt: skip
+                    grad_out = _weight_grad(grad, gated)
+            if need_single and need_weight:
+                grad_single = torch.empty(rows, channels, dtype=grad.dtype, device=dev)
+                parts = torch.empty(lib.oops_linear_grad_parts(code, rows, width, channels), width, channels,
+                                    dtype=torch.float32, device=dev)  # fmt: skip
+                _lib.check(lib.oops_linear_grad_products(
+                    code, rows, width, channels, _ptr(grad_logits), width, _ptr(weight), weight.stride(0),
+                    _ptr(single), single.stride(0), _ptr(grad_single), channels, _ptr(parts), stream),
+                    "gate gradients")  # fmt: skip
+                grad_weight = sums.add(parts, grad.dtype)
+            elif need_single:
+                grad_single = grad_logits @ weight
+            elif need_weight:
+                grad_weight = _weight_grad(grad_logits, single)
+            sums.run(stream)
+        return grad_att.view(att5.shape) if need_att else None, grad_single, grad_weight, grad_out
+
+
 def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_weight: Tensor) -> Tensor:
     """The stage's output ``(*prefix, Q, O)`` for attention viewed ``(*prefix, Q, H, D)`` (prefix rank 1 or 2)."""
 
     ok, dtype = _kernel_eligible(att_qhd, single, gate_weight)
     if not ok:
         return F.linear(_composed(att_qhd, single, gate_weight), output_weight)
-    gated = _gate_values(att_qhd, single, gate_weight, dtype)
-    if not torch.is_grad_enabled() or output_weight.dtype != gated.dtype:
-        return F.linear(gated, output_weight)
-    return _OutputProjection.apply(gated, output_weight)
-
-
-def _gate_values(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, dtype: torch.dtype) -> Tensor:
-    """Gated values ``(*prefix, Q, H*D)`` from the HIP kernels."""
-
-    single = single if single.dtype == dtype else single.to(dtype)
-    weight = gate_weight if gate_weight.dtype == dtype else gate_weight.to(dtype)
-    att5 = att_qhd if att_qhd.dim() == 5 else att_qhd.unsqueeze(0)
-    channels = single.shape[-1]
-    single_rows = single.reshape(-1, channels)
-    if single_rows.stride(1) != 1:
-        single_rows = single_rows.contiguous()
-    if weight.stride(1) != 1:
-        weight = weight.contiguous()
-    needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (att_qhd, single_rows, weight))
-    if needs_custom_op(att5):
+    att5, single_rows, weight = _operands(att_qhd, single, gate_weight, dtype)
+    traced = needs_custom_op(att5)
+    shape = att_qhd.shape[:-2]
+    if not traced and _stage_ok(att5, single_rows, weight, output_weight):
+        operands = (att5, single_rows, weight, output_weight)
+        if torch.is_grad_enabled() and any(t.requires_grad for t in operands):
+            out = _EagerStage.apply(*operands)
+        else:
+            out, _ = _stage_forward(*operands, False)
+        return out.view(*shape, out.shape[-1])
+    needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (att5, single_rows, weight))
+    if traced:
         gated, _ = gate_forward(att5, single_rows, weight, needs_grad)
     elif needs_grad:
         gated = _EagerGate.apply(att5, single_rows, weight)
     else:
         gated, _ = _forward_impl(att5, single_rows, weight, False)
-    return gated.view(*att_qhd.shape[:-2], att_qhd.shape[-2] * att_qhd.shape[-1])
+    gated = gated.view(*shape, gated.shape[-1])
+    if not torch.is_grad_enabled() or output_weight.dtype != gated.dtype:
+        return F.linear(gated, output_weight)
+    return _OutputProjection.apply(gated, output_weight)
+
+
+def _operands(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, dtype: torch.dtype):
+    """The kernels' operands: attention (B, S, Q, H, D), single rows and gate weight with unit-stride channels."""
+
+    single = single if single.dtype == dtype else single.to(dtype)
+    weight = gate_weight if gate_weight.dtype == dtype else gate_weight.to(dtype)
+    att5 = att_qhd if att_qhd.dim() == 5 else att_qhd.unsqueeze(0)
+    single_rows = single.reshape(-1, single.shape[-1])
+    if single_rows.stride(1) != 1:
+        single_rows = single_rows.contiguous()
+    if weight.stride(1) != 1:
+        weight = weight.contiguous()
+    return att5, single_rows, weight
 
 
 def gate_attention_output(attention, single, gate_weight: Tensor, output_weight: Tensor):

@@ -34,6 +34,7 @@ SOURCES = (
     "attn_bwd_fused.hip",
     "attn_f32.hip",
     "gate.hip",
+    "gate_stage.hip",
     "trimul.hip",
     "trimul_f32.hip",
     "reduce.hip",

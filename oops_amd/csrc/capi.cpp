@@ -556,6 +556,65 @@ int oops_gate_multiply_backward(const oops_gate_geometry* geo, const void* atten
                             "gate multiply backward");
 }
 
+int oops_gate_stage_supported(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row,
+                              const void* single, const void* weight, const void* attention,
+                              const void* output_weight) {
+  g_last_error.clear();
+  if (check_gate(geo)) return 0;
+  return oops::gate_stage_ok(*geo, out_channels, wo_row, single, weight, attention, output_weight) ? 1 : 0;
+}
+
+int oops_gate_stage_forward(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row, const void* single,
+                            const void* weight, const void* attention, const void* output_weight, void* out,
+                            void* logits, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_gate(geo)) return rc;
+  if (!single || !weight || !attention || !output_weight || !out)
+    return fail(OOPS_EINVAL, "single, both weights, attention and out must be non-NULL");
+  if (!oops::gate_stage_ok(*geo, out_channels, wo_row, single, weight, attention, output_weight) || !aligned16(out) ||
+      !aligned16(logits))
+    return fail(OOPS_EINVAL, "operands that the gated output stage's pass does not serve (%lld output channels)",
+                out_channels);
+  return gate_launch_result(oops::launch_gate_stage_forward(*geo, out_channels, wo_row, single, weight, attention,
+                                                            output_weight, out, logits,
+                                                            static_cast<hipStream_t>(stream)),
+                            "gated output stage");
+}
+
+int oops_gate_stage_backward(const oops_gate_geometry* geo, int64_t out_channels, int64_t wo_row, const void* grad,
+                             const void* attention, const void* logits, const void* output_weight,
+                             void* grad_attention, void* grad_logits, float* g_parts, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_gate(geo)) return rc;
+  if (!grad || !attention || !logits || !output_weight || !grad_attention || !grad_logits || !g_parts)
+    return fail(OOPS_EINVAL, "operands, gradients and partials must be non-NULL");
+  if (!oops::gate_stage_ok(*geo, out_channels, wo_row, grad, logits, attention, output_weight) ||
+      !aligned16(grad_attention) || !aligned16(grad_logits))
+    return fail(OOPS_EINVAL, "operands that the gated output stage's pass does not serve (%lld output channels)",
+                out_channels);
+  return gate_launch_result(oops::launch_gate_stage_backward(*geo, out_channels, wo_row, grad, attention, logits,
+                                                             output_weight, grad_attention, grad_logits, g_parts,
+                                                             static_cast<hipStream_t>(stream)),
+                            "gated output stage backward");
+}
+
+size_t oops_linear_grad_parts(int32_t dtype, int64_t rows, int64_t k, int64_t n) {
+  g_last_error.clear();
+  return (size_t)oops::row_grad_parts(dtype, rows, k, n);
+}
+
+int oops_linear_grad_products(int32_t dtype, int64_t rows, int64_t k, int64_t n, const void* x, int64_t x_row,
+                              const void* w, int64_t w_row, const void* y, int64_t y_row, void* d, int64_t d_row,
+                              float* g_parts, void* stream) {
+  g_last_error.clear();
+  if (!x || !w || !y || !d || !g_parts) return fail(OOPS_EINVAL, "operands must be non-NULL");
+  if (!oops::linear_grads_ok(dtype, rows, k, n, x, x_row, w, w_row, y, y_row, d, d_row))
+    return fail(OOPS_EINVAL, "operands that the linear gradient products do not serve (k %lld, n %lld)", k, n);
+  return gate_launch_result(oops::launch_linear_grads(dtype, rows, k, n, x, x_row, w, w_row, y, y_row, d, d_row,
+                                                      g_parts, static_cast<hipStream_t>(stream)),
+                            "linear gradient products");
+}
+
 int oops_layer_norm_rows_forward(const oops_row_norm_geometry* geo, const void* x, const float* weight,
                                  const float* bias, void* y, float* mean, float* rstd, void* stream) {
   g_last_error.clear();

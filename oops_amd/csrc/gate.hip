@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "attn_fast_common.h"
+#include "gate_device.h"
 #include "gate_kernels.h"
 
 namespace oops {
@@ -64,20 +65,6 @@ GateArgs make_args(const oops_gate_geometry& g) {
   a.width = g.width;
   a.channels = g.channels;
   return a;
-}
-
-template <typename T>
-__device__ __forceinline__ float to_f(T x) {
-  return (float)x;
-}
-// x rounded to T and back (identity for float)
-template <typename T>
-__device__ __forceinline__ float rnd(float x) {
-  return (float)(T)x;
-}
-// 1 / (1 + 2^(-x log2 e)) on the hardware exp2 and reciprocal
-__device__ __forceinline__ float sigmoid_f(float x) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2e));
 }
 
 // element offset of row r's attention values (head 0, d 0)
