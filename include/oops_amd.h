@@ -402,6 +402,19 @@ size_t oops_sum_partials_workspace_bytes(const oops_sum_segment* segments, int32
 int oops_sum_partials(const oops_sum_segment* segments, int32_t num_segments, void* workspace,
                       size_t workspace_bytes, void* stream);
 
+/* The factor backward together with the products of its result, for 16-bit pairs with 64 < C, H <= 128 and
+ * positions a multiple of 32 (no mask gradient): with d_proj the gradient oops_trimul_factors_backward writes
+ *   grad_xn [R][C] (rows C apart) += d_proj^T . W      (added in float32, rounded once)
+ *   w_parts: d_proj . xn   -> float32 partials [parts][4H][C]
+ *   b_parts: row sums of d_proj before its rounding -> float32 partials [parts][4H] (may be NULL)
+ * with parts = oops_trimul_factor_grad_parts (0: not served; use oops_trimul_factors_backward and GEMMs).
+ * Replaces the reference's factor backward with its projection GEMMs
+ * (triangle_multiplication/triton/generic.py:960-1018). */
+size_t oops_trimul_factor_grad_parts(const oops_trimul_geometry* geo);
+int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normalized, const void* weight,
+                             const float* bias, const void* mask, const void* grad_factors, void* grad_xn,
+                             float* w_parts, float* b_parts, void* stream);
+
 /* The products of the gated output's backward that share one operand X [R][128] (16-bit, C = H = 128):
  *   d = X W              W [128][128] (rows w_row apart) -> d [R][128] (rows d_row apart), the dtype
  *   g_parts: X^T Y       Y [R][128] (rows y_row apart)   -> float32 partials [parts][128][128]

@@ -69,6 +69,8 @@ EXPORTED_SYMBOLS = (
     "oops_trimul_output_backward",
     "oops_trimul_output_pair_forward",
     "oops_trimul_output_pair_backward",
+    "oops_trimul_factor_grad_parts",
+    "oops_trimul_factor_grads",
     "oops_trimul_output_grad_parts",
     "oops_trimul_output_grad_products",
     "oops_sum_partials_workspace_bytes",
@@ -244,6 +246,10 @@ def load() -> ctypes.CDLL:
         lib.oops_trimul_output_pair_forward.restype = i32
         lib.oops_trimul_output_pair_backward.argtypes = [tg, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_trimul_output_pair_backward.restype = i32
+        lib.oops_trimul_factor_grad_parts.argtypes = [tg]
+        lib.oops_trimul_factor_grad_parts.restype = sz
+        lib.oops_trimul_factor_grads.argtypes = [tg, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+        lib.oops_trimul_factor_grads.restype = i32
         lib.oops_trimul_output_grad_parts.argtypes = [tg]
         lib.oops_trimul_output_grad_parts.restype = sz
         lib.oops_trimul_output_grad_products.argtypes = [tg, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, vp]

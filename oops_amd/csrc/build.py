@@ -37,6 +37,7 @@ SOURCES = (
     "gate_stage.hip",
     "trimul.hip",
     "trimul_f32.hip",
+    "trimul_grad.hip",
     "reduce.hip",
     "capi.cpp",
 )

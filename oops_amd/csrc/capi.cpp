@@ -870,6 +870,32 @@ int oops_trimul_output_backward(const oops_trimul_geometry* geo, const void* nor
                             "triangle multiplication output backward");
 }
 
+size_t oops_trimul_factor_grad_parts(const oops_trimul_geometry* geo) {
+  g_last_error.clear();
+  if (check_trimul(geo)) return 0;
+  return (size_t)oops::trimul_factor_grad_parts(*geo);
+}
+
+int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normalized, const void* weight,
+                             const float* bias, const void* mask, const void* grad_factors, void* grad_xn,
+                             float* w_parts, float* b_parts, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_trimul(geo)) return rc;
+  if (!oops::trimul_factor_grad_parts(*geo))
+    return fail(OOPS_EINVAL, "the factor gradients' pass serves 16-bit pairs with 64 < C, H <= 128 and positions in "
+                             "32s");
+  if (!normalized || !weight || !grad_factors || !grad_xn || !w_parts)
+    return fail(OOPS_EINVAL, "operands and weight partials must be non-NULL");
+  if (geo->has_mask && !mask) return fail(OOPS_EINVAL, "has_mask is set but mask is NULL");
+  if (!aligned16(normalized) || !aligned16(weight) || !aligned16(grad_factors) || !aligned16(grad_xn))
+    return fail(OOPS_EINVAL, "operands must be 16-byte aligned");
+  return gate_launch_result(
+      oops::launch_trimul_factor_grad(*geo, normalized, weight, bias,
+                                      geo->has_mask ? static_cast<const float*>(mask) : nullptr, grad_factors,
+                                      grad_xn, w_parts, b_parts, static_cast<hipStream_t>(stream)),
+      "triangle multiplication factor gradients");
+}
+
 size_t oops_trimul_output_grad_parts(const oops_trimul_geometry* geo) {
   g_last_error.clear();
   if (check_trimul(geo)) return 0;

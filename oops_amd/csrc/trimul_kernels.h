@@ -54,6 +54,12 @@ hipError_t launch_trimul_output_grad(const oops_trimul_geometry& g, const void* 
                                      int64_t w_row, const void* y, int64_t y_row, void* d, int64_t d_row,
                                      float* g_parts, float* s_parts, hipStream_t stream);
 
+// the factor backward with its products in one pass (trimul_grad.hip, oops_trimul_factor_grads)
+int64_t trimul_factor_grad_parts(const oops_trimul_geometry& g);
+hipError_t launch_trimul_factor_grad(const oops_trimul_geometry& g, const void* normalized, const void* weight,
+                                     const float* bias, const float* mask, const void* grad_factors, void* grad_xn,
+                                     float* w_parts, float* b_parts, hipStream_t stream);
+
 // float32 pairs (trimul_f32.hip): the same contracts on the exact float32 matrix core
 hipError_t launch_trimul_factors_f32(const oops_trimul_geometry& g, const void* normalized, const void* weight,
                                      const float* bias, const void* mask, void* factors, const void* grad_factors,

@@ -547,16 +547,26 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
                    "triangle_multiplication output LayerNorm backward")  # fmt: skip
         d_factors = torch.empty_like(factors)
         _contract(factors, d_factors, _pairs(blocks), direction, grad=True, grad_out=d_comb)
-        d_proj = torch.empty(4 * H, R, dtype=dtype, device=dev)
-        mparts = torch.empty(lib.oops_trimul_mask_parts(ctypes.byref(geo)), R, dtype=torch.float32,
-                             device=dev) if want_mask else None  # fmt: skip
-        bparts = torch.empty(lib.oops_trimul_bias_parts(ctypes.byref(geo)), 4 * H, dtype=torch.float32, device=dev)
-        _lib.check(lib.oops_trimul_factors_backward(ctypes.byref(geo), _ptr(xn), _ptr(w_cat), _ptr(b_cat),
-                                                    _ptr(mask), _ptr(d_factors), _ptr(d_proj), _ptr(mparts),
-                                                    _ptr(bparts), stream),
-                   "triangle_multiplication factor backward")  # fmt: skip
-        d_xn = d_xn.addmm_(d_proj.t(), w_cat[:, :C])  # in place: no copy of d_xn into a new result
-        d_wcat = sums.add(_long_k_partials(d_proj, xn[:, :C]), dtype)
+        parts = 0 if want_mask else lib.oops_trimul_factor_grad_parts(ctypes.byref(geo))
+        if parts:
+            # one pass: the factor backward, its products with the weights (added to d_xn) and with xn
+            w_parts = torch.empty(parts, 4 * H, C, dtype=torch.float32, device=dev)
+            bparts = torch.empty(parts, 4 * H, dtype=torch.float32, device=dev)
+            _lib.check(lib.oops_trimul_factor_grads(ctypes.byref(geo), _ptr(xn), _ptr(w_cat), _ptr(b_cat), _ptr(mask),
+                                                    _ptr(d_factors), _ptr(d_xn), _ptr(w_parts), _ptr(bparts), stream),
+                       "triangle_multiplication factor gradients")  # fmt: skip
+            d_wcat = sums.add(w_parts, dtype)
+        else:
+            d_proj = torch.empty(4 * H, R, dtype=dtype, device=dev)
+            mparts = torch.empty(lib.oops_trimul_mask_parts(ctypes.byref(geo)), R, dtype=torch.float32,
+                                 device=dev) if want_mask else None  # fmt: skip
+            bparts = torch.empty(lib.oops_trimul_bias_parts(ctypes.byref(geo)), 4 * H, dtype=torch.float32, device=dev)
+            _lib.check(lib.oops_trimul_factors_backward(ctypes.byref(geo), _ptr(xn), _ptr(w_cat), _ptr(b_cat),
+                                                        _ptr(mask), _ptr(d_factors), _ptr(d_proj), _ptr(mparts),
+                                                        _ptr(bparts), stream),
+                       "triangle_multiplication factor backward")  # fmt: skip
+            d_xn = d_xn.addmm_(d_proj.t(), w_cat[:, :C])  # in place: no copy of d_xn into a new result
+            d_wcat = sums.add(_long_k_partials(d_proj, xn[:, :C]), dtype)
         if b_cat is not None:
             sums.add(bparts, out=d_views[0])
 

@@ -1,0 +1,84 @@
+"""The triangle multiplication's factor backward with its products in one pass (oops_trimul_factor_grads)
+against the separate factor backward (oops_trimul_factors_backward, the same 16-bit projection gradients) and
+float64 products of its result: one tile and several runs of tiles, groups that end inside a run, channel and
+hidden sizes below 128, with and without a mask and biases."""
+
+import ctypes
+
+import pytest
+import torch
+
+from oops_amd import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize(
+    "dtype,groups,positions,c,h,masked,biases",
+    [
+        (torch.bfloat16, 1, 32, 128, 128, True, True),
+        (torch.float16, 3, 32 * 5, 128, 128, False, True),
+        (torch.bfloat16, 5, 32 * 27, 128, 72, True, False),
+        (torch.float16, 2, 32 * 300, 88, 128, True, True),
+        (torch.bfloat16, 1, 32 * 2500, 120, 104, True, True),
+        (torch.bfloat16, 7, 32 * 310, 128, 128, False, False),
+    ],
+)
+def test_factor_grads(dtype, groups, positions, c, h, masked, biases):
+    lib = _lib.load()
+    gen = torch.Generator(device=DEV).manual_seed(positions)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=gen)  # noqa: E731
+    R = groups * positions
+    xn = rand(R, c).to(dtype)
+    w = (rand(4 * h, c) * c**-0.5).to(dtype)
+    bias = rand(4 * h) if biases else None
+    mask = (torch.rand(R, device=DEV, generator=gen) > 0.2).float() if masked else None
+    gf = rand(2, groups, h, positions).to(dtype)
+    before = rand(R, c).to(dtype)
+    geo = _lib.TrimulGeometry()
+    geo.dtype = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16
+    geo.channels, geo.hidden, geo.has_mask = c, h, masked
+    geo.groups, geo.positions, geo.c_row, geo.h_row, geo.eps = groups, positions, c, h, 1e-5
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    stream = torch.cuda.current_stream().cuda_stream
+    d_proj = torch.empty(4 * h, R, dtype=dtype, device=DEV)
+    old_b = torch.empty(lib.oops_trimul_bias_parts(ctypes.byref(geo)), 4 * h, device=DEV)
+    assert 0 == lib.oops_trimul_factors_backward(ctypes.byref(geo), ptr(xn), ptr(w), ptr(bias), ptr(mask), ptr(gf),
+                                                 ptr(d_proj), None, ptr(old_b), stream), lib.oops_last_error()
+    parts = lib.oops_trimul_factor_grad_parts(ctypes.byref(geo))
+    assert 1 <= parts <= 256
+    d_xn = before.clone()
+    wp = torch.full((parts, 4 * h, c), float("nan"), device=DEV)
+    bp = torch.full((parts, 4 * h), float("nan"), device=DEV)
+    assert 0 == lib.oops_trimul_factor_grads(ctypes.byref(geo), ptr(xn), ptr(w), ptr(bias), ptr(mask), ptr(gf),
+                                             ptr(d_xn), ptr(wp), ptr(bp), stream), lib.oops_last_error()
+    torch.cuda.synchronize()
+    p64, x64, w64 = d_proj.double(), xn.double(), w.double()
+    # one rounding of a float32 sum of 4 h + 1 terms: half a unit of the result and the sum's float32 errors
+    # (at most 4 h + 1 roundings of 2^-24 of the magnitudes)
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    want = before.double() + p64.t() @ w64
+    mag = before.double().abs() + p64.t().abs() @ w64.abs()
+    assert ((d_xn.double() - want).abs() <= unit * want.abs() + (4 * h + 1) * 2.0**-24 * mag + 1e-7).all()
+    # float32 sums over the tokens: at most R roundings of 2^-24 of the magnitudes in any order; the sums here
+    # are of runs, so their errors stay far inside sqrt(R) of them
+    want, mag = p64 @ x64, p64.abs() @ x64.abs()
+    assert ((wp.double().sum(0) - want).abs() <= 4 * R**0.5 * 2.0**-24 * mag + 1e-9).all()
+    # the separate backward sums the same float32 values
+    want, mag = old_b.double().sum(0), p64.abs().sum(1)
+    assert ((bp.double().sum(0) - want).abs() <= 8 * R**0.5 * 2.0**-24 * mag + 1e-6).all()
+
+
+def test_factor_grads_served_range():
+    lib = _lib.load()
+
+    def parts(dtype=_lib.BF16, c=128, h=128, groups=1, positions=64):
+        geo = _lib.TrimulGeometry()
+        geo.dtype, geo.channels, geo.hidden, geo.has_mask = dtype, c, h, 0
+        geo.groups, geo.positions, geo.c_row, geo.h_row, geo.eps = groups, positions, (c + 7) // 8 * 8, (h + 7) // 8 * 8, 1e-5
+        return lib.oops_trimul_factor_grad_parts(ctypes.byref(geo))
+
+    assert parts() == 1
+    for change in (dict(dtype=_lib.F32), dict(c=64), dict(c=136), dict(c=100), dict(h=64), dict(h=136), dict(positions=81)):
+        assert parts(**change) == 0, change
