@@ -415,6 +415,21 @@ int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normal
                              const float* bias, const void* mask, const void* grad_factors, void* grad_xn,
                              float* w_parts, float* b_parts, void* stream);
 
+/* The gated output's backward with its products in one pass, for 16-bit pairs with 64 < C, H <= 128 in multiples
+ * of 8, c_row = C and h_row = H: with grad_value and grad_gate the gradients oops_trimul_output_backward writes
+ *   grad_normalized [R][H] = grad_value . W_out      wo_parts: grad_value^T . normalized, partials [parts][C][H]
+ *   grad_xn [R][C] = grad_gate . W_gate              wg_parts: grad_gate^T . xn, partials [parts][C][C]
+ *   b_parts: column sums of grad_value, then of grad_gate, float32 partials [2][parts][C]
+ * with parts = oops_trimul_output_grads_parts (0: not served).  n, n_pad: 0, or the sides of a padded pair
+ * (oops_trimul_output_pair_backward).  Replaces the reference's output backward and the GEMMs and column sums
+ * behind it (triangle_multiplication/triton/generic.py:820-856). */
+size_t oops_trimul_output_grads_parts(const oops_trimul_geometry* geo);
+int oops_trimul_output_grads(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                             const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                             const float* output_bias, const float* gate_bias, const void* grad_out,
+                             void* grad_normalized, void* grad_xn, float* wo_parts, float* wg_parts, float* b_parts,
+                             void* stream);
+
 /* The products of the gated output's backward that share one operand X [R][128] (16-bit, C = H = 128):
  *   d = X W              W [128][128] (rows w_row apart) -> d [R][128] (rows d_row apart), the dtype
  *   g_parts: X^T Y       Y [R][128] (rows y_row apart)   -> float32 partials [parts][128][128]

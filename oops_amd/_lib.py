@@ -71,6 +71,8 @@ EXPORTED_SYMBOLS = (
     "oops_trimul_output_pair_backward",
     "oops_trimul_factor_grad_parts",
     "oops_trimul_factor_grads",
+    "oops_trimul_output_grads_parts",
+    "oops_trimul_output_grads",
     "oops_trimul_output_grad_parts",
     "oops_trimul_output_grad_products",
     "oops_sum_partials_workspace_bytes",
@@ -250,6 +252,10 @@ def load() -> ctypes.CDLL:
         lib.oops_trimul_factor_grad_parts.restype = sz
         lib.oops_trimul_factor_grads.argtypes = [tg, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         lib.oops_trimul_factor_grads.restype = i32
+        lib.oops_trimul_output_grads_parts.argtypes = [tg]
+        lib.oops_trimul_output_grads_parts.restype = sz
+        lib.oops_trimul_output_grads.argtypes = [tg, i64, i64] + [vp] * 13
+        lib.oops_trimul_output_grads.restype = i32
         lib.oops_trimul_output_grad_parts.argtypes = [tg]
         lib.oops_trimul_output_grad_parts.restype = sz
         lib.oops_trimul_output_grad_products.argtypes = [tg, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, vp]

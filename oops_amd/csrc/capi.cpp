@@ -896,6 +896,36 @@ int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normal
       "triangle multiplication factor gradients");
 }
 
+size_t oops_trimul_output_grads_parts(const oops_trimul_geometry* geo) {
+  g_last_error.clear();
+  if (check_trimul(geo)) return 0;
+  return (size_t)oops::trimul_output_grads_parts(*geo);
+}
+
+int oops_trimul_output_grads(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
+                             const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                             const float* output_bias, const float* gate_bias, const void* grad_out,
+                             void* grad_normalized, void* grad_xn, float* wo_parts, float* wg_parts, float* b_parts,
+                             void* stream) {
+  g_last_error.clear();
+  if (int rc = check_trimul(geo)) return rc;
+  if (!oops::trimul_output_grads_parts(*geo))
+    return fail(OOPS_EINVAL, "the output gradients' pass serves 16-bit pairs with 64 < C, H <= 128");
+  if (!normalized || !pair_normalized || !output_weight || !gate_weight || !grad_out || !grad_normalized || !grad_xn ||
+      !wo_parts || !wg_parts || !b_parts)
+    return fail(OOPS_EINVAL, "operands, gradients and partials must be non-NULL");
+  if (!aligned16(normalized) || !aligned16(pair_normalized) || !aligned16(output_weight) || !aligned16(gate_weight) ||
+      !aligned16(grad_out) || !aligned16(grad_normalized) || !aligned16(grad_xn))
+    return fail(OOPS_EINVAL, "operands must be 16-byte aligned");
+  if ((n || n_pad) && !output_pair_ok(*geo, n, n_pad))
+    return fail(OOPS_EINVAL, "not a padded pair that is served (sides %lld and %lld)", n, n_pad);
+  return gate_launch_result(
+      oops::launch_trimul_output_grads(*geo, n, n_pad, normalized, pair_normalized, output_weight, gate_weight,
+                                       output_bias, gate_bias, grad_out, grad_normalized, grad_xn, wo_parts, wg_parts,
+                                       b_parts, static_cast<hipStream_t>(stream)),
+      "triangle multiplication output gradients");
+}
+
 size_t oops_trimul_output_grad_parts(const oops_trimul_geometry* geo) {
   g_last_error.clear();
   if (check_trimul(geo)) return 0;

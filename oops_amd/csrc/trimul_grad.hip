@@ -1,5 +1,5 @@
-// The factor projections' backward of the triangle multiplication in one pass over the tokens (gfx950):
-// 16-bit pairs with 64 < C, H <= 128 and positions a multiple of 32, no mask gradient.
+// The triangle multiplication's factor and output backwards, each with its products in one pass (gfx950; the
+// output's is below).  The factor projections' backward: 16-bit pairs with 64 < C, H <= 128 and positions a multiple of 32, no mask gradient.
 //
 //   value, gate = xn W^T + b (recomputed), d_proj = the gate's backward of the factor gradients
 //   d_xn += d_proj W        d_W = d_proj^T xn        d_b = column sums of d_proj
@@ -295,12 +295,274 @@ __global__ __launch_bounds__(512, 2) void trimul_factor_grad_kernel(FactorGradAr
   }
 }
 
+// ------------------------------------------------------------------ gated output
+// The backward of out = value * sigmoid(gate), value = nrm Wo^T + bo, gate = xn Wg^T + bg, with its products,
+// in one pass over the rows (16-bit, 64 < C, H <= 128):
+//
+//   g_value = d_out s            d_nrm = g_value Wo     d_Wo = g_value^T nrm    d_bo = column sums
+//   g_gate = d_out value s (1 - s)  d_xn = g_gate Wg    d_Wg = g_gate^T xn      d_bg = column sums
+//
+// As separate launches (the elementwise backward with the recomputed projections, then one pass per gradient
+// for its products) the 512 x 512 pair of 128 channels took 98 + 2 x 48 us and 740 MB; the tensors that must
+// move are 335 MB (68 us), and this kernel takes 86 us.  The scheme is the one above with both weights (2 x 32 KB) in LDS: wave (grp, th)
+// owns channels 32 grp .. + 31 of the tile's tokens 32 th .. + 31; d_out comes through the transposed read in
+// the accumulators' order.  The tiles (64 tokens) come by direct-to-LDS loads one tile ahead, the exchange
+// takes the place of its tile's inputs.  The two token halves' weight gradients meet in LDS at the end.
+constexpr int kOutTok = 64;
+
+struct OutputGradArgs {
+  const void* nrm;   // [R][h_row]
+  const void* xn;    // [R][c_row]
+  const void* wo;    // [C][h_row]
+  const void* wg;    // [C][c_row]
+  const float* bo;
+  const float* bg;
+  const void* gout;  // [R][C], or [n * n][C] of a padded pair
+  void* d_nrm;       // [R][H]
+  void* d_xn;        // [R][C]
+  float* wo_parts;   // [run][C][H]
+  float* wg_parts;   // [run][C][C]
+  float* b_parts;    // [2][run][C]
+  int64_t rows, runs;
+  int C, H, c_row, h_row, tpw;
+  uint32_t n, n_pad;  // padded pair: sides of the pair and of the grid of the rows (else 0)
+};
+
+template <typename T>
+__global__ __launch_bounds__(512, 2) void trimul_output_grads_kernel(OutputGradArgs a) {
+  using E = Elem<T>;
+  using Frag = typename E::Frag;
+  constexpr int RT = kOutTok, TILE = RT * kWide, WT = kWide * kWide;
+  // wo, wg; two slots of nrm, xn and d_out tiles (a slot's first 32 KB are its tile's exchange [256 m][64 tokens]
+  // afterwards); at the end a token half's weight gradients
+  __shared__ __attribute__((aligned(16))) T lds[2 * WT + 6 * TILE];
+  static_assert(sizeof(lds) >= (4 * 128 * 64 + 2 * kWide) * sizeof(float), "final sums");
+  T* const wo_l = lds;
+  T* const wg_l = lds + WT;
+
+  const int64_t run = xcd_tile(blockIdx.x, gridDim.x, 0);
+  if (run >= a.runs) return;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 31, g2 = lane >> 5;
+  const int grp = wave & 3, th = wave >> 2;
+  const int C = a.C, H = a.H;
+  const int64_t R = a.rows;
+  const int64_t tiles = (R + RT - 1) / RT, tile0 = run * a.tpw;
+  const int count = (int)(tiles - tile0 < a.tpw ? tiles - tile0 : a.tpw);
+
+  {
+    const __amdgpu_buffer_rsrc_t r1 = make_rsrc(a.wo, (uint32_t)(C * a.h_row * 2));
+    const __amdgpu_buffer_rsrc_t r2 = make_rsrc(a.wg, (uint32_t)(C * a.c_row * 2));
+#pragma unroll
+    for (int j = 0; j < WT / 8 / 512; ++j) {
+      const int id = tid + 512 * j, m = id >> 4, c = (id & 15) * 8;
+      const int o = (c >> 6) * kWide * 64 + wide_off(m, c & 63);
+      const uint4 u1 = buffer_load16(r1, m < C && c < a.h_row ? (uint32_t)((m * a.h_row + c) * 2) : kOut);
+      const uint4 u2 = buffer_load16(r2, m < C && c < a.c_row ? (uint32_t)((m * a.c_row + c) * 2) : kOut);
+      *reinterpret_cast<uint4*>(&wo_l[o]) = u1;
+      *reinterpret_cast<uint4*>(&wg_l[o]) = u2;
+    }
+  }
+
+  const int ch = 32 * grp + lq;  // this lane's channel
+  const float bv = a.bo && ch < C ? a.bo[ch] : 0.f;
+  const float bg = a.bg && ch < C ? -a.bg[ch] * kLog2e : 0.f;
+  float bsum_v = 0.f, bsum_g = 0.f;
+  f32x16 gv[4], gg[4];  // d_Wo and d_Wg of the wave's channels, columns 32 n ..
+#pragma unroll
+  for (int n = 0; n < 4; ++n) gv[n] = gg[n] = f32x16{};
+
+  // tile it's rows into its slot by direct-to-LDS loads (rows past R: zeros): this lane's row and columns of
+  // the wave's two 1 KB pieces of each input
+  int d_row[2], d_col[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int slot = (wave * 2 + k) * 64 + lane;
+    d_row[k] = (slot >> 3) % RT;
+    d_col[k] = (slot / (RT * 8)) * 64 + (wide_off(d_row[k], (slot & 7) * 8) - d_row[k] * 64);
+  }
+  auto request = [&](int it) {
+    const int64_t r0 = (tile0 + it) * RT;
+    const int64_t left = it < count ? R - r0 : 0;
+    const int nrows = (int)(left < RT ? left : RT);
+    const int64_t base = nrows ? r0 : 0;
+    const u32x4 s1 = rsrc_words(static_cast<const T*>(a.nrm) + base * a.h_row, (uint32_t)(nrows * a.h_row * 2));
+    const u32x4 s2 = rsrc_words(static_cast<const T*>(a.xn) + base * a.c_row, (uint32_t)(nrows * a.c_row * 2));
+    // d_out rows: of the tile, or of the pair's cells from the tile's first grid row on
+    int64_t u0 = base;
+    uint32_t u_bytes = (uint32_t)(nrows * C * 2), i0 = 0;
+    if (a.n) {
+      i0 = (uint32_t)base / a.n_pad;
+      const bool in = nrows && i0 < a.n;
+      u0 = in ? (int64_t)i0 * a.n : 0;
+      u_bytes = in ? (uint32_t)(((int64_t)a.n * a.n - u0) * C * 2) : 0u;
+    }
+    const u32x4 s3 = rsrc_words(static_cast<const T*>(a.gout) + u0 * C, u_bytes);
+    T* const at = lds + 2 * WT + (it & 1) * 3 * TILE + wave * 1024;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int r = d_row[k], c = d_col[k];
+      const bool ok = r < nrows;
+      dma16_asm(s1, at + 512 * k, ok && c < a.h_row ? (uint32_t)((r * a.h_row + c) * 2) : kOut, 0);
+      dma16_asm(s2, at + TILE + 512 * k, ok && c < a.c_row ? (uint32_t)((r * a.c_row + c) * 2) : kOut, 0);
+      uint32_t u = (uint32_t)r;
+      bool live = ok && c < C;
+      if (a.n) {
+        const uint32_t p = (uint32_t)base + (uint32_t)r, i = p / a.n_pad, j = p - i * a.n_pad;
+        u = (i - i0) * a.n + j;
+        live = live && i < a.n && j < a.n;
+      }
+      dma16_asm(s3, at + 2 * TILE + 512 * k, live ? (u * (uint32_t)C + (uint32_t)c) * 2 : kOut, 0);
+    }
+  };
+  vmem_wait_all();  // no compiler-visible load outstanding once the requests start
+  request(0);
+
+  const TrLane t0 = wide_tr_lane(lane, 0), t1 = wide_tr_lane(lane, 32);
+  const TrLane tg = grp & 1 ? t1 : t0, tt = th ? t1 : t0;
+  const int c0 = 32 * grp + 16 * g2;
+  for (int it = 0; it < count; ++it) {
+    // tile it has arrived (four stores per iteration were issued after its request)
+    if (it > 0)
+      vmem_wait<4>();
+    else
+      vmem_wait<0>();
+    lds_barrier();  // the tile (and the weights) are written; every wave is done with the other slot
+    request(it + 1);
+    T* const nrm_l = lds + 2 * WT + (it & 1) * 3 * TILE;
+    T* const xn_l = nrm_l + TILE;
+    T* const do_l = xn_l + TILE;
+    T* const ex_l = nrm_l;
+    const int64_t r0 = (tile0 + it) * RT + 32 * th;  // this wave's tokens
+
+    // ---- projections: lane = channel, entry 4q + i = token 8q + 4 g2 + i.  Each SIMD holds one wave of
+    // either token half: one half's MFMAs first, so that the other's run beside its arithmetic
+    if (th == 0) __builtin_amdgcn_s_setprio(2);
+    f32x16 av, ag;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const int col = (16 * ks & 63) + 8 * g2;
+      const int xo = (ks >> 2) * RT * 64 + wide_off(32 * th + lq, col), wo = (ks >> 2) * kWide * 64 + wide_off(ch, col);
+      av = E::mma(lds_frag<T>(nrm_l + xo), lds_frag<T>(wo_l + wo), ks == 0 ? f32x16{} : av);
+      ag = E::mma(lds_frag<T>(xn_l + xo), lds_frag<T>(wg_l + wo), ks == 0 ? f32x16{} : ag);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    uint32_t pv[8], pg[8];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int slab = (32 * th + 16 * ks) * 64;
+      const Frag df = lds_read_tr_frag_sw<T>(do_l + (grp >> 1) * RT * 64 + slab + 32 * (grp & 1), tg);
+#pragma unroll
+      for (int qq = 0; qq < 2; ++qq) {
+        const int q = 2 * ks + qq;
+        float o[4], og[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = av[4 * q + i] + bv, d = (float)df[4 * qq + i];
+          const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(ag[4 * q + i], -kLog2e, bg)));
+          o[i] = d * s;
+          og[i] = d * v * s * (1.f - s);
+        }
+        bsum_v += (o[0] + o[1]) + (o[2] + o[3]);
+        bsum_g += (og[0] + og[1]) + (og[2] + og[3]);
+        pv[2 * q] = pack2<T>(o[0], o[1]), pv[2 * q + 1] = pack2<T>(o[2], o[3]);
+        pg[2 * q] = pack2<T>(og[0], og[1]), pg[2 * q + 1] = pack2<T>(og[2], og[3]);
+      }
+      // ---- d_Wo += g_value^T nrm, d_Wg += g_gate^T xn
+      const Frag fv = __builtin_bit_cast(Frag, make_uint4(pv[4 * ks], pv[4 * ks + 1], pv[4 * ks + 2], pv[4 * ks + 3]));
+      const Frag fg = __builtin_bit_cast(Frag, make_uint4(pg[4 * ks], pg[4 * ks + 1], pg[4 * ks + 2], pg[4 * ks + 3]));
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const int at = (n >> 1) * RT * 64 + slab + 32 * (n & 1);
+        gv[n] = E::mma(fv, lds_read_tr_frag_sw<T>(nrm_l + at, (n & 1) ? t1 : t0), gv[n]);
+        gg[n] = E::mma(fg, lds_read_tr_frag_sw<T>(xn_l + at, (n & 1) ? t1 : t0), gg[n]);
+      }
+    }
+    // ---- exchange: [m][64 tokens], m = channel (value), 128 + channel (gate)
+    lds_barrier();  // every wave is done with the inputs
+    uint4 lo, hi;
+    trade16(pv, lo, hi);
+    *reinterpret_cast<uint4*>(&ex_l[wide_off(ch, 32 * th + 16 * g2)]) = lo;
+    *reinterpret_cast<uint4*>(&ex_l[wide_off(ch, 32 * th + 16 * g2 + 8)]) = hi;
+    trade16(pg, lo, hi);
+    *reinterpret_cast<uint4*>(&ex_l[wide_off(kWide + ch, 32 * th + 16 * g2)]) = lo;
+    *reinterpret_cast<uint4*>(&ex_l[wide_off(kWide + ch, 32 * th + 16 * g2 + 8)]) = hi;
+    lds_barrier();  // exchange written
+
+    // ---- d_nrm and d_xn: columns 32 grp .., tokens 32 th ..; lane = token
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const T* wt = (k ? wg_l : wo_l) + (grp >> 1) * kWide * 64 + 32 * (grp & 1);
+      const T* et = ex_l + k * kWide * 64 + 32 * th;
+      f32x16 acc;
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks)
+        acc = E::mma(lds_read_tr_frag_sw<T>(wt + 16 * ks * 64, tg), lds_read_tr_frag_sw<T>(et + 16 * ks * 64, tt),
+                     ks == 0 ? f32x16{} : acc);
+      uint32_t p[8];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        p[2 * q] = pack2<T>(acc[4 * q], acc[4 * q + 1]);
+        p[2 * q + 1] = pack2<T>(acc[4 * q + 2], acc[4 * q + 3]);
+      }
+      trade16(p, lo, hi);
+      const int width = k ? C : H;
+      const int64_t left = R - r0;
+      const int nrows = (int)(left < 0 ? 0 : left < 32 ? left : 32);
+      const __amdgpu_buffer_rsrc_t ds =
+          make_rsrc(static_cast<T*>(k ? a.d_xn : a.d_nrm) + (nrows ? r0 : 0) * width, (uint32_t)(nrows * width * 2));
+      const uint32_t off = (uint32_t)((lq * width + c0) * 2);
+      buffer_store16(ds, lq < nrows && c0 < width ? off : kOut, lo);
+      buffer_store16(ds, lq < nrows && c0 + 8 < width ? off + 16 : kOut, hi);
+    }
+  }
+
+  // the second token half's sums through LDS (32 KB per channel group, then the bias sums)
+  vmem_wait_all();  // the last request has landed
+  __syncthreads();
+  float* const red = reinterpret_cast<float*>(lds) + grp * 128 * 64;
+  float* const bred = reinterpret_cast<float*>(lds) + 4 * 128 * 64;
+  bsum_v += __shfl_xor(bsum_v, 32);
+  bsum_g += __shfl_xor(bsum_g, 32);
+  if (th == 1) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        red[(16 * n + e) * 64 + lane] = gv[n][e];
+        red[(64 + 16 * n + e) * 64 + lane] = gg[n][e];
+      }
+    if (g2 == 0) bred[ch] = bsum_v, bred[kWide + ch] = bsum_g;
+  }
+  __syncthreads();
+  if (th == 0) {
+    float* op = a.wo_parts + run * C * H;
+    float* gp = a.wg_parts + run * C * C;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int c = 32 * n + lq;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 32 * grp + 8 * q + 4 * g2 + i, e = 4 * q + i;
+          if (m < C && c < H) op[(int64_t)m * H + c] = gv[n][e] + red[(16 * n + e) * 64 + lane];
+          if (m < C && c < C) gp[(int64_t)m * C + c] = gg[n][e] + red[(64 + 16 * n + e) * 64 + lane];
+        }
+    }
+    if (g2 == 0 && ch < C) {
+      a.b_parts[run * C + ch] = bsum_v + bred[ch];
+      a.b_parts[(a.runs + run) * C + ch] = bsum_g + bred[kWide + ch];
+    }
+  }
+}
+
 struct GradRuns {
   int tpw;
   int64_t runs;
 };
-GradRuns grad_runs(const oops_trimul_geometry& g) {
-  const int64_t tiles = g.groups * g.positions / kTok;
+GradRuns grad_runs(const oops_trimul_geometry& g, int tokens) {
+  const int64_t tiles = (g.groups * g.positions + tokens - 1) / tokens;
   const int64_t tpw = std::max<int64_t>(kGradMinTiles, (tiles + kGradWgs - 1) / kGradWgs);
   return {(int)tpw, (tiles + tpw - 1) / tpw};
 }
@@ -311,7 +573,7 @@ int64_t trimul_factor_grad_parts(const oops_trimul_geometry& g) {
   if (g.dtype != OOPS_BF16 && g.dtype != OOPS_F16) return 0;
   if (g.hidden <= 64 || g.hidden > kWide || g.c_row <= 64 || g.c_row > kWide || g.channels % 8 || g.c_row % 8) return 0;
   if (g.groups < 1 || g.positions < kTok || g.positions % kTok) return 0;
-  return grad_runs(g).runs;
+  return grad_runs(g, kTok).runs;
 }
 
 hipError_t launch_trimul_factor_grad(const oops_trimul_geometry& g, const void* normalized, const void* weight,
@@ -322,7 +584,7 @@ hipError_t launch_trimul_factor_grad(const oops_trimul_geometry& g, const void* 
   a.d_xn = grad_xn, a.w_parts = w_parts, a.b_parts = b_parts;
   a.rows = g.groups * g.positions, a.positions = g.positions, a.groups = g.groups;
   a.C = g.channels, a.H = g.hidden, a.c_row = (int)g.c_row;
-  const GradRuns pl = grad_runs(g);
+  const GradRuns pl = grad_runs(g, kTok);
   a.tpw = pl.tpw, a.runs = pl.runs;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)xcd_grid(a.runs, 0)), dim3(512), 0, stream, a);
@@ -332,6 +594,36 @@ hipError_t launch_trimul_factor_grad(const oops_trimul_geometry& g, const void* 
     return mask ? go(trimul_factor_grad_kernel<__bf16, true>) : go(trimul_factor_grad_kernel<__bf16, false>);
   if (g.dtype == OOPS_F16)
     return mask ? go(trimul_factor_grad_kernel<_Float16, true>) : go(trimul_factor_grad_kernel<_Float16, false>);
+  return hipErrorInvalidValue;
+}
+
+int64_t trimul_output_grads_parts(const oops_trimul_geometry& g) {
+  if (g.dtype != OOPS_BF16 && g.dtype != OOPS_F16) return 0;
+  if (g.hidden <= 64 || g.hidden > kWide || g.channels <= 64 || g.channels > kWide) return 0;
+  if (g.channels % 8 || g.hidden % 8 || g.c_row != g.channels || g.h_row != g.hidden) return 0;
+  if (g.groups < 1 || g.positions < 1 || g.groups * g.positions >= (int64_t(1) << 31)) return 0;
+  return grad_runs(g, kOutTok).runs;
+}
+
+hipError_t launch_trimul_output_grads(const oops_trimul_geometry& g, int64_t n, int64_t n_pad, const void* normalized,
+                                      const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                      const float* output_bias, const float* gate_bias, const void* grad_out,
+                                      void* grad_normalized, void* grad_xn, float* wo_parts, float* wg_parts,
+                                      float* b_parts, hipStream_t stream) {
+  OutputGradArgs a{};
+  a.nrm = normalized, a.xn = pair_normalized, a.wo = output_weight, a.wg = gate_weight;
+  a.bo = output_bias, a.bg = gate_bias, a.gout = grad_out, a.d_nrm = grad_normalized, a.d_xn = grad_xn;
+  a.wo_parts = wo_parts, a.wg_parts = wg_parts, a.b_parts = b_parts;
+  a.rows = g.groups * g.positions, a.C = g.channels, a.H = g.hidden, a.c_row = (int)g.c_row, a.h_row = (int)g.h_row;
+  a.n = (uint32_t)n, a.n_pad = (uint32_t)n_pad;
+  const GradRuns pl = grad_runs(g, kOutTok);
+  a.tpw = pl.tpw, a.runs = pl.runs;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)xcd_grid(a.runs, 0)), dim3(512), 0, stream, a);
+    return hipGetLastError();
+  };
+  if (g.dtype == OOPS_BF16) return go(trimul_output_grads_kernel<__bf16>);
+  if (g.dtype == OOPS_F16) return go(trimul_output_grads_kernel<_Float16>);
   return hipErrorInvalidValue;
 }
 

@@ -60,6 +60,14 @@ hipError_t launch_trimul_factor_grad(const oops_trimul_geometry& g, const void* 
                                      const float* bias, const float* mask, const void* grad_factors, void* grad_xn,
                                      float* w_parts, float* b_parts, hipStream_t stream);
 
+// the gated output's backward with its products in one pass (trimul_grad.hip, oops_trimul_output_grads)
+int64_t trimul_output_grads_parts(const oops_trimul_geometry& g);
+hipError_t launch_trimul_output_grads(const oops_trimul_geometry& g, int64_t n, int64_t n_pad, const void* normalized,
+                                      const void* pair_normalized, const void* output_weight, const void* gate_weight,
+                                      const float* output_bias, const float* gate_bias, const void* grad_out,
+                                      void* grad_normalized, void* grad_xn, float* wo_parts, float* wg_parts,
+                                      float* b_parts, hipStream_t stream);
+
 // float32 pairs (trimul_f32.hip): the same contracts on the exact float32 matrix core
 hipError_t launch_trimul_factors_f32(const oops_trimul_geometry& g, const void* normalized, const void* weight,
                                      const float* bias, const void* mask, void* factors, const void* grad_factors,

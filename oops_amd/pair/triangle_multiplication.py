@@ -501,34 +501,33 @@ def _backward_impl(dout: Tensor, pair: Tensor, mask: Optional[Tensor], w_cat: Te
         return pair.new_empty(0, dtype=torch.float32)
 
     with _on_device(dev):
-        g_val = torch.empty(R, cp, dtype=dtype, device=dev)
-        g_gate = torch.empty(R, cp, dtype=dtype, device=dev)
-        ptrs = (_ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog), _ptr(bo), _ptr(bog), _ptr(dout), _ptr(g_val), _ptr(g_gate),
-                stream)  # fmt: skip
-        _lib.check(lib.oops_trimul_output_pair_backward(ctypes.byref(geo), n, side, *ptrs) if n else
-                   lib.oops_trimul_output_backward(ctypes.byref(geo), *ptrs),
-                   "triangle_multiplication output backward")  # fmt: skip
-        gv, gg = g_val[:, :C], g_gate[:, :C]
         # every float32 partial (K-chunk products, per-workgroup sums) is summed by one launch at the end
         sums = PartialSums()
-        parts = lib.oops_trimul_output_grad_parts(ctypes.byref(geo))
+        saved = (_ptr(nrm), _ptr(xn), _ptr(wo), _ptr(wog), _ptr(bo), _ptr(bog), _ptr(dout))
+        parts = lib.oops_trimul_output_grads_parts(ctypes.byref(geo))
         if parts:
-            # C = H = 128: one pass over each gradient gives its GEMM with the weight, its weight-gradient
-            # and bias-gradient partials (oops_trimul_output_grad_products)
+            # one pass: the output backward, its products with the weights and with the saved rows
             d_nrm = torch.empty(R, H, dtype=dtype, device=dev)
             d_xn = torch.empty(R, C, dtype=dtype, device=dev)
-            g_parts = torch.empty(2, parts, C, C, dtype=torch.float32, device=dev)
-            s_parts = torch.empty(2, parts, C, dtype=torch.float32, device=dev)
-            for i, (x, w, y, d) in enumerate(((g_val, wo, nrm, d_nrm), (g_gate, wog, xn, d_xn))):
-                _lib.check(lib.oops_trimul_output_grad_products(
-                    ctypes.byref(geo), _ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(y), y.stride(0), _ptr(d),
-                    d.stride(0), _ptr(g_parts[i]), _ptr(s_parts[i]), stream), "triangle_multiplication output gradients")  # fmt: skip
-            d_wo, d_wog = sums.add(g_parts[0], dtype), sums.add(g_parts[1], dtype)
+            wo_parts = torch.empty(parts, C, H, dtype=torch.float32, device=dev)
+            wog_parts = torch.empty(parts, C, C, dtype=torch.float32, device=dev)
+            b_parts = torch.empty(2, parts, C, dtype=torch.float32, device=dev)
+            _lib.check(lib.oops_trimul_output_grads(ctypes.byref(geo), n, side, *saved, _ptr(d_nrm), _ptr(d_xn),
+                                                    _ptr(wo_parts), _ptr(wog_parts), _ptr(b_parts), stream),
+                       "triangle_multiplication output gradients")  # fmt: skip
+            d_wo, d_wog = sums.add(wo_parts, dtype), sums.add(wog_parts, dtype)
             if bo is not None:
-                sums.add(s_parts[0], out=d_views[1])
+                sums.add(b_parts[0], out=d_views[1])
             if bog is not None:
-                sums.add(s_parts[1], out=d_views[2])
+                sums.add(b_parts[1], out=d_views[2])
         else:
+            g_val = torch.empty(R, cp, dtype=dtype, device=dev)
+            g_gate = torch.empty(R, cp, dtype=dtype, device=dev)
+            ptrs = (*saved, _ptr(g_val), _ptr(g_gate), stream)
+            _lib.check(lib.oops_trimul_output_pair_backward(ctypes.byref(geo), n, side, *ptrs) if n else
+                       lib.oops_trimul_output_backward(ctypes.byref(geo), *ptrs),
+                       "triangle_multiplication output backward")  # fmt: skip
+            gv, gg = g_val[:, :C], g_gate[:, :C]
             d_nrm = gv.mm(wo[:, :H]).contiguous()  # (R, H)
             d_xn = gg.mm(wog[:, :C])  # (R, C)
             d_wo = sums.add(_long_k_partials(gv.t(), nrm[:, :H]), dtype)

@@ -1,5 +1,5 @@
-"""The triangle multiplication's factor backward with its products in one pass (oops_trimul_factor_grads)
-against the separate factor backward (oops_trimul_factors_backward, the same 16-bit projection gradients) and
+"""The triangle multiplication's factor and output backwards, each with its products in one pass
+(oops_trimul_factor_grads, oops_trimul_output_grads).  The factor pass is held against the separate factor backward (oops_trimul_factors_backward, the same 16-bit projection gradients) and
 float64 products of its result: one tile and several runs of tiles, groups that end inside a run, channel and
 hidden sizes below 128, with and without a mask and biases."""
 
@@ -68,6 +68,70 @@ def test_factor_grads(dtype, groups, positions, c, h, masked, biases):
     # the separate backward sums the same float32 values
     want, mag = old_b.double().sum(0), p64.abs().sum(1)
     assert ((bp.double().sum(0) - want).abs() <= 8 * R**0.5 * 2.0**-24 * mag + 1e-6).all()
+
+
+@pytest.mark.parametrize(
+    "dtype,groups,positions,n,c,h,biases",
+    [
+        (torch.bfloat16, 1, 1, 0, 128, 128, True),  # one row; either side of a 64-row tile
+        (torch.float16, 3, 173, 0, 128, 72, False),
+        (torch.bfloat16, 1, 64 * 64, 61, 128, 128, True),  # a 61 x 61 pair on a 64 x 64 grid of rows
+        (torch.float16, 1, 104 * 104, 99, 96, 128, True),
+        (torch.bfloat16, 7, 4097, 0, 120, 104, True),
+        (torch.bfloat16, 1, 300 * 300, 0, 128, 128, True),
+    ],
+)
+def test_output_grads(dtype, groups, positions, n, c, h, biases):
+    """oops_trimul_output_grads against the separate output backward (oops_trimul_output_backward) and float64
+    products of its 16-bit gradients."""
+
+    lib = _lib.load()
+    gen = torch.Generator(device=DEV).manual_seed(positions)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=gen)  # noqa: E731
+    R = groups * positions
+    nrm, xn = rand(R, h).to(dtype), rand(R, c).to(dtype)
+    wo, wg = (rand(c, h) * h**-0.5).to(dtype), (rand(c, c) * c**-0.5).to(dtype)
+    bo, bg = (rand(c), rand(c)) if biases else (None, None)
+    gout = rand(n * n if n else R, c).to(dtype)
+    side = round(positions**0.5) if n else 0
+    if n:  # the same gradient on the grid of rows
+        full = torch.zeros(side, side, c, dtype=dtype, device=DEV)
+        full[:n, :n] = gout.view(n, n, c)
+        full = full.view(R, c)
+    else:
+        full = gout
+    geo = _lib.TrimulGeometry()
+    geo.dtype = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16
+    geo.channels, geo.hidden, geo.has_mask = c, h, 0
+    geo.groups, geo.positions, geo.c_row, geo.h_row, geo.eps = groups, positions, c, h, 1e-5
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    stream = torch.cuda.current_stream().cuda_stream
+    saved = [ptr(t) for t in (nrm, xn, wo, wg, bo, bg)]
+    g_val, g_gate = torch.empty(R, c, dtype=dtype, device=DEV), torch.empty(R, c, dtype=dtype, device=DEV)
+    assert 0 == lib.oops_trimul_output_backward(ctypes.byref(geo), *saved, ptr(full), ptr(g_val), ptr(g_gate),
+                                                stream), lib.oops_last_error()
+    parts = lib.oops_trimul_output_grads_parts(ctypes.byref(geo))
+    assert 1 <= parts <= 256
+    d_nrm, d_xn = torch.empty(R, h, dtype=dtype, device=DEV), torch.empty(R, c, dtype=dtype, device=DEV)
+    nan = float("nan")
+    wop, wgp = torch.full((parts, c, h), nan, device=DEV), torch.full((parts, c, c), nan, device=DEV)
+    bp = torch.full((2, parts, c), nan, device=DEV)
+    assert 0 == lib.oops_trimul_output_grads(ctypes.byref(geo), n, side, *saved, ptr(gout), ptr(d_nrm), ptr(d_xn),
+                                             ptr(wop), ptr(wgp), ptr(bp), stream), lib.oops_last_error()
+    torch.cuda.synchronize()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for k, (g, w, rows, d, wp) in enumerate(((g_val, wo, nrm, d_nrm, wop), (g_gate, wg, xn, d_xn, wgp))):
+        g64, w64, r64 = g.double(), w.double(), rows.double()
+        # the gradients themselves may round one way here and the other way there (one unit of each); then one
+        # rounding of a float32 sum of c terms
+        mag = g64.abs() @ w64.abs()
+        flips = unit * mag
+        assert ((d.double() - g64 @ w64).abs() <= unit * (g64 @ w64).abs() + flips + c * 2.0**-24 * mag + 1e-7).all()
+        mag = g64.abs().t() @ r64.abs()
+        bound = 4 * R**0.5 * 2.0**-24 * mag + unit * mag / max(1.0, R**0.5) * 8 + 1e-9
+        assert ((wp.double().sum(0) - g64.t() @ r64).abs() <= bound).all()
+        # the bias sums take the float32 values: half a unit of each against the rounded ones
+        assert ((bp[k].double().sum(0) - g64.sum(0)).abs() <= unit * g64.abs().sum(0) + 1e-6).all()
 
 
 def test_factor_grads_served_range():
