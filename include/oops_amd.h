@@ -217,7 +217,7 @@ int oops_gate_multiply_backward(const oops_gate_geometry* geo, const void* atten
                                 const void* grad, void* grad_attention, void* grad_logits, void* stream);
 
 /* The whole stage in one pass over its rows (16-bit dtypes; C, D and O multiples of 8, C, H*D and O at most
- * 256, a_sd = 1, 16-byte aligned rows, attention values within 2 GiB):
+ * 256, or 384 up to 16384 rows, a_sd = 1, 16-byte aligned rows, attention values within 2 GiB):
  *   forward: out [rows][O] = gated . Wo^T, Wo [O][H*D] (row stride wo_row); logits kept unless NULL.
  *   backward: from grad [rows][O] (the gradient of out) the attention and logit gradients of
  *     oops_gate_multiply_backward applied to grad . Wo, and float32 partials of Wo's gradient
@@ -236,7 +236,7 @@ int oops_gate_stage_backward(const oops_gate_geometry* geo, int64_t out_channels
                              void* grad_attention, void* grad_logits, float* g_parts, void* stream);
 
 /* Gradient products of a linear layer over many rows in one pass (16-bit; k and n multiples of 8 and at most
- * 256, 16-byte aligned rows): d [rows][n] = x . w (x [rows][k], w [k][n]) and float32 partials
+ * 384, 16-byte aligned rows): d [rows][n] = x . w (x [rows][k], w [k][n]) and float32 partials
  * [parts][k][n] of x^T . y (y [rows][n]).  parts = oops_linear_grad_parts (0: not served). */
 size_t oops_linear_grad_parts(int32_t dtype, int64_t rows, int64_t k, int64_t n);
 int oops_linear_grad_products(int32_t dtype, int64_t rows, int64_t k, int64_t n, const void* x, int64_t x_row,

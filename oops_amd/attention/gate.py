@@ -8,9 +8,9 @@ oops/attention/pair_bias/gated_pair_bias_attention.py:33-126):
 
 ``attention`` is head-major ``(*prefix, H, Q, D)``; its ``(Q, H, D)`` view is
 read in place through its strides (no transposed copy).  On the GPU an eager
-16-bit call of at most 256 channels on each side runs as one HIP kernel
-forward and two backward (``_EagerStage``: every tensor is read and written
-once).  Wider 16-bit operands and traced code run the gate projection, the
+16-bit call of at most 256 channels on each side (384 for few rows) runs as one
+HIP kernel forward and two backward (``_EagerStage``: every tensor is read and
+written once).  Wider 16-bit operands and traced code run the gate projection, the
 sigmoid and the product in one HIP kernel (MFMA, the logits kept for the
 backward); other dtypes and layouts compute the logits with ``F.linear`` and
 apply the gate with the HIP elementwise kernel; the output projection and the

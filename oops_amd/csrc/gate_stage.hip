@@ -1,4 +1,5 @@
-// The gated output stage as whole passes over its rows (gfx950, 16-bit operands, C, H*D and O at most 256):
+// The gated output stage as whole passes over its rows (gfx950, 16-bit operands, C, H*D and O at most 256, or
+// at most 384 for few rows):
 //
 //   forward       out = (round(sigmoid(single Wg^T)) * attention) Wo^T           gate_stage_forward_kernel
 //   backward 1    d_gated = d_out Wo, its gate backward, d_Wo = d_out^T gated    row_grad_kernel<GATE>
@@ -17,7 +18,8 @@
 // library GEMMs, chunked weight gradients): forward 108 us for 149, backward 1 142 us for 205, backward 2
 // 85 us for 119, the stage forward and backward 484 -> 306 us.  Few rows gain from the launches: 128 rows
 // forward 50 -> 18 us, forward and backward 256 -> 183 us, so there is no lower limit on the rows.  The
-// upper limit of 256 channels is the register file: a wider weight does not fit beside the accumulators.
+// upper limits are the register file's: both 256-wide weights fit beside the forward's accumulators, a 384-wide
+// one beside the gradients' (with a few spilled registers).
 //
 // A tile is stored as 64-column panels [row][64] with XOR-swizzled 16-byte chunks, so that a row-fragment
 // read (one operand of X W) and a transposed read (both operands of X^T Y) come from the same copy.
@@ -37,6 +39,12 @@ namespace {
 constexpr int kStageCols = 128;  // columns of D and of the weight gradient per workgroup (row_grad_kernel)
 constexpr int kStageRows = 64;   // rows per tile (row_grad_kernel)
 constexpr int kStageWgs = 256;   // workgroups: one per CU
+constexpr int kWideCols = 384;   // the largest C, H*D and O
+// Past 256 channels the forward streams its weights for every 32 rows, which is right for few rows only: forward
+// / forward and backward at 384 channels, eager, against the separate launches: 384 rows 23 / 128 us for 65 / 239,
+// 16384 rows 42 / 120 us for 72 / 304 (replayed from a graph, without host time: 32 / 55 for 26 / 46 and 46 /
+// 116 for 41 / 155).  Further up the streamed weights cost more than the launches save.
+constexpr int64_t kWideRows = 16384;
 
 struct StageArgs {
   const void* x;       // forward: single [rows][kx]; gradients: X [rows][kx]
@@ -228,8 +236,9 @@ __global__ __launch_bounds__(512, 2) void gate_stage_forward_kernel(StageArgs a)
     }
     uint4* p0 = reinterpret_cast<uint4*>(yt + panel_off<RT>(row, c0));
     uint4* p1 = reinterpret_cast<uint4*>(yt + panel_off<RT>(row, c0 + 8));
-    *p0 = gate_product<T>(lo, *p0);
-    *p1 = gate_product<T>(hi, *p1);
+    // (columns past H*D stay zero whatever their padded logits are: an infinite `single` makes those NaN)
+    *p0 = c0 < a.n ? gate_product<T>(lo, *p0) : make_uint4(0, 0, 0, 0);
+    *p1 = c0 + 8 < a.n ? gate_product<T>(hi, *p1) : make_uint4(0, 0, 0, 0);
     lds_barrier();  // gated rows written
     f32x16 acc = f32x16{};
 #pragma unroll
@@ -244,9 +253,89 @@ __global__ __launch_bounds__(512, 2) void gate_stage_forward_kernel(StageArgs a)
   vmem_wait_all();  // the ring's last requests land before the LDS is given back
 }
 
+constexpr int kWideThreads = kWideCols / 32 * 64;
+
+// The forward for up to 384 channels and few rows (the single representation): one 32-row tile per workgroup,
+// the weights' fragments straight from L2 (they do not fit in a workgroup's registers beside each other).  One
+// wave per 32 channels, all of its fragments in flight at once.
+template <typename T, bool LOGITS>
+__global__ __launch_bounds__(kWideThreads, 3) void gate_stage_wide_kernel(StageArgs a) {
+  using E = Elem<T>;
+  using Frag = typename E::Frag;
+  constexpr int RT = 32, P = kWideCols, KS = P / 16;
+  __shared__ __attribute__((aligned(16))) T x_lds[RT * P];
+  __shared__ __attribute__((aligned(16))) T y_lds[RT * P];  // attention -> gated
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 31, g2 = lane >> 5;
+  const int64_t r0 = (int64_t)blockIdx.x * RT;
+  const int nrows = (int)(a.rows - r0 < RT ? a.rows - r0 : RT);
+  auto load_block = [&](const void* w, int64_t w_row, int rows, int k_end, Frag (&f)[KS]) {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(w, (uint32_t)(((rows - 1) * w_row + k_end) * 2));
+    const int c = 32 * wave + lq;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int k = 16 * ks + 8 * g2;
+      f[ks] = __builtin_bit_cast(Frag, buffer_load16(rs, c < rows && k < k_end ? (uint32_t)((c * w_row + k) * 2) : kOut));
+    }
+  };
+  Frag wf[KS];
+  load_block(a.w, a.w_row, a.n, a.kx, wf);
+  {
+    const __amdgpu_buffer_rsrc_t xs =
+        make_rsrc(static_cast<const T*>(a.x) + r0 * a.x_row, (uint32_t)(((nrows - 1) * a.x_row + a.kx) * 2));
+    const __amdgpu_buffer_rsrc_t ys = make_rsrc(a.y, a.a_bytes);
+#pragma unroll
+    for (int j = 0; j < RT * P / 8 / kWideThreads; ++j) {
+      const int id = tid + kWideThreads * j, r = id / (P / 8), c = (id % (P / 8)) * 8;
+      const bool ok = r < nrows;
+      const uint4 xv = buffer_load16(xs, ok && c < a.kx ? (uint32_t)((r * a.x_row + c) * 2) : kOut);
+      const uint4 yv = buffer_load16(
+          ys, ok && c < a.n ? att_row_bytes(a, (uint32_t)r0 + r) + 2 * ((uint32_t)(c / a.width) * a.a_sh + (uint32_t)(c % a.width))
+                            : kOut);
+      *reinterpret_cast<uint4*>(&x_lds[panel_off<RT>(r, c)]) = xv;
+      *reinterpret_cast<uint4*>(&y_lds[panel_off<RT>(r, c)]) = yv;
+    }
+  }
+  __syncthreads();
+
+  auto product = [&](const T* tile, const Frag (&f)[KS], uint4& lo, uint4& hi) {
+    f32x16 acc = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = E::mma(f[ks], lds_frag<T>(tile + panel_off<RT>(lq, 16 * ks + 8 * g2)), acc);
+    round_run<T>(acc, lo, hi);
+  };
+  uint4 lo, hi;
+  if (32 * wave < a.n) {
+    product(x_lds, wf, lo, hi);
+    const int c0 = 32 * wave + 16 * g2;
+    if constexpr (LOGITS) {
+      const __amdgpu_buffer_rsrc_t lr = make_rsrc(static_cast<T*>(a.e) + r0 * a.n, (uint32_t)(nrows * a.n * 2));
+      const uint32_t off = (uint32_t)((lq * a.n + c0) * 2);
+      buffer_store16(lr, lq < nrows && c0 < a.n ? off : kOut, lo);
+      buffer_store16(lr, lq < nrows && c0 + 8 < a.n ? off + 16 : kOut, hi);
+    }
+    uint4* p0 = reinterpret_cast<uint4*>(y_lds + panel_off<RT>(lq, c0));
+    uint4* p1 = reinterpret_cast<uint4*>(y_lds + panel_off<RT>(lq, c0 + 8));
+    // (columns past H*D stay zero whatever their padded logits are: an infinite `single` makes those NaN)
+    *p0 = c0 < a.n ? gate_product<T>(lo, *p0) : make_uint4(0, 0, 0, 0);
+    *p1 = c0 + 8 < a.n ? gate_product<T>(hi, *p1) : make_uint4(0, 0, 0, 0);
+  }
+  load_block(a.w_out, a.w_out_row, a.o, a.n, wf);
+  __syncthreads();  // gated rows written
+  if (32 * wave < a.o) {
+    product(y_lds, wf, lo, hi);
+    const int c0 = 32 * wave + 16 * g2;
+    const __amdgpu_buffer_rsrc_t orr = make_rsrc(static_cast<T*>(a.d) + r0 * a.o, (uint32_t)(nrows * a.o * 2));
+    const uint32_t off = (uint32_t)((lq * a.o + c0) * 2);
+    buffer_store16(orr, lq < nrows && c0 < a.o ? off : kOut, lo);
+    buffer_store16(orr, lq < nrows && c0 + 8 < a.o ? off + 16 : kOut, hi);
+  }
+}
+
 // ------------------------------------------------------------------ gradients
 // D = X W (the gate's backward applied to it with GATE) and partials of X^T Y (Y = the gated rows with GATE)
-// for 128 columns n0 .. n0 + 127 of W, Y, D and all KX (128 or 256, padded like P above) columns of X.
+// for 128 columns n0 .. n0 + 127 of W, Y, D and all KX (128, 256 or 384, padded like P above) columns of X.
 // Wave (cg, rg) computes columns 32 cg .. + 31 of D's tile rows 32 rg .. + 31, and X columns
 // (KX / 4) cg .. of X^T Y's columns 64 rg .. + 63.  Splitting the columns over workgroups halves the
 // float32 partials (a 256 x 256 partial per CU is 64 MB per launch) and the accumulators; the two
@@ -375,24 +464,21 @@ __global__ __launch_bounds__(512, 2) void row_grad_kernel(StageArgs a) {
     }
     const int n = n0 + c0;
     if constexpr (GATE) {
-      uint4* y0 = reinterpret_cast<uint4*>(yt + panel_off<RT>(row, c0));
-      uint4* y1 = reinterpret_cast<uint4*>(yt + panel_off<RT>(row, c0 + 8));
-      const uint4 l0 = *reinterpret_cast<const uint4*>(yt + YT + panel_off<RT>(row, c0));
-      const uint4 l1 = *reinterpret_cast<const uint4*>(yt + YT + panel_off<RT>(row, c0 + 8));
-      uint4 a0, a1, e0, e1, v0, v1;
-      gate_backward_run<T>(lo, *y0, l0, a0, e0, v0);
-      gate_backward_run<T>(hi, *y1, l1, a1, e1, v1);
-      *y0 = v0;
-      *y1 = v1;
       const uint32_t bytes = (uint32_t)(nrows * a.n * 2);
       const __amdgpu_buffer_rsrc_t ar = make_rsrc(static_cast<T*>(a.d) + r0 * a.n, bytes);
       const __amdgpu_buffer_rsrc_t er = make_rsrc(static_cast<T*>(a.e) + r0 * a.n, bytes);
-      const uint32_t off = (uint32_t)((row * a.n + n) * 2);
-      const uint32_t o0 = row < nrows && n < a.n ? off : kOut, o1 = row < nrows && n + 8 < a.n ? off + 16 : kOut;
-      buffer_store16(ar, o0, a0);
-      buffer_store16(ar, o1, a1);
-      buffer_store16(er, o0, e0);
-      buffer_store16(er, o1, e1);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        uint4* y = reinterpret_cast<uint4*>(yt + panel_off<RT>(row, c0 + 8 * k));
+        const uint4 l = *reinterpret_cast<const uint4*>(yt + YT + panel_off<RT>(row, c0 + 8 * k));
+        uint4 da, dl, gated;
+        gate_backward_run<T>(k ? hi : lo, *y, l, da, dl, gated);
+        *y = gated;
+        const uint32_t off = row < nrows && n + 8 * k < a.n ? (uint32_t)((row * a.n + n + 8 * k) * 2) : kOut;
+        buffer_store16(ar, off, da);
+        buffer_store16(er, off, dl);
+        asm volatile("" ::: "memory");  // one run of eight at a time: fewer live registers
+      }
       lds_barrier();  // gated rows written
     } else {
       const __amdgpu_buffer_rsrc_t dr =
@@ -459,7 +545,7 @@ bool rows_fit(int64_t stride, int64_t count) { return stride * count * 2 < (int6
 
 int64_t row_grad_parts(int dtype, int64_t rows, int64_t k, int64_t n) {
   if (dtype != OOPS_BF16 && dtype != OOPS_F16) return 0;
-  if (rows < 1 || rows >= (int64_t(1) << 31) || k < 8 || k > 256 || n < 8 || n > 256 || k % 8 || n % 8) return 0;
+  if (rows < 1 || rows >= (int64_t(1) << 31) || k < 8 || k > kWideCols || n < 8 || n > kWideCols || k % 8 || n % 8) return 0;
   return run_plan(rows, kStageRows, kStageWgs / ((n + kStageCols - 1) / kStageCols)).runs;
 }
 
@@ -468,6 +554,7 @@ bool gate_stage_ok(const oops_gate_geometry& g, int64_t out_channels, int64_t wo
   const int64_t n = (int64_t)g.heads * g.width;
   if (row_grad_parts(g.dtype, g.rows, n, g.channels) == 0 || row_grad_parts(g.dtype, g.rows, out_channels, n) == 0)
     return false;
+  if (std::max({n, (int64_t)g.channels, out_channels}) > 256 && g.rows > kWideRows) return false;
   if (g.width % 8 || g.a_sd != 1 || g.s_row % 8 || g.w_row % 8 || wo_row % 8) return false;
   int64_t extent = g.width;
   const int64_t sizes[4] = {g.rows / (g.tokens * g.groups), g.groups, g.tokens, g.heads};
@@ -478,8 +565,8 @@ bool gate_stage_ok(const oops_gate_geometry& g, int64_t out_channels, int64_t wo
     if (sizes[i] > 1) extent += (sizes[i] - 1) * strides[i];
   }
   if (g.rows % (g.tokens * g.groups) || extent > (int64_t(1) << 30)) return false;
-  if (g.s_row < 0 || g.w_row < 0 || wo_row < 0 || !rows_fit(g.s_row, kStageRows) || !rows_fit(g.w_row, 256) ||
-      !rows_fit(wo_row, 256))
+  if (g.s_row < 0 || g.w_row < 0 || wo_row < 0 || !rows_fit(g.s_row, kStageRows) || !rows_fit(g.w_row, kWideCols) ||
+      !rows_fit(wo_row, kWideCols))
     return false;
   for (const void* p : {single, weight, attention, output_weight})
     if (reinterpret_cast<uintptr_t>(p) & 15) return false;
@@ -513,7 +600,19 @@ hipError_t launch_gate_stage_forward(const oops_gate_geometry& g, int64_t out_ch
   a.x = single, a.w = weight, a.w_out = output_weight, a.d = out, a.e = logits;
   a.x_row = g.s_row, a.w_row = g.w_row, a.w_out_row = wo_row;
   a.kx = g.channels, a.n = g.heads * g.width, a.o = (int)out_channels;
-  const bool wide = std::max({a.kx, a.n, a.o}) > 128;
+  const int most = std::max({a.kx, a.n, a.o});
+  if (most > 256) {
+    return by_half(g.dtype, [&](auto tag) -> hipError_t {
+      using T = decltype(tag);
+      const dim3 grid((unsigned)((g.rows + 31) / 32));
+      if (logits)
+        hipLaunchKernelGGL((gate_stage_wide_kernel<T, true>), grid, dim3(kWideThreads), 0, stream, a);
+      else
+        hipLaunchKernelGGL((gate_stage_wide_kernel<T, false>), grid, dim3(kWideThreads), 0, stream, a);
+      return hipGetLastError();
+    });
+  }
+  const bool wide = most > 128;
   const RunPlan pl = run_plan(g.rows, wide ? 32 : 64, kStageWgs);
   a.tpw = pl.tpw, a.tiles = pl.runs;
   return by_half(g.dtype, [&](auto tag) -> hipError_t {
@@ -539,7 +638,9 @@ hipError_t launch_row_grad(int dtype, StageArgs& a, hipStream_t stream) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)xcd_grid(a.tiles, 0)), dim3(512), 0, stream, a);
       return hipGetLastError();
     };
-    return a.kx > 128 ? go(row_grad_kernel<T, 256, GATE>) : go(row_grad_kernel<T, 128, GATE>);
+    return a.kx > 256   ? go(row_grad_kernel<T, 384, GATE>)
+           : a.kx > 128 ? go(row_grad_kernel<T, 256, GATE>)
+                        : go(row_grad_kernel<T, 128, GATE>);
   });
 }
 }  // namespace
@@ -561,7 +662,7 @@ bool linear_grads_ok(int dtype, int64_t rows, int64_t k, int64_t n, const void* 
   for (const void* p : {x, w, y, d})
     if (reinterpret_cast<uintptr_t>(p) & 15) return false;
   for (int64_t s : {x_row, w_row, y_row, d_row})
-    if (s < 0 || s % 8 || !rows_fit(s, 256)) return false;
+    if (s < 0 || s % 8 || !rows_fit(s, kWideCols)) return false;
   return x_row >= k && d_row >= n;
 }
 

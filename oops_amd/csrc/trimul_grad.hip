@@ -1,5 +1,6 @@
 // The triangle multiplication's factor and output backwards, each with its products in one pass (gfx950; the
-// output's is below).  The factor projections' backward: 16-bit pairs with 64 < C, H <= 128 and positions a multiple of 32, no mask gradient.
+// output's is below).  The factor projections' backward, for 16-bit pairs with 64 < C, H <= 128 and positions a
+// multiple of 32, without a mask gradient:
 //
 //   value, gate = xn W^T + b (recomputed), d_proj = the gate's backward of the factor gradients
 //   d_xn += d_proj W        d_W = d_proj^T xn        d_b = column sums of d_proj

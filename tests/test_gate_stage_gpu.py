@@ -1,7 +1,7 @@
 """The gated output stage as one pass over its rows (oops_gate_stage_*, oops_linear_grad_products): values and
 gradients against the same formula in float64 on the same 16-bit inputs, at the edges of its row tiles (32 and
-64), of its 128-column blocks and of its 256-channel range, over strided operands, and the forms it hands to
-the separate operators (missing gradients, a second derivative)."""
+64), of its 128-column blocks and of its 256- and 384-channel ranges, over strided operands, with infinite
+inputs, and the forms it hands to the separate operators (missing gradients, a second derivative)."""
 
 import pytest
 import torch
@@ -82,6 +82,10 @@ CASES = [
     ((3,), 5, 45, 24, 96, 40),  # 120 channels in 16-channel runs
     ((3,), 17, 45, 8, 96, 136),
     ((1,), 16, 200, 16, 72, 256),
+    ((1,), 16, 95, 24, 384, 384),  # the wide forward: more than 256 channels somewhere
+    ((2,), 11, 33, 24, 16, 40),
+    ((1,), 2, 129, 16, 264, 8),
+    ((3,), 4, 31, 32, 72, 376),
     ((2, 9), 4, 997, 32, 64, 128),
     ((5,), 8, 4001, 32, 256, 256),
 ]
@@ -142,9 +146,26 @@ def test_gate_stage_not_served():
     """Operands outside the one-pass kernels' range keep the separate operators."""
 
     served = dict(dtype=torch.bfloat16, prefix=(1,), heads=4, q=9, d=32, c=128, o=128)
-    for change in (dict(dtype=torch.float32), dict(d=20), dict(c=264), dict(o=264), dict(heads=9), dict(o=12), dict(c=12)):
+    for change in (dict(dtype=torch.float32), dict(d=20), dict(c=392), dict(o=392), dict(heads=13), dict(o=12), dict(c=12),
+                   dict(c=384, q=16385)):  # fmt: skip
         att, single, wg, wo = _inputs(**{**served, **change})
         att5, rows, weight = G._operands(att.transpose(-3, -2), single, wg, att.dtype)
         assert not G._stage_ok(att5, rows, weight, wo)
         out = oops_amd.gate_attention_output(att, single, wg, wo)
         assert out.shape == (*single.shape[:-1], wo.shape[0])
+
+
+@pytest.mark.parametrize("heads,c,o", [(5, 128, 128), (9, 64, 136), (11, 72, 264)])
+def test_gate_stage_infinite_inputs(heads, c, o):
+    """An infinite input saturates the gates of its row; channels that only pad the kernels' tiles add nothing."""
+
+    att, single, wg, wo = (t.detach() for t in _inputs(torch.bfloat16, (1,), heads, 40, 24, c, o))
+    single[0, 3, 5] = float("inf")
+    att[0, 1, 7, 2] = float("-inf")
+    att5, rows, weight = G._operands(att.transpose(-3, -2), single, wg, torch.bfloat16)
+    assert G._stage_ok(att5, rows, weight, wo)
+    gate = torch.sigmoid((single.double() @ wg.double().t()).float())
+    want = (gate.bfloat16() * att.transpose(-3, -2).flatten(-2)).double() @ wo.double().t()
+    got = oops_amd.gate_attention_output(att, single, wg, wo)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert got[0, 3].isfinite().all()
