@@ -409,7 +409,7 @@ int oops_sum_partials(const oops_sum_segment* segments, int32_t num_segments, vo
  *   b_parts: row sums of d_proj before its rounding -> float32 partials [parts][4H] (may be NULL)
  * with parts = oops_trimul_factor_grad_parts (0: not served; use oops_trimul_factors_backward and GEMMs).
  * Replaces the reference's factor backward with its projection GEMMs
- * (triangle_multiplication/triton/generic.py:960-1018). */
+ * (triangle_multiplication/triton/kernel.py:190-364, generic.py:1022-1092). */
 size_t oops_trimul_factor_grad_parts(const oops_trimul_geometry* geo);
 int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normalized, const void* weight,
                              const float* bias, const void* mask, const void* grad_factors, void* grad_xn,
@@ -422,7 +422,7 @@ int oops_trimul_factor_grads(const oops_trimul_geometry* geo, const void* normal
  *   b_parts: column sums of grad_value, then of grad_gate, float32 partials [2][parts][C]
  * with parts = oops_trimul_output_grads_parts (0: not served).  n, n_pad: 0, or the sides of a padded pair
  * (oops_trimul_output_pair_backward).  Replaces the reference's output backward and the GEMMs and column sums
- * behind it (triangle_multiplication/triton/generic.py:820-856). */
+ * behind it (triangle_multiplication/triton/generic.py:820-824, :842-856). */
 size_t oops_trimul_output_grads_parts(const oops_trimul_geometry* geo);
 int oops_trimul_output_grads(const oops_trimul_geometry* geo, int64_t n, int64_t n_pad, const void* normalized,
                              const void* pair_normalized, const void* output_weight, const void* gate_weight,

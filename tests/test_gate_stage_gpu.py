@@ -169,3 +169,31 @@ def test_gate_stage_infinite_inputs(heads, c, o):
     got = oops_amd.gate_attention_output(att, single, wg, wo)
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
     assert got[0, 3].isfinite().all()
+
+
+@pytest.mark.parametrize("c", [256, 384])
+def test_gate_stage_graph_replays(c):
+    operands = _inputs(torch.bfloat16, (2,), c // 32, 150, 32, c, c)
+    grad = torch.randn(2, 150, c, device="cuda").bfloat16()
+
+    def step():
+        return torch.autograd.grad(oops_amd.gate_attention_output(*operands), operands, grad)
+
+    want = [g.clone() for g in step()]
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step()
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(3):
+        for g in got:
+            g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want))
+        step()
+        torch.cuda.synchronize()

@@ -146,3 +146,73 @@ def test_factor_grads_served_range():
     assert parts() == 1
     for change in (dict(dtype=_lib.F32), dict(c=64), dict(c=136), dict(c=100), dict(h=64), dict(h=136), dict(positions=81)):
         assert parts(**change) == 0, change
+
+
+@pytest.mark.parametrize("n,mask_grad", [(32, False), (32, True), (20, False)])
+def test_routes_agree(n, mask_grad, monkeypatch):
+    """The operator's backward through both passes, through the output pass alone (a mask gradient, or positions
+    that are no multiple of 32), and through the separate kernels: every gradient within the roundings of the
+    16-bit intermediates that only the separate kernels write (a few units of the largest value)."""
+
+    import oops_amd
+
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    rand = lambda *s, scale=1.0: (torch.randn(*s, device=DEV, generator=gen) * scale).bfloat16().requires_grad_()  # noqa: E731
+    c = 128
+    names = ("input_norm_weight input_norm_bias left_value_weight left_gate_weight right_value_weight "
+             "right_gate_weight output_norm_weight output_norm_bias output_weight output_gate_weight").split()
+    weights = {k: rand(c) if "norm" in k else rand(c, c, scale=c**-0.5) for k in names}
+    biases = {k: rand(c, scale=0.2) for k in ("left_value_bias left_gate_bias right_value_bias right_gate_bias "
+                                              "output_bias output_gate_bias").split()}
+    pair = rand(n, n, c)
+    mask = torch.rand(n, n, device=DEV, generator=gen).requires_grad_(mask_grad)
+    dy = rand(n, n, c).detach()
+    leaves = [pair, *weights.values(), *biases.values()] + ([mask] if mask_grad else [])
+
+    def grads():
+        out = oops_amd.triangle_multiplication(pair, mask, direction="outgoing", **weights, **biases)
+        return torch.autograd.grad(out, leaves, dy)
+
+    got = grads()
+    lib = _lib.load()
+    for name in ("oops_trimul_factor_grad_parts", "oops_trimul_output_grads_parts"):
+        monkeypatch.setattr(lib, name, lambda geo: 0)
+    for x, y in zip(got, grads()):
+        assert (x.double() - y.double()).abs().max() <= 8 * 2.0**-8 * y.double().abs().max()
+
+
+def test_graph_replays():
+    """Both passes under graph capture: every replay equals the eager gradients."""
+
+    import oops_amd
+
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    rand = lambda *s: (torch.randn(*s, device=DEV, generator=gen) * 0.3).bfloat16().requires_grad_()  # noqa: E731
+    c, n = 128, 48
+    names = ("input_norm_weight input_norm_bias left_value_weight left_gate_weight right_value_weight "
+             "right_gate_weight output_norm_weight output_norm_bias output_weight output_gate_weight").split()
+    weights = {k: rand(c) if "norm" in k else rand(c, c) for k in names}
+    pair, dy = rand(n, n, c), rand(n, n, c).detach()
+    leaves = [pair, *weights.values()]
+
+    def step():
+        return torch.autograd.grad(oops_amd.triangle_multiplication(pair, None, direction="incoming", **weights), leaves, dy)
+
+    want = [g.clone() for g in step()]
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step()
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(3):
+        for g in got:
+            g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want))
+        step()
+        torch.cuda.synchronize()
