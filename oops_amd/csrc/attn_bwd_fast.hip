@@ -25,8 +25,8 @@ namespace oops {
 
 using namespace fast;
 
-// XW: the bias weight in two terms (see exact_weight).
-template <typename T, int DP, bool HAS_BIAS, int R, bool XW = false>
+// XB: the bias is added in float32 (see ExactBias).
+template <typename T, int DP, bool HAS_BIAS, int R, bool XB = false>
 __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -101,10 +101,10 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
       vf[r][s] = __builtin_bit_cast(Frag, buffer_load16(v_rsrc, ok ? (uint32_t)((key * (int)S.v_si + col) * 2) : kOut));
     }
   }
+  const ExactBias<T> xb(a.scale);
+  constexpr bool LAST = XB && ExactBias<T>::kLast;
   Frag ident[2];
-  identity_frags<T>(ident, 1.0f / a.scale, lane);
-  Frag ident_low[2];
-  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
+  identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
 
   // ---- per-thread staging offsets (bytes); the step adds q0 * stride via soffset
   __amdgpu_buffer_rsrc_t q_rsrc[R], do_rsrc[R], l_rsrc[R], d_rsrc[R];
@@ -171,8 +171,8 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
       }
     }
   };
-  // -LSE is the S accumulator's input, in units of the unscaled scores
-  const float inv_c1 = 1.0f / (a.scale * kLog2e);
+  // -LSE is the S accumulator's input, in units of the unscaled scores (XB: added to x)
+  const float inv_c1 = XB ? 1.0f : 1.0f / (a.scale * kLog2e);
   auto store_stage = [&](int buf, const Stage& st) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
     }
   };
 
-  const float c1 = a.scale * kLog2e;
+  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
   f32x16 dk[R][NDT], dv[R][NDT];
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -212,25 +212,29 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
 #pragma unroll
       for (int qr = 0; qr < 2; ++qr) {
         // S - LSE / c1: the accumulator starts from -LSE / c1
-        f32x16 sacc = *reinterpret_cast<const f32x16*>(&nlse_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16]);
-        if constexpr (HAS_BIAS) {
+        // (XB: from zero, the LSE comes off x)
+        const float* nlse = &nlse_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16];
+        f32x16 sacc = XB ? f32x16{} : *reinterpret_cast<const f32x16*>(nlse);
+        auto add_bias = [&] {
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][0]), ident[0], sacc);
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][1]), ident[1], sacc);
-          if constexpr (XW) {
-            sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][0]), ident_low[0], sacc);
-            sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][1]), ident_low[1], sacc);
-          }
-        }
+        };
+        if constexpr (HAS_BIAS && !LAST) add_bias();
+        if constexpr (XB && !LAST) xb.scale_first(sacc);
         f32x16 pacc = *reinterpret_cast<const f32x16*>(&ndlt_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16]);
 #pragma unroll
         for (int s = 0; s < NQF; ++s) {
           sacc = E::mma(lds_frag<T>(qt + swz_off<DP>(32 * qr + lq, s * 16 + g2 * 8)), kf[r][s], sacc);
           pacc = E::mma(lds_frag<T>(dt + swz_off<DP>(32 * qr + lq, s * 16 + g2 * 8)), vf[r][s], pacc);
         }
+        if constexpr (LAST) {
+          xb.scale_first(sacc);
+          add_bias();
+        }
         float p[16], ds[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          p[j] = __builtin_amdgcn_exp2f(sacc[j] * c1);
+          p[j] = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, nlse[j]) : sacc[j] * c1);
           if (wave_masked[r]) p[j] = kvalid[r] ? p[j] : 0.0f;
           ds[j] = p[j] * pacc[j];
         }
@@ -327,18 +331,19 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
 // FULL_DBIAS: some sample has a per-group bias whose dBias = dS is written
 // here.  Both only add code that costs registers when compiled in.  FOLD
 // (bf16, bias, at most kFoldTiles key tiles): the key masks are folded into
-// the bias fragments (fold_bias) instead of selected per score.  XW: the bias
-// weight in two terms (see exact_weight).
+// the bias fragments (fold_bias) instead of selected per score.  XB: the bias
+// is added in float32 (see ExactBias).
 // The lean instances (D <= 32, no per-score mask code, no full dBias) start
 // dP from a register tile of -delta instead of zero (one VALU add less per
 // score) and are built for four waves per SIMD, which the extra 16 registers
 // still fit.
 template <int DP, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD>
 constexpr bool kLeanDq = DP == 32 && (!MASKED_TILES || FOLD) && !FULL_DBIAS;
-template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD, bool XW = false>
+template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FULL_DBIAS, bool FOLD, bool XB = false>
 __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ? 4 : OOPS_DQ_OCC)) void attn_dq_fast_kernel(
     BwdArgsT<T, T> a) {
   constexpr bool LEAN = kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD>;
+  constexpr bool LAST = XB && ExactBias<T>::kLast;
   static_assert(!FOLD || (MASKED_TILES && HAS_BIAS && sizeof(T) == 2), "fold: masked bf16 tiles with a bias");
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -502,16 +507,15 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     }
     ndelta = -dl;
   }
-  // the pack of the fused dK/dV + dBias kernel: per (g, h) row, -LSE / c of
+  const ExactBias<T> xb(a.scale);
+  // the pack of the fused dK/dV + dBias kernel: per (g, h) row, -LSE / c (XB: -LSE) of
   // the Lq queries (lanes 0..31), then -delta (lanes 32..63)
   if (a.ld_pack != nullptr && qv) {
     float* const pk_row = a.ld_pack + 2 * (lidx - q_lane);
-    pk_row[g2 * Lq + q_lane] = g2 ? ndelta : neg_lse * (1.0f / (a.scale * kLog2e));
+    pk_row[g2 * Lq + q_lane] = g2 ? ndelta : neg_lse * (XB ? 1.0f : 1.0f / (a.scale * kLog2e));
   }
   Frag ident[2];
-  identity_frags<T>(ident, 1.0f / a.scale, lane);
-  Frag ident_low[2];
-  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
+  identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
 
   const T* kbase = a.k + S.k_off + g * S.k_sg + h * S.k_sh;
   const T* vbase = a.v + S.v_off + g * S.v_sg + h * S.v_sh;
@@ -630,7 +634,7 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     return t;
   };
 
-  const float c1 = a.scale * kLog2e;
+  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
   f32x16 nd_tile;  // LEAN: the dP accumulator's starting value
 #pragma unroll
   for (int j = 0; j < 16; ++j) nd_tile[j] = LEAN ? ndelta : 0.0f;
@@ -648,29 +652,29 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     const uint4* fm = reinterpret_cast<const uint4*>(&fold_lds[FOLD ? (t * 2 + g2) * 16 : 0]);
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      f32x16 sacc;
-      if constexpr (HAS_BIAS) {
+      f32x16 sacc = f32x16{};
+      auto add_bias = [&] {
         const uint4 b0 = FOLD ? fold_bias(bf[t2][0], fm[t2 * 2]) : bf[t2][0];
         const uint4 b1 = FOLD ? fold_bias(bf[t2][1], fm[t2 * 2 + 1]) : bf[t2][1];
-        sacc = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
+        sacc = E::mma(ident[0], __builtin_bit_cast(Frag, b0), sacc);
         sacc = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc);
-        if constexpr (XW) {
-          sacc = E::mma(ident_low[0], __builtin_bit_cast(Frag, b0), sacc);
-          sacc = E::mma(ident_low[1], __builtin_bit_cast(Frag, b1), sacc);
-        }
-      } else {
-        sacc = f32x16{};
-      }
+      };
+      if constexpr (HAS_BIAS && !LAST) add_bias();
+      if constexpr (XB && !LAST) xb.scale_first(sacc);
       f32x16 pacc = LEAN ? nd_tile : f32x16{};
 #pragma unroll
       for (int s = 0; s < NQF; ++s) {
         sacc = E::mma(lds_frag<T>(kt + (32 * t2 + lq) * LD + s * 16 + g2 * 8), qf[s], sacc);
         pacc = E::mma(lds_frag<T>(vt + (32 * t2 + lq) * LD + s * 16 + g2 * 8), df[s], pacc);
       }
+      if constexpr (LAST) {
+        xb.scale_first(sacc);
+        add_bias();
+      }
       float ds[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[j], c1, neg_lse));
+        float p = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, neg_lse) : __builtin_fmaf(sacc[j], c1, neg_lse));
         if constexpr (MASKED) {
           const int kk = 32 * t2 + ((j >> 2) << 3) + (j & 3);
           p = ((lb >> kk) & 1) ? p : 0.0f;
@@ -759,8 +763,10 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
 // dS block accumulates in registers (no atomics).  Partial sums per part are
 // added by attn_dbias_reduce_kernel.
 // Reference: _backward_shared_bias (oops/attention/triangle/triton/kernel.py:721-873).
-// MASKED_TILES: as in attn_dq_fast_kernel.
-template <typename T, int DP, bool MASKED_TILES>
+// MASKED_TILES, XB: as in attn_dq_fast_kernel; with XB the logits are the
+// generic kernels' x = scale log2 e Q.K + log2 e b, the second term being what
+// the block keeps.
+template <typename T, int DP, bool MASKED_TILES, bool XB = false>
 __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(BwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -820,12 +826,11 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
   const bool qv = q_lane < Lq;
   const float c1 = a.scale * kLog2e;
 
-  // bias contribution of this (query, key) block, shared by every group
+  // bias contribution of this (query, key) block, shared by every group (XB: log2 e b)
   f32x16 bacc[2];
   {
-    Frag ident[2], ident_low[2];
-    identity_frags<T>(ident, 1.0f / a.scale, lane);
-    identity_low_frags<T>(ident_low, a.exact_weight ? 1.0f / a.scale : 1.0f, lane);  // (zeros for weight 1)
+    Frag ident[2];
+    identity_frags<T>(ident, XB ? ExactBias<T>::kBlockWeight : 1.0f / a.scale, lane);
     // (from the fragment-major copy, or from the aligned bias rows when there is none)
     const T* brow = a.bias + S.b_off + h * S.b_sh + (int64_t)q_lane * S.b_si;
     const int qt = qb * 4 + wave;
@@ -846,7 +851,10 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
           u = finite16<T>(u);
         }
         bacc[t2] = E::mma(ident[c], __builtin_bit_cast(Frag, u), bacc[t2]);
-        if (a.exact_weight) bacc[t2] = E::mma(ident_low[c], __builtin_bit_cast(Frag, u), bacc[t2]);
+      }
+      if constexpr (XB) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) bacc[t2][j] = ExactBias<T>::log2_bias(bacc[t2][j]);
       }
     }
   }
@@ -998,7 +1006,7 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
       constexpr bool MASKED = decltype(masked)::value;
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
-        f32x16 sacc = bacc[t2];
+        f32x16 sacc = XB ? f32x16{} : bacc[t2];
         f32x16 pacc = nd;
 #pragma unroll
         for (int s = 0; s < NQF; ++s) {
@@ -1007,7 +1015,8 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[j], c1, nlse));
+          float p = __builtin_amdgcn_exp2f(XB ? __builtin_fmaf(sacc[j], c1, bacc[t2][j]) + nlse
+                                              : __builtin_fmaf(sacc[j], c1, nlse));
           if constexpr (MASKED) {
             const int kk = 32 * t2 + ((j >> 2) << 3) + (j & 3);
             p = ((lb >> kk) & 1) ? p : 0.0f;
@@ -1056,12 +1065,15 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
   template __global__ void attn_dkv_fast_kernel<T, DP, false, 1>(BwdArgsT<T, T>); \
   OOPS_DQ_FAST_INST(T, DP, true)                                                 \
   OOPS_DQ_FAST_INST(T, DP, false)                                                \
+  template __global__ void attn_dbias_fast_kernel<T, DP, true, true>(BwdArgsT<T, T>); \
   template __global__ void attn_dbias_fast_kernel<T, DP, false>(BwdArgsT<T, T>);     \
   template __global__ void attn_dbias_fast_kernel<T, DP, true>(BwdArgsT<T, T>);
 OOPS_BWD_FAST_INST(__bf16, 32)
 OOPS_BWD_FAST_INST(__bf16, 64)
 template __global__ void attn_dq_fast_kernel<__bf16, 32, true, true, false, true>(BwdArgsT<__bf16, __bf16>);
 template __global__ void attn_dq_fast_kernel<__bf16, 64, true, true, false, true>(BwdArgsT<__bf16, __bf16>);
+template __global__ void attn_dq_fast_kernel<__bf16, 32, true, true, false, true, true>(BwdArgsT<__bf16, __bf16>);
+template __global__ void attn_dq_fast_kernel<__bf16, 64, true, true, false, true, true>(BwdArgsT<__bf16, __bf16>);
 OOPS_BWD_FAST_INST(_Float16, 32)
 OOPS_BWD_FAST_INST(_Float16, 64)
 
@@ -1090,7 +1102,7 @@ hipError_t launch_dkv_fast(const oops_attn_geometry& geo, const Plan& plan, cons
     fill_bwd_args(a, geo, plan, L);
     // OOPS_DKV_ROWS=2: two rows per workgroup share each bias fragment (row-shared
     // biases only); it costs a wave of occupancy and measured slower at the headline shape
-    const bool pair = !rest && !a.exact_weight && OOPS_DKV_ROWS == 2 && a.bias != nullptr && !plan.any_full && plan.dkv_tiles_r2 > 0;
+    const bool pair = !rest && !exact_bias(geo) && OOPS_DKV_ROWS == 2 && a.bias != nullptr && !plan.any_full && plan.dkv_tiles_r2 > 0;
     a.uniform_tiles = pair ? plan.dkv_uniform_r2 : plan.dkv_uniform;
     a.total_tiles = pair ? plan.dkv_tiles_r2 : plan.dkv_tiles;
     if (rest) {
@@ -1100,7 +1112,7 @@ hipError_t launch_dkv_fast(const oops_attn_geometry& geo, const Plan& plan, cons
     }
     if (a.total_tiles == 0) return hipSuccess;
     const dim3 grid((unsigned)xcd_grid(a.total_tiles, xcd_chunk(a.uniform_tiles)));
-    if (a.exact_weight)
+    if (exact_bias(geo))
       hipLaunchKernelGGL((attn_dkv_fast_kernel<T, DP, true, 1, true>), grid, dim3(256), 0, stream, a);
     else if (pair)
       hipLaunchKernelGGL((attn_dkv_fast_kernel<T, DP, true, 2>), grid, dim3(256), 0, stream, a);
@@ -1126,27 +1138,31 @@ hipError_t launch_dq_fast(const oops_attn_geometry& geo, const Plan& plan, const
     a.fused_max_lq = L.qc != nullptr && plan.fused_split ? kFusedMaxLen : 0;
     const dim3 grid((unsigned)xcd_grid(plan.fwd_tiles, xcd_chunk(plan.fwd_uniform)));
     const bool full = a.dbias != nullptr && plan.any_full;
-    auto go = [&](auto has_bias, auto masked, auto full_db, auto fold) {
+    auto go = [&](auto has_bias, auto masked, auto full_db, auto fold, auto exact) {
       hipLaunchKernelGGL((attn_dq_fast_kernel<T, DP, decltype(has_bias)::value, decltype(masked)::value,
-                                              decltype(full_db)::value, decltype(fold)::value>),
+                                              decltype(full_db)::value, decltype(fold)::value, decltype(exact)::value>),
                          grid, dim3(256), 0, stream, a);
     };
+    using Yes = std::true_type;
+    using No = std::false_type;
     auto by_full = [&](auto has_bias, auto masked) {
-      if constexpr (decltype(has_bias)::value && decltype(masked)::value && std::is_same_v<T, __bf16>) {
-        if (!full && fold_masks_ok(plan)) return go(has_bias, masked, std::false_type{}, std::true_type{});
+      if constexpr (decltype(has_bias)::value && decltype(masked)::value) {
+        constexpr bool kFold = std::is_same_v<T, __bf16>;
+        const bool fold = kFold && !full && fold_masks_ok(plan);
+        // (an exact bias comes with shared biases only: no full dBias)
+        if (exact_bias(geo))
+          return fold ? go(Yes{}, Yes{}, No{}, std::bool_constant<kFold>{}, Yes{}) : go(Yes{}, Yes{}, No{}, No{}, Yes{});
+        if (fold) return go(has_bias, masked, No{}, std::bool_constant<kFold>{}, No{});
       }
-      if (full) go(has_bias, masked, std::true_type{}, std::false_type{});
-      else go(has_bias, masked, std::false_type{}, std::false_type{});
+      if (full) go(has_bias, masked, Yes{}, No{}, No{});
+      else go(has_bias, masked, No{}, No{}, No{});
     };
     auto by_mask = [&](auto has_bias) {
-      if (plan.masked_tiles) by_full(has_bias, std::true_type{});
-      else by_full(has_bias, std::false_type{});
+      if (plan.masked_tiles || (decltype(has_bias)::value && exact_bias(geo))) by_full(has_bias, Yes{});
+      else by_full(has_bias, No{});
     };
-    // (an exact weight comes with shared biases only: no full dBias)
-    if (a.exact_weight)
-      hipLaunchKernelGGL((attn_dq_fast_kernel<T, DP, true, true, false, false, true>), grid, dim3(256), 0, stream, a);
-    else if (a.bias != nullptr) by_mask(std::true_type{});
-    else by_mask(std::false_type{});
+    if (a.bias != nullptr) by_mask(Yes{});
+    else by_mask(No{});
     return hipGetLastError();
   });
 }
@@ -1165,7 +1181,9 @@ hipError_t launch_dbias_fast(const oops_attn_geometry& geo, const Plan& plan, co
     if (rest) a.fused_max_lq = kFusedMaxLen;
     if (a.total_tiles == 0) return hipSuccess;
     const dim3 grid((unsigned)xcd_grid(a.total_tiles, xcd_chunk(a.uniform_tiles)));
-    if (plan.masked_tiles)
+    if (exact_bias(geo))
+      hipLaunchKernelGGL((attn_dbias_fast_kernel<T, DP, true, true>), grid, dim3(256), 0, stream, a);
+    else if (plan.masked_tiles)
       hipLaunchKernelGGL((attn_dbias_fast_kernel<T, DP, true>), grid, dim3(256), 0, stream, a);
     else
       hipLaunchKernelGGL((attn_dbias_fast_kernel<T, DP, false>), grid, dim3(256), 0, stream, a);

@@ -15,7 +15,8 @@
 // with RW = 8 all eight waves work on one row, wave w taking the tiles w,
 // w + 8, w + 16, w + 24 (Lq <= 1024).  Every lane owns one key (the MFMA
 // column).  Per step a wave computes, for one query tile,
-//   S  = Q K^T (+ bias by an identity MFMA, - LSE as the accumulator input),
+//   S  = Q K^T (+ bias by an identity MFMA, - LSE as the accumulator input;
+//        bias rows that are not 16-byte aligned: in float32, see ExactBias),
 //   dP = dO V^T - delta,   P = exp2(S * scale * log2 e),   dS = P * dP,
 //   dV^T += dO^T P,  dK^T += Q^T dS,  region[step] += dS.
 // The dBias region of a wave (32 keys x its query tiles) stays in registers
@@ -114,7 +115,8 @@ struct RingStage {
   float ld[64];  // -LSE / c of the 32 queries, then -delta
 };
 
-template <typename T, bool MASKED, int NS, int RW>
+// XB: the bias is added in float32 (see ExactBias).
+template <typename T, bool MASKED, int NS, int RW, bool XB>
 __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -188,7 +190,9 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
   const int g_end = __builtin_amdgcn_readfirstlane((int)(G * (part + 1) / P));
   const int D = a.head_size;
   const int nqt = (Lq + 31) >> 5;  // <= NS * 4 (the launch picks NS for the longest sample)
-  const float c1 = a.scale * kLog2e;
+  const ExactBias<T> xb(a.scale);
+  constexpr bool LAST = XB && ExactBias<T>::kLast;
+  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
   const int key = kb * 32 + lq;  // this lane's key
   const bool has_mask = MASKED && a.mask != nullptr && S.m_off >= 0;
 
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
   const int64_t db_si = S.db_si;
 
   Frag ident[2];
-  identity_frags<T>(ident, 1.0f / a.scale, lane);
+  identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
   const TrLane trl = tr_lane<32>(lane, 0);
 
   // The resources of group g's (g, h) blocks of the compact Q and dO copies
@@ -487,17 +491,24 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
       if (i * kRowWaves + wq < nqt && g_live) {
       const T* qt_ = reinterpret_cast<const T*>(cur.q);
       const T* dt_ = reinterpret_cast<const T*>(cur.d);
-      f32x16 sacc = *reinterpret_cast<const f32x16*>(&cur.ld[g2 * 16]);
-      {
+      // (XB: from zero, the LSE comes off x)
+      f32x16 sacc = XB ? f32x16{} : *reinterpret_cast<const f32x16*>(&cur.ld[g2 * 16]);
+      auto add_bias = [&] {
         const T* bq = bias_lds + (i * kRowWaves + wq) * 2 * 64 * 8 + lane * 8;
         sacc = E::mma(lds_frag<T>(bq), ident[0], sacc);
         sacc = E::mma(lds_frag<T>(bq + 64 * 8), ident[1], sacc);
-      }
+      };
+      if constexpr (!LAST) add_bias();
+      if constexpr (XB && !LAST) xb.scale_first(sacc);
       f32x16 pacc = *reinterpret_cast<const f32x16*>(&cur.ld[32 + g2 * 16]);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         sacc = E::mma(lds_frag<T>(qt_ + swz_off<32>(lq, s * 16 + g2 * 8)), kf[s], sacc);
         pacc = E::mma(lds_frag<T>(dt_ + swz_off<32>(lq, s * 16 + g2 * 8)), vf[s], pacc);
+      }
+      if constexpr (LAST) {
+        xb.scale_first(sacc);
+        add_bias();
       }
       // two halves of 8 scores: each half's P and dS feed their MFMAs at once
 #pragma unroll
@@ -506,7 +517,7 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int j = 8 * m + e;
-          p[e] = __builtin_amdgcn_exp2f(sacc[j] * c1);
+          p[e] = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, cur.ld[g2 * 16 + j]) : sacc[j] * c1);
           if (MASKED && wave_masked) p[e] = kvalid ? p[e] : 0.0f;
           ds[e] = p[e] * pacc[j];
           region[i][j] += ds[e];
@@ -584,8 +595,7 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
 }  // namespace
 
 bool dkvb_fused_ok(const oops_attn_geometry& geo, const Plan& plan) {
-  // (its registers and LDS have no room for the second term of an exact weight)
-  return geo.force_generic == 0 && !exact_weight(geo) && fast_path_ok(geo, plan) && plan.dp == kCompactRow && plan.all_shared &&
+  return geo.force_generic == 0 && fast_path_ok(geo, plan) && plan.dp == kCompactRow && plan.all_shared &&
          plan.bias_frag && plan.fused_max_len_q <= kFusedMaxLen && (plan.fused_tiles > 0 || plan.fused_long_tiles > 0);
 }
 
@@ -601,9 +611,12 @@ hipError_t launch_dkvb_fused(const oops_attn_geometry& geo, const Plan& plan, co
       a.uniform_tiles = uniform;
       a.total_tiles = tiles;
       const dim3 grid((unsigned)xcd_grid(tiles, xcd_chunk(uniform)));
-      hipLaunchKernelGGL(
-          (attn_dkvb_fast_kernel<T, decltype(masked)::value, decltype(nsc)::value, decltype(rwc)::value>), grid,
-          dim3(512), 0, stream, a);
+      auto launch = [&](auto exact) {
+        hipLaunchKernelGGL((attn_dkvb_fast_kernel<T, decltype(masked)::value, decltype(nsc)::value, decltype(rwc)::value,
+                                                  decltype(exact)::value>),
+                           grid, dim3(512), 0, stream, a);
+      };
+      exact_bias(geo) ? launch(std::true_type{}) : launch(std::false_type{});
     };
     using RW2 = std::integral_constant<int, 2>;
     using RW4 = std::integral_constant<int, 4>;

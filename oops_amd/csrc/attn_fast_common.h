@@ -99,13 +99,6 @@ __device__ __forceinline__ void identity_frags(typename Elem<T>::Frag (&id)[2], 
   }
 }
 
-// The identity fragments of the part of weight w that its rounding to T drops
-// (w - T(w), itself rounded to T): with both, the weight has twice T's bits.
-template <typename T>
-__device__ __forceinline__ void identity_low_frags(typename Elem<T>::Frag (&id)[2], float w, int lane) {
-  identity_frags<T>(id, w - Elem<T>::to_f((T)w), lane);
-}
-
 // The identity MFMA that adds the bias multiplies every bias element of a
 // 16-key chunk by the zeros of the other keys' columns, so a non-finite bias
 // element (an additive -inf mask) would make the whole chunk NaN.  Bias
@@ -127,28 +120,71 @@ __device__ __forceinline__ uint4 finite16(uint4 u) {
   return make_uint4(finite2<T>(u.x), finite2<T>(u.y), finite2<T>(u.z), finite2<T>(u.w));
 }
 
-// The same for biases that would otherwise take the generic kernels, which
-// add the bias in float32 arithmetic: a row whose kept keys all have a -inf
-// bias is a masked row (output 0), and a NaN or +inf bias at a kept key makes
-// its row NaN.  NaN reads as +max here.  In bfloat16 +-max times a weight of
-// at least 1.0625 overflows to +-inf, which gives both.  A float16 maximum
-// stays finite, so finite float16 elements are clamped to +-60000 (a logit
-// difference of 5504 at least remains: the same softmax) and the forward
-// takes a row maximum beyond +-62750 as a marked element's.
-constexpr float kEdgeLogit = 62750.0f * kLog2e;
+// A bias that the kernels add as the generic ones do (ExactBias): its
+// non-finite elements become marks.  bfloat16: +-max, which finite elements
+// may hold as well, but times log2 e those are infinite in the generic kernels
+// too.  float16: +-65504, the finite elements halved (exact but for
+// subnormals, whose last bit then weighs 2^-25, half of float32's rounding of
+// a logit of 1).  NaN is marked as +inf: either at a kept key makes its row
+// NaN.
 template <typename T>
-__device__ __forceinline__ uint32_t edge1(uint32_t b) {
+__device__ __forceinline__ uint32_t marked1(uint32_t b) {
   constexpr bool kBf = std::is_same_v<T, __bf16>;
   constexpr uint32_t kExp = kBf ? 0x7F80u : 0x7C00u, kMax = kBf ? 0x7F7Fu : 0x7BFFu;
-  const uint32_t neg = b & 0x8000u, mag = b & 0x7FFFu;
-  if (mag >= kExp) return mag == kExp ? neg | kMax : kMax;
-  return neg | (!kBf && mag > 0x7B53u ? 0x7B53u : mag);  // (0x7B53: 60000)
+  const uint32_t mag = b & 0x7FFFu;
+  if (mag >= kExp) return mag == kExp ? (b & 0x8000u) | kMax : kMax;
+  if constexpr (kBf) return b;
+  else return __builtin_bit_cast(uint16_t, (T)((float)__builtin_bit_cast(T, (uint16_t)b) * 0.5f));
 }
 template <typename T>
-__device__ __forceinline__ uint4 edge16(uint4 u) {
-  auto two = [](uint32_t d) { return edge1<T>(d & 0xFFFFu) | (edge1<T>(d >> 16) << 16); };
+__device__ __forceinline__ uint4 marked16(uint4 u) {
+  auto two = [](uint32_t d) { return marked1<T>(d & 0xFFFFu) | (marked1<T>(d >> 16) << 16); };
   return make_uint4(two(u.x), two(u.y), two(u.z), two(u.w));
 }
+
+// The float32 bias of the routes that replace the generic kernels (bias rows
+// that are not 16-byte aligned).  Those compute x = scale log2 e Q.K +
+// log2 e b in float32; a weight 1/scale rounded to 16 bits would change b by
+// up to 2^-9 of itself.  So the identity MFMA's weight is exact here, and the
+// vector unit scales one of the two terms by a float32 factor (one
+// multiplication per score, two in float16).  b is the element, or the mark of
+// one that is not finite (marked1): a mark has to make the logit infinite, a
+// finite element only where it does in the generic kernels.
+//   bfloat16: kWeight b + (kWeight scale) Q.K, Q.K first.  kWeight b overflows
+//     for exactly the elements whose log2 e b does, the marks among them
+//     (b / scale would for smaller ones).
+//   float16: b / scale + Q.K, b first: the MFMA's 2 (b / 2) is at most 65504, a
+//     mark's 131008; of these only the mark is infinite times 2^112.
+// x is rounded before the maximum or the LSE is taken off it, as in the
+// generic kernels: a fused multiply-add would leave the product's rounding,
+// which is more than exp2 can take where every logit of a row is large (a row
+// of -1e9, or of half the lowest bfloat16).
+template <typename T>
+struct ExactBias {
+  static constexpr bool kBf = std::is_same_v<T, __bf16>;
+  static constexpr bool kLast = kBf;  // the bias is added after Q.K
+  static constexpr float kWeight = kBf ? 1.4453125f : 2.0f;
+  float scale;
+  __device__ __forceinline__ explicit ExactBias(float s) : scale(s) {}
+  // the first term, before the second is added to it
+  __device__ __forceinline__ void scale_first(f32x16& s) const {
+    const float r = kBf ? kWeight * scale : 0x1p-112f / scale;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s[j] = kBf ? s[j] * r : (s[j] * 0x1p112f) * r;
+  }
+  // log2 units per unit of the sum
+  __device__ __forceinline__ float unit() const { return kBf ? kLog2e / kWeight : scale * kLog2e; }
+  // x (the sum s in log2 units, rounded) + c
+  static __device__ __forceinline__ float log2_less(float s, float unit, float c) {
+#pragma clang fp contract(off)
+    return s * unit + c;
+  }
+  // log2 e b of an identity MFMA with weight kBlockWeight alone (marks: infinite)
+  static constexpr float kBlockWeight = kBf ? 1.0f : 2.0f;
+  static __device__ __forceinline__ float log2_bias(float b) {
+    return kBf ? b * kLog2e : (b * 0x1p112f) * (kLog2e * 0x1p-112f);
+  }
+};
 
 // Key masks folded into the bias operand of the identity MFMA (bf16, row-
 // shared key masks, at most kFoldTiles 64-key tiles): a masked key's bias

@@ -309,7 +309,6 @@ hipError_t launch_forward(const oops_attn_geometry& geo, const Plan& plan, const
     a.vec_ok = geo.vec_ok != 0;
     a.bias_vec = geo.vec_ok == 1;
     a.lazy = 0.0f;
-    a.edge_bias = 0;
     a.scale = geo.scale;
     if constexpr (std::is_same_v<T, float>) {
       if (plan.fwd_tiles > 0 && attn_f32_ok(geo, plan)) {

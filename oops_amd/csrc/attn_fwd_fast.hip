@@ -32,7 +32,8 @@
 // reference's _attend (oops/attention/triangle/triton/kernel.py:151-262):
 // masked keys read as -inf logits with zero K/V, fully masked rows give
 // O = 0 and LSE = 0.  The bias weight 1/scale is rounded to the input dtype
-// (relative error <= 2^-9 for bf16), below the rounding of P itself.
+// (relative error <= 2^-9 for bf16), below the rounding of P itself, where the
+// bias rows are 16-byte aligned; others are added in float32 (ExactBias).
 #include "attn_fast_common.h"
 
 
@@ -47,9 +48,10 @@ constexpr int kRing = 4;  // K/V tile buffers in LDS
 // out-of-range keys; without it the per-score mask code is not compiled
 // (it costs registers even when never executed).  FOLD (bf16, bias, at most
 // kFoldTiles key tiles): the masks are folded into the bias fragments
-// instead of selected per score.  XW: the bias weight in two terms
-// (identity_low_frags; see exact_weight).
-template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FOLD, bool XW = false>
+// instead of selected per score.  XB: the bias is added in float32 and the
+// row sums are those of the float32 probabilities, as in the generic kernel
+// (see ExactBias).
+template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FOLD, bool XB = false>
 __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArgsT<T, T> a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -138,11 +140,11 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
           Frag, qv && col < D ? *reinterpret_cast<const uint4*>(qrow + col) : make_uint4(0, 0, 0, 0));
     }
   }
-  // identity A-fragments carrying the bias weight 1/scale: MFMA c adds bias keys 16c..16c+15
+  // identity A-fragments carrying the bias weight (1/scale; see ExactBias otherwise): MFMA c adds bias keys
+  // 16c..16c+15
+  const ExactBias<T> xb(a.scale);
   Frag ident[2];
-  identity_frags<T>(ident, 1.0f / a.scale, lane);
-  Frag ident_low[2];
-  if constexpr (XW) identity_low_frags<T>(ident_low, 1.0f / a.scale, lane);
+  identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
 
   // ---- fixed per-lane offsets (bytes) of the direct-to-LDS tile loads:
   // wave w fills rows 16w .. 16w+15 of the K and V tiles; lane l writes slot
@@ -241,7 +243,16 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 #pragma unroll
       for (int c = 0; c < 2; ++c) bf[t2][c] = buffer_load16_s(b_rsrc, t < ntiles ? b_off[t2][c] + s : kOut, 0);
   };
-  // S^T of a tile (bias by identity MFMA, then Q K^T) from LDS buffer buf
+  // S^T of a tile (bias by identity MFMA and Q K^T) from LDS buffer buf
+  constexpr bool LAST = XB && ExactBias<T>::kLast;
+  auto qk_tile = [&](auto bc, int t2, const f32x16& from, f32x16& acc) {
+#pragma unroll
+    for (int s = 0; s < NQF; ++s) {
+      const Frag kf = __builtin_bit_cast(
+          Frag, *reinterpret_cast<const uint4*>(kbuf(bc) + swz_off<DP>(32 * t2 + lq, s * 16 + g2 * 8)));
+      acc = E::mma(kf, qf[s], s == 0 ? from : acc);
+    }
+  };
   auto scores = [&](auto bc, int t, const uint4 (&bf)[2][2], f32x16 (&sacc)[2]) {
     const uint4* fm = reinterpret_cast<const uint4*>(&fold_lds[FOLD ? (t * 2 + g2) * 16 : 0]);
 #pragma unroll
@@ -252,21 +263,17 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
         const uint4 r1 = use_bf ? bf[t2][1] : finite16<T>(bf[t2][1]);
         const uint4 b0 = FOLD ? fold_bias(r0, fm[t2 * 2]) : r0;
         const uint4 b1 = FOLD ? fold_bias(r1, fm[t2 * 2 + 1]) : r1;
-        sacc[t2] = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
-        sacc[t2] = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
-        if constexpr (XW) {
-          sacc[t2] = E::mma(ident_low[0], __builtin_bit_cast(Frag, b0), sacc[t2]);
-          sacc[t2] = E::mma(ident_low[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
+        if constexpr (LAST) {
+          qk_tile(bc, t2, f32x16{}, sacc[t2]);
+          xb.scale_first(sacc[t2]);
         }
+        sacc[t2] = E::mma(ident[0], __builtin_bit_cast(Frag, b0), LAST ? sacc[t2] : f32x16{});
+        sacc[t2] = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
+        if constexpr (XB && !LAST) xb.scale_first(sacc[t2]);
       } else {
         sacc[t2] = f32x16{};
       }
-#pragma unroll
-      for (int s = 0; s < NQF; ++s) {
-        const Frag kf = __builtin_bit_cast(
-            Frag, *reinterpret_cast<const uint4*>(kbuf(bc) + swz_off<DP>(32 * t2 + lq, s * 16 + g2 * 8)));
-        sacc[t2] = E::mma(kf, qf[s], sacc[t2]);
-      }
+      if constexpr (!LAST) qk_tile(bc, t2, sacc[t2], sacc[t2]);
     }
   };
 
@@ -281,7 +288,7 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
     return t;
   };
 
-  const float c1 = a.scale * kLog2e;
+  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
   float m_run = kNegInf;  // reference max (log2 units), raised lazily
   float neg_m = 0.0f;     // -m_run (0 while no key has been seen)
   float l_run = 0.0f;     // this lane's partial row sum
@@ -329,6 +336,8 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
     }
     // the row sum: one v_dot2 chain into l_run (the exponentials between its
     // links hide their latency; no chain registers to clear or add up)
+    float psum = 0.0f;  // XB: the tile's sum before the rounding of P
+    auto less_max = [&](float s) { return XB ? xb.log2_less(s, c1, neg_m) : __builtin_fmaf(s, c1, neg_m); };
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
@@ -337,9 +346,12 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
           P2 pr;
-          pr[0] = (T)__builtin_amdgcn_exp2f(__builtin_fmaf(sacc[t2][8 * m + e], c1, neg_m));
-          pr[1] = (T)__builtin_amdgcn_exp2f(__builtin_fmaf(sacc[t2][8 * m + e + 1], c1, neg_m));
-          l_run = Pair<T>::dot(pr, ones, l_run);
+          const float p0 = __builtin_amdgcn_exp2f(less_max(sacc[t2][8 * m + e]));
+          const float p1 = __builtin_amdgcn_exp2f(less_max(sacc[t2][8 * m + e + 1]));
+          pr[0] = (T)p0;
+          pr[1] = (T)p1;
+          if constexpr (XB) psum += p0 + p1;
+          else l_run = Pair<T>::dot(pr, ones, l_run);
           pf[e] = pr[0];
           pf[e + 1] = pr[1];
         }
@@ -349,6 +361,7 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
           oacc[t] = E::mma(vf, pf, oacc[t]);
         }
       }
+    if constexpr (XB) l_run += psum;
   };
 
   // ---- pipeline.  Step i computes tile t0 from ring buffer i % kRing.  It
@@ -402,17 +415,7 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 
   // ---- epilogue
   const float l_tot = sum_halves(l_run);
-  float inv = 1.0f / (l_tot == 0.0f ? 1.0f : l_tot);
-  float lse = l_tot == 0.0f ? 0.0f : (m_run == kNegInf ? 0.0f : m_run) + __log2f(l_tot);
-  if constexpr (HAS_BIAS && std::is_same_v<T, _Float16>) {
-    if (a.edge_bias) {
-      // only -inf biases at the kept keys: a fully masked row; a NaN or +inf one: NaN (see edge16)
-      if (m_run < -kEdgeLogit) lse = inv = 0.0f;
-      uint32_t nan_bits = 0x7FC00000u;
-      asm volatile("" : "+v"(nan_bits));  // (opaque: this file is compiled without NaN semantics)
-      if (m_run > kEdgeLogit) lse = inv = __builtin_bit_cast(float, nan_bits);
-    }
-  }
+  const float inv = 1.0f / (l_tot == 0.0f ? 1.0f : l_tot);
   if (qv) {
     const int64_t o_row = S.o_off + g * S.o_sg + h * S.o_sh + (int64_t)q_lane * S.o_si;
     T* orow = a.out + o_row;
@@ -428,7 +431,10 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
       store_tile<T>(orow, t * 32, D, g2, o, 1.0f);
       if (lrow) store_tile<T>(lrow, t * 32, D, g2, r, 1.0f);
     }
-    if (g2 == 0 && a.lse != nullptr) a.lse[S.l_off + ((int64_t)g * H + h) * Lq + q_lane] = lse;
+    if (g2 == 0 && a.lse != nullptr) {
+      const float m_use = m_run == kNegInf ? 0.0f : m_run;
+      a.lse[S.l_off + ((int64_t)g * H + h) * Lq + q_lane] = l_tot == 0.0f ? 0.0f : m_use + __log2f(l_tot);
+    }
   }
 }
 
@@ -441,6 +447,8 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 OOPS_FWD_FAST_INST(__bf16, 32)
 template __global__ void attn_fwd_fast_kernel<__bf16, 32, true, true, true>(FwdArgsT<__bf16, __bf16>);
 template __global__ void attn_fwd_fast_kernel<__bf16, 64, true, true, true>(FwdArgsT<__bf16, __bf16>);
+template __global__ void attn_fwd_fast_kernel<__bf16, 32, true, true, true, true>(FwdArgsT<__bf16, __bf16>);
+template __global__ void attn_fwd_fast_kernel<__bf16, 64, true, true, true, true>(FwdArgsT<__bf16, __bf16>);
 OOPS_FWD_FAST_INST(__bf16, 64)
 OOPS_FWD_FAST_INST(_Float16, 32)
 OOPS_FWD_FAST_INST(_Float16, 64)
@@ -449,33 +457,17 @@ bool fold_masks_ok(const Plan& plan) { return plan.max_len_k <= 64 * kFoldTiles;
 
 // Bias rows that are not 16-byte aligned (an odd number of keys) reach the
 // fast kernels only through the fragment-major copy, so every sample's bias
-// must be shared by its rows.  The bias weight 1/scale must be large enough
-// that the largest bfloat16 times it is infinite (see edge16).  Measured at
-// 331 residues, 4 heads of 32, masked, bf16, forward and backward: generic
-// kernels 2304 us, this route 325 us; at 127 MSA rows x 277 tokens, 8 heads,
-// float16, forward: 237 and 54 us.
+// must be shared by its rows.  The generic kernels served these calls before,
+// and what they compute stays: the kernels add such a bias in float32 and
+// treat its non-finite elements the same way (ExactBias), which holds for
+// scales of this range.  Measured at 331 residues, 4 heads of 32, masked, bf16,
+// forward and backward: generic kernels 2363 us, this route 352 us (329 us with the bias weight and the row sum in 16 bits); at 127 MSA
+// rows x 277 tokens, 8 heads, float16, forward: 237 and 56 us (54).
 static bool unaligned_bias_ok(const oops_attn_geometry& geo, const Plan& plan) {
-  const float w = 1.0f / geo.scale;
-  return plan.all_shared && geo.scale > 0.0f && w >= 1.0625f && w <= 16384.0f;
+  return plan.all_shared && geo.scale >= 0x1p-14f && geo.scale <= 1.0f;
 }
 
-// The generic kernels, which add the bias in float32, served unaligned bias
-// rows before.  So that no such call loses precision by the faster route, the
-// bias weight keeps at least four bits more than the inputs have (relative
-// error up to 2^-12 in bfloat16, 2^-15 in float16): where one rounding to the
-// input dtype does not (head sizes 24 and 48 in bfloat16, 32 in float16),
-// two more identity MFMAs per score tile add the rounding's rest.
-bool exact_weight(const oops_attn_geometry& geo) {
-  if (!bias_unaligned(geo)) return false;
-  const int drop = geo.dtype == OOPS_F16 ? 13 : 16;  // float32 mantissa bits that T does not have
-  const float w = 1.0f / geo.scale;
-  uint32_t u;
-  __builtin_memcpy(&u, &w, 4);
-  u = (u + (1u << (drop - 1)) - 1u + ((u >> drop) & 1u)) & ~((1u << drop) - 1u);  // nearest even
-  float r;
-  __builtin_memcpy(&r, &u, 4);
-  return !(__builtin_fabsf(r - w) <= w * (geo.dtype == OOPS_F16 ? 0x1p-15f : 0x1p-12f));
-}
+bool exact_bias(const oops_attn_geometry& geo) { return bias_unaligned(geo); }
 
 bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan) {
   if (geo.force_generic == 1) return false;
@@ -498,8 +490,7 @@ bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan) {
 // reads a fragment with one contiguous 1 KB load instead of 32 rows of
 // 32 bytes (which the L1 serves one row at a time).  One thread per entry.
 // ALIGNED: the bias rows start 16-byte aligned; else their elements are read
-// one by one and non-finite ones are marked so that the kernels treat them as
-// the generic ones do (edge16).
+// one by one, non-finite ones marked (see ExactBias).
 template <typename T, bool ALIGNED>
 __global__ __launch_bounds__(256) void attn_bias_frag_kernel(const T* __restrict__ bias, T* __restrict__ bf,
                                                              const int64_t* table, int num_samples, int H,
@@ -531,8 +522,8 @@ __global__ __launch_bounds__(256) void attn_bias_frag_kernel(const T* __restrict
       for (int j = 0; j < 8; ++j) e[j] = k + j < S.Lk ? row[k + j] : (T)0.0f;
       v = __builtin_bit_cast(uint4, e);
     }
-    // (non-finite elements read as +-max: see finite2)
-    v = ALIGNED ? fast::finite16<T>(v) : fast::edge16<T>(v);
+    // (non-finite elements of aligned rows read as +-max: see finite2)
+    v = ALIGNED ? fast::finite16<T>(v) : fast::marked16<T>(v);
   }
   const int64_t dst = (int64_t)s * sample_stride + ((((int64_t)h * nqt + qt) * nkt + kt) * 2 + c) * 512 + lane * 8;
   *reinterpret_cast<uint4*>(bf + dst) = v;
@@ -582,8 +573,7 @@ bool launch_forward_fast(const oops_attn_geometry& geo, const Plan& plan, const 
     a.bias_vec = geo.vec_ok == 1;
     a.scale = geo.scale;
     // (the generic kernels keep the exact maximum: so does the route that replaces them)
-    a.lazy = bias_unaligned(geo) ? 0.0f : kLazyRescale;
-    a.edge_bias = bias_unaligned(geo);
+    a.lazy = exact_bias(geo) ? 0.0f : kLazyRescale;
     a.total_tiles = plan.fwd_tiles;
     a.head_group = head_group(geo);
     a.bias_frag = static_cast<const T*>(bias_frag);
@@ -591,22 +581,23 @@ bool launch_forward_fast(const oops_attn_geometry& geo, const Plan& plan, const 
     a.bf_nqt = plan.bf_nqt;
     a.bf_nkt = plan.bf_nkt;
     const dim3 grid((unsigned)xcd_grid(plan.fwd_tiles, xcd_chunk(plan.fwd_uniform)));
-    auto go = [&](auto has_bias, auto masked, auto fold) {
+    auto go = [&](auto has_bias, auto masked, auto fold, auto exact) {
       hipLaunchKernelGGL((attn_fwd_fast_kernel<T, DP, decltype(has_bias)::value, decltype(masked)::value,
-                                               decltype(fold)::value>),
+                                               decltype(fold)::value, decltype(exact)::value>),
                          grid, dim3(256), 0, stream, a);
     };
-    if (a.bias != nullptr && exact_weight(geo)) {
-      hipLaunchKernelGGL((attn_fwd_fast_kernel<T, DP, true, true, false, true>), grid, dim3(256), 0, stream, a);
-      *err = hipGetLastError();
-      return;
-    }
+    using Yes = std::true_type;
+    using No = std::false_type;
     auto by_mask = [&](auto has_bias) {
-      if constexpr (decltype(has_bias)::value && std::is_same_v<T, __bf16>) {
-        if (plan.masked_tiles && fold_masks_ok(plan)) return go(has_bias, std::true_type{}, std::true_type{});
+      if constexpr (decltype(has_bias)::value) {
+        constexpr bool kFold = std::is_same_v<T, __bf16>;
+        const bool fold = kFold && fold_masks_ok(plan);
+        // (every instance with an exact bias knows masked tiles: the last key tile is a short one)
+        if (exact_bias(geo)) return fold ? go(Yes{}, Yes{}, std::bool_constant<kFold>{}, Yes{}) : go(Yes{}, Yes{}, No{}, Yes{});
+        if (plan.masked_tiles && fold) return go(Yes{}, Yes{}, std::bool_constant<kFold>{}, No{});
       }
-      if (plan.masked_tiles) go(has_bias, std::true_type{}, std::false_type{});
-      else go(has_bias, std::false_type{}, std::false_type{});
+      if (plan.masked_tiles) go(has_bias, Yes{}, No{}, No{});
+      else go(has_bias, No{}, No{}, No{});
     };
     if (a.bias != nullptr) by_mask(std::true_type{});
     else by_mask(std::false_type{});

@@ -27,7 +27,6 @@ struct FwdArgsT {
   int bias_vec;  // rows of the bias 16-byte aligned
   float scale;
   float lazy;    // fast kernels: log2 slack of the running max (see kLazyRescale)
-  int edge_bias; // fast kernels: bias_frag marks non-finite float16 elements (see edge16)
   const T* bias_frag;        // fragment-major copy of the shared biases, or nullptr
   int64_t bf_sample_stride;  // elements per sample in bias_frag
   int bf_nqt, bf_nkt;        // 32-query / 32-key tiles per head in bias_frag
@@ -81,7 +80,6 @@ struct BwdArgsT {
   int64_t bf_sample_stride;
   int bf_nqt, bf_nkt;
   int delta_in_dq;           // fast dQ kernel computes delta (and stores it) instead of reading it
-  int exact_weight;          // fast kernels: the bias weight in two terms
   int direct_dbias;          // float32 dQ kernel: shared biases have one group, dBias = dS is written there
 };
 
@@ -188,8 +186,8 @@ struct Plan {
 bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan);
 // fast_path_ok but for how the bias is read: the fragment-major copy may be planned
 bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan);
-// the bias weight of the identity MFMAs takes two terms (see exact_weight in attn_fwd_fast.hip)
-bool exact_weight(const oops_attn_geometry& geo);
+// the fast kernels add the bias in float32, as the generic ones do (see ExactBias in attn_fast_common.h)
+bool exact_bias(const oops_attn_geometry& geo);
 // bias rows that are not 16-byte aligned: only the fragment-major copy can be read
 inline bool bias_unaligned(const oops_attn_geometry& geo) { return geo.has_bias && geo.vec_ok == OOPS_VEC_QKV; }
 // key masks may be folded into the bias fragments (every sample's keys fit the fold table)
@@ -267,7 +265,6 @@ inline void fill_bwd_args(BwdArgsT<T, BT>& a, const oops_attn_geometry& geo, con
   a.bf_nqt = plan.bf_nqt;
   a.bf_nkt = plan.bf_nkt;
   a.delta_in_dq = 0;
-  a.exact_weight = geo.has_bias && exact_weight(geo);
   a.direct_dbias = 0;
 }
 
