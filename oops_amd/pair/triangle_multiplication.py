@@ -334,6 +334,7 @@ def _contract(factors: Tensor, out: Tensor, blocks, direction: str, grad: bool =
 # mask and biases: forward 141 and 139 us at 101 residues, 140 and 210 at 301, 245 and 506 at 509; forward +
 # backward 997 and 1909 us at 509)
 PAD_MIN_SIDE = 96
+_F32_TINY = torch.finfo(torch.float32).tiny
 
 
 def _padded_side(n: int, grouped: Tensor, hidden: int) -> int:
@@ -758,7 +759,9 @@ def _run(grouped: Tensor, mask: Optional[Tensor], blocks, direction, weights, bi
     _admit(grouped, weights, biases)
     if len(blocks) == 1:
         n = blocks[0][1]
-        side = _padded_side(n, grouped, weights[2].shape[0])
+        # (the combined values of a padded cell are zeros: without a positive eps_out the output LayerNorm would
+        # divide them by 0, and 0 * inf would reach every gradient)
+        side = _padded_side(n, grouped, weights[2].shape[0]) if eps_out >= _F32_TINY else n
         blocks = [(0, side)]
     flat = [v for block in blocks for v in block]
     rest = (flat, direction, float(eps_in), float(eps_out))

@@ -64,3 +64,25 @@ def test_against_unpadded(monkeypatch, offset):
         err = (a.float() - b.float()).norm() / b.float().norm()
         # one rounding of bfloat16 intermediates differs at most where a library GEMM sums in another order
         assert err <= 2.0**-8, float(err)
+
+
+@pytest.mark.parametrize("eps", [0.0, 1e-50, 1e-12])
+def test_small_output_eps(eps):
+    """An output LayerNorm without (or with an all but vanishing) eps: no cell of the pair has equal channels, so
+    every value is finite, as on the unpadded kernels."""
+
+    n, c, dtype = 101, 64, torch.bfloat16
+    g = torch.Generator().manual_seed(3)
+    pair = torch.randn(1, n, n, c, generator=g).to(dtype).to(DEV).requires_grad_(True)
+    dout = torch.randn(1, n, n, c, generator=g).to(dtype).to(DEV)
+    weights, bs = _params(dtype, c, c, seed=4, biases=True)
+    kwargs = dict(zip(mod._WEIGHT_NAMES + mod._BIAS_NAMES, (*weights, *bs)))
+    leaves = [pair, *(t for t in kwargs.values() if t.requires_grad)]
+
+    def run(e):
+        out = triangle_multiplication(pair, None, direction="outgoing", output_norm_eps=e, **kwargs)
+        return (out, *torch.autograd.grad(out, leaves, dout))
+
+    for a, b in zip(run(eps), run(1e-10)):  # (1e-10 is nothing beside the variances here)
+        assert bool(a.isfinite().all())
+        assert (a.float() - b.float()).norm() <= 2.0**-8 * b.float().norm()
