@@ -436,7 +436,9 @@ def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_we
     att5, single_rows, weight = _operands(att_qhd, single, gate_weight, dtype)
     traced = needs_custom_op(att5)
     shape = att_qhd.shape[:-2]
-    if not traced and _stage_ok(att5, single_rows, weight, output_weight):
+    # (a tangent of the output weight is the projection's to carry: the stage's kernels would drop it)
+    stage = not traced and not forward_mode_active(output_weight)
+    if stage and _stage_ok(att5, single_rows, weight, output_weight):
         operands = (att5, single_rows, weight, output_weight)
         if torch.is_grad_enabled() and any(t.requires_grad for t in operands):
             out = _EagerStage.apply(*operands)

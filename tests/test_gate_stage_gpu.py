@@ -197,3 +197,21 @@ def test_gate_stage_graph_replays(c):
         assert all(torch.equal(g, w) for g, w in zip(got, want))
         step()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("c", [128, 384])
+def test_tangent_of_output_weight(c):
+    """The output is linear in the output weight, so its tangent is the stage of the weight's; with gradients the
+    projection refuses forward mode."""
+
+    att, single, wg, wo = _inputs(torch.bfloat16, (1,), 4, 40, 32, c, c)
+    tangent = torch.randn_like(wo)
+    with torch.autograd.forward_ad.dual_level():
+        with torch.no_grad():
+            dual = torch.autograd.forward_ad.make_dual(wo.detach(), tangent)
+            out = torch.autograd.forward_ad.unpack_dual(oops_amd.gate_attention_output(att, single, wg, dual))
+            want = oops_amd.gate_attention_output(att, single, wg, tangent)
+        assert out.tangent is not None
+        torch.testing.assert_close(out.tangent, want, rtol=2.0**-6, atol=2.0**-6)
+        with pytest.raises(RuntimeError):
+            oops_amd.gate_attention_output(att, single, wg, torch.autograd.forward_ad.make_dual(wo, tangent))
