@@ -134,7 +134,7 @@ def _backward_impl(
     """(grad_attention, grad_logits), each ``(rows, H*D)`` or empty when not needed."""
 
     lib = _lib.load()
-    grad = grad.contiguous()
+    grad = grad.resolve_neg().contiguous()
     grad_attention = torch.empty_like(logits) if need_attention else logits.new_empty(0)
     grad_logits = torch.empty_like(logits) if need_logits else logits.new_empty(0)
     if need_attention or need_logits:
@@ -461,6 +461,8 @@ def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_we
 def _operands(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, dtype: torch.dtype):
     """The kernels' operands: attention (B, S, Q, H, D), single rows and gate weight with unit-stride channels."""
 
+    # (raw pointers cannot observe a lazy negation)
+    att_qhd, single, gate_weight = (t.resolve_neg() if t.is_neg() else t for t in (att_qhd, single, gate_weight))
     single = single if single.dtype == dtype else single.to(dtype)
     weight = gate_weight if gate_weight.dtype == dtype else gate_weight.to(dtype)
     att5 = att_qhd if att_qhd.dim() == 5 else att_qhd.unsqueeze(0)

@@ -215,3 +215,23 @@ def test_tangent_of_output_weight(c):
         torch.testing.assert_close(out.tangent, want, rtol=2.0**-6, atol=2.0**-6)
         with pytest.raises(RuntimeError):
             oops_amd.gate_attention_output(att, single, wg, torch.autograd.forward_ad.make_dual(wo, tangent))
+
+
+@pytest.mark.parametrize("dtype,c", [(torch.bfloat16, 64), (torch.bfloat16, 512), (torch.float32, 64)])
+def test_lazily_negated_operands(dtype, c):
+    """Negated views of each operand and of the gradient, in one pass (64 channels) and in separate operators."""
+
+    leaves = _inputs(dtype, (2,), 2, 33, c // 2, c, c)
+    grad = torch.randn(2, 33, c, device="cuda").to(dtype)
+
+    def run(operands, g):
+        out = oops_amd.gate_attention_output(*operands)
+        return (out, *torch.autograd.grad(out, leaves, g))
+
+    want = run(leaves, grad)
+    for i in range(5):
+        neg = [torch._neg_view(-t) if i == j else t for j, t in enumerate(leaves)]
+        g = torch._neg_view(-grad) if i == 4 else grad
+        assert (neg + [g])[i].is_neg()
+        for a, b in zip(run(neg, g), want):
+            torch.testing.assert_close(a, b)
