@@ -45,6 +45,7 @@ from ._runtime import (
 from .pair_bias import pair_bias_attention
 
 _OPERATOR = "gate_attention_output"
+_PLAIN = (Tensor, torch.nn.Parameter)
 _DTYPE_CODE = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 
 
@@ -434,7 +435,8 @@ def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_we
     if not ok:
         return F.linear(_composed(att_qhd, single, gate_weight), output_weight)
     att5, single_rows, weight = _operands(att_qhd, single, gate_weight, dtype)
-    traced = needs_custom_op(att5)
+    # (a subclass in the place of any operand goes through its own dispatch)
+    traced = needs_custom_op(att5) or any(type(t) not in _PLAIN for t in (single, gate_weight, output_weight))
     shape = att_qhd.shape[:-2]
     # (a tangent of the output weight is the projection's to carry: the stage's kernels would drop it)
     stage = not traced and not forward_mode_active(output_weight)

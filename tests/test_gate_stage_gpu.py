@@ -235,3 +235,33 @@ def test_lazily_negated_operands(dtype, c):
         assert (neg + [g])[i].is_neg()
         for a, b in zip(run(neg, g), want):
             torch.testing.assert_close(a, b)
+
+
+class _Wrapped(torch.Tensor):
+    """A wrapper without storage of its own, as quantised and distributed tensors are."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        out = torch.Tensor._make_wrapper_subclass(cls, inner.shape, strides=inner.stride(), dtype=inner.dtype,
+                                                  device=inner.device)  # fmt: skip
+        out.inner = inner
+        return out
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        unwrap = lambda t: t.inner if isinstance(t, cls) else t  # noqa: E731
+        return func(*torch.utils._pytree.tree_map(unwrap, args), **(kwargs or {}))
+
+
+@pytest.mark.parametrize("which", [1, 2, 3])
+@pytest.mark.parametrize("c", [128, 512])
+def test_subclass_operands(which, c):
+    """A wrapper in the place of single, gate weight or output weight is dispatched, not read."""
+
+    operands = [t.detach() for t in _inputs(torch.bfloat16, (1,), 4, 48, c // 4, c, c)]
+    want = oops_amd.gate_attention_output(*operands)
+    operands[which] = _Wrapped(operands[which])
+    with torch.no_grad():
+        got = oops_amd.gate_attention_output(*operands)
+    got = got.inner if isinstance(got, _Wrapped) else got
+    torch.testing.assert_close(got, want, rtol=2.0**-6, atol=2.0**-6)
