@@ -661,8 +661,10 @@ bool linear_grads_ok(int dtype, int64_t rows, int64_t k, int64_t n, const void* 
   if (row_grad_parts(dtype, rows, k, n) == 0) return false;
   for (const void* p : {x, w, y, d})
     if (reinterpret_cast<uintptr_t>(p) & 15) return false;
-  for (int64_t s : {x_row, w_row, y_row, d_row})
-    if (s < 0 || s % 8 || !rows_fit(s, kWideCols)) return false;
+  // (offsets within a tile's rows, and over all of the weight's: gate_stage_ok's limits)
+  for (int64_t s : {x_row, y_row, d_row})
+    if (s < 0 || s % 8 || !rows_fit(s, kStageRows)) return false;
+  if (w_row < 0 || w_row % 8 || !rows_fit(w_row, kWideCols)) return false;
   return x_row >= k && d_row >= n;
 }
 

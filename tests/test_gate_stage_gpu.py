@@ -265,3 +265,19 @@ def test_subclass_operands(which, c):
         got = oops_amd.gate_attention_output(*operands)
     got = got.inner if isinstance(got, _Wrapped) else got
     torch.testing.assert_close(got, want, rtol=2.0**-6, atol=2.0**-6)
+
+
+def test_far_apart_rows():
+    """Rows of `single` 4M elements apart: the forward takes them, so the backward does."""
+
+    dtype, c, rows = torch.bfloat16, 64, 5
+    att, _, wg, wo = _inputs(dtype, (1,), 2, rows, c // 2, c, c)
+    single = torch.randn(1, rows, 1 << 22, device="cuda", dtype=dtype)[..., :c].requires_grad_()
+    grad = torch.randn(1, rows, c, device="cuda").to(dtype)
+
+    def run(s):
+        out = oops_amd.gate_attention_output(att, s, wg, wo)
+        return (out, *torch.autograd.grad(out, (att, s, wg, wo), grad))
+
+    for a, b in zip(run(single), run(single.detach().contiguous().requires_grad_())):
+        assert torch.equal(a, b)
