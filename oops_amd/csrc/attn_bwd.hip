@@ -776,10 +776,11 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
       if (err == hipSuccess) err = hipGetLastError();
     };
     const bool f32 = attn_f32_ok(geo, plan);
-    // float32: the shared dBias comes from the dQ kernel (all phases run, or none of it is wanted)
+    // float32: the shared dBias comes from the dQ kernel in a call that asks for both (a call with one of the
+    // phases runs the kernels of that phase)
     const bool both = (phases & OOPS_PHASE_DQ) && (phases & OOPS_PHASE_DBIAS) && a.dbias != nullptr;
     const bool f32_fused = f32 && plan.f32_fused && both;
-    const bool f32_direct = f32 && plan.f32_direct;
+    const bool f32_direct = f32 && plan.f32_direct && both;
     const bool need_dq = dq != nullptr || (a.dbias != nullptr && (plan.any_full || f32_fused || f32_direct));
     const bool run_dq = (phases & OOPS_PHASE_DQ) && need_dq && plan.fwd_tiles > 0;
     // the fast dQ kernel computes delta itself when it runs first
@@ -787,6 +788,7 @@ hipError_t launch_backward(const oops_attn_geometry& geo, const Plan& plan, cons
     auto launch_f32 = [&](int phase) {
       if constexpr (std::is_same_v<T, float>) {
         a.delta_in_dq = 1;
+        a.direct_dbias = f32_direct;
         if (err == hipSuccess) err = launch_backward_f32(plan, a, phase, stream);
       }
     };

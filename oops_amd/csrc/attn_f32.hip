@@ -943,7 +943,6 @@ hipError_t launch_backward_f32(const Plan& plan, BwdArgsT<float, float> a, int p
     else go(std::integral_constant<int, 8>{});
     return hipGetLastError();
   }
-  a.direct_dbias = plan.f32_direct;
   const int64_t tiles = phase == OOPS_PHASE_DQ ? plan.fwd_tiles : phase == OOPS_PHASE_DKV ? plan.dkv_tiles : plan.sbias_tiles;
   a.total_tiles = tiles;
   a.uniform_tiles = phase == OOPS_PHASE_DQ ? plan.fwd_uniform : phase == OOPS_PHASE_DKV ? plan.dkv_uniform : plan.sbias_uniform;

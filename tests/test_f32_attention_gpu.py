@@ -4,7 +4,7 @@ class, bias layout and mask, against the float64 oracle at the float32 criterion
 import pytest
 import torch
 
-from oops_amd import pair_bias_attention, triangle_attention
+from oops_amd import _lib, pair_bias_attention, triangle_attention
 from oops_amd.attention import _core
 
 from test_triangle_gpu import make_case, run_and_check
@@ -95,3 +95,17 @@ def test_rectangular_misaligned_bias_and_partial_gradients():
         want = run()
     for g_, w in zip(got, want):
         torch.testing.assert_close(g_, w, rtol=1e-5, atol=1e-5)
+
+
+def test_single_group_phases():
+    """A call for the shared dBias alone (no dQ) writes it, though the dQ kernel would when both are asked."""
+
+    q, k, v, _, bias, dout = make_case(torch.float32, prefix=(1,), rows=1, cols=129, head=32, masked=False, seed=6)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v, bias)]
+    out = triangle_attention(*leaves[:3], None, leaves[3])
+    want = torch.autograd.grad(out, leaves[3], dout.to(DEV), retain_graph=True)[0]
+    junk = torch.full((1 << 22,), 7.0, device=DEV)  # (what the allocator hands out next)
+    del junk
+    with _core.profile_phases(_lib.PHASE_DELTA | _lib.PHASE_DBIAS):
+        got = torch.autograd.grad(out, leaves[3], dout.to(DEV))[0]
+    torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5)
