@@ -898,7 +898,7 @@ void by_dp(const Plan& plan, F&& f) {
 // alone.
 bool attn_f32_ok(const oops_attn_geometry& geo, const Plan& plan) {
   return geo.force_generic != 1 && geo.dtype == OOPS_F32 && plan.dp <= 64 && geo.head_size % 4 == 0 &&
-         geo.vec_ok != 0 && !plan.any_pair_mask && plan.offsets_32bit && plan.q_offsets_32bit && plan.max_len_k <= 32 * kF32MaxTiles;
+         geo.vec_ok != 0 && !plan.any_pair_mask && !plan.any_bare && plan.offsets_32bit && plan.q_offsets_32bit && plan.max_len_k <= 32 * kF32MaxTiles;
 }
 
 // The dQ + dBias kernel: its sums of all key tiles have to fit the registers

@@ -472,7 +472,7 @@ bool exact_bias(const oops_attn_geometry& geo) { return bias_unaligned(geo); }
 bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan) {
   if (geo.force_generic == 1) return false;
   if (geo.dtype == OOPS_F32 || plan.dp > 64 || plan.max_len_k > 64 * kMaxKeyTiles || plan.any_pair_mask ||
-      !geo.vec_ok || geo.head_size % 8 != 0 || !plan.offsets_32bit)
+      plan.any_bare || !geo.vec_ok || geo.head_size % 8 != 0 || !plan.offsets_32bit)
     return false;
   if (geo.has_bias && geo.bias_dtype != geo.dtype) return false;
   return !bias_unaligned(geo) || unaligned_bias_ok(geo, plan);

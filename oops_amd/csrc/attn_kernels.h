@@ -154,6 +154,7 @@ struct Plan {
   int fast_parts = 1;                            // largest per-sample part count (fast path)
   int64_t fast_part_groups = 1;                  // groups per part the fast path aims at
   bool any_full = false, any_shared = false;
+  bool any_bare = false;                         // has_bias, but some sample has none (generic kernels only)
   bool all_shared = false;                       // every sample has a row-shared bias
   // fused dK/dV + shared dBias kernel (attn_bwd_fused.hip): 32-key blocks x group ranges
   int64_t fused_tiles = 0, fused_uniform = 0;

@@ -130,6 +130,7 @@ int make_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
       const int64_t qspan = (S.Lq * std::max({S.q_si, S.o_si, S.do_si}) + geo->head_size) * elt;
       if (qspan >= lim) plan.q_offsets_32bit = false;
     }
+    if (geo->has_bias && S.b_off < 0) plan.any_bare = true;
     if (geo->has_bias && S.b_off >= 0) {
       if (S.bias_mode == OOPS_BIAS_FULL) plan.any_full = true;
       if (S.bias_mode == OOPS_BIAS_SHARED) {

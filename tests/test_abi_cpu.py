@@ -277,3 +277,22 @@ def test_trimul_output_grad_validation(lib):
         tg.dtype, tg.channels, tg.hidden = dtype, c, h
         assert lib.oops_trimul_output_grad_parts(ctypes.byref(tg)) == 0
         assert lib.oops_trimul_output_grad_products(ctypes.byref(tg), *args) != 0
+
+
+@pytest.mark.parametrize("dtype", [_lib.BF16, _lib.F32])
+def test_sample_without_bias_in_a_biased_table(lib, dtype):
+    """Only the generic kernels know a sample without a bias (negative b_off) beside biased ones: no copy of
+    the bias, no dQ + dBias partials, as with the generic kernels forced."""
+
+    table = c3_table(n=128)
+    bare = list(table)
+    bare[_lib.T_B_OFF], bare[_lib.T_BIAS_MODE] = -1, _lib.BIAS_NONE
+    bare[_lib.T_L_OFF] = 128 * 4 * 128
+    for rows in (table + bare, bare + table):
+        geo, keep = _geometry(rows, dtype=dtype)
+        forced, keep2 = _geometry(rows, dtype=dtype)
+        forced.force_generic = 1
+        for size in (lib.oops_attn_forward_workspace_bytes, lib.oops_attn_backward_workspace_bytes):
+            assert size(ctypes.byref(geo)) == size(ctypes.byref(forced))
+    geo, keep = _geometry(table + table, dtype=dtype)  # (both biased: the copy is there)
+    assert (lib.oops_attn_forward_workspace_bytes(ctypes.byref(geo)) > 0) == (dtype == _lib.BF16)

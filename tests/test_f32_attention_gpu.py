@@ -109,3 +109,31 @@ def test_single_group_phases():
     with _core.profile_phases(_lib.PHASE_DELTA | _lib.PHASE_DBIAS):
         got = torch.autograd.grad(out, leaves[3], dout.to(DEV))[0]
     torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sample_without_bias(dtype):
+    """A table whose first sample has no bias beside a biased one, forward and backward, against calls of its own."""
+
+    s, n, h, d = 3, 72, 2, 32
+    q, k, v, mask, bias, dout = make_case(dtype, prefix=(2,), rows=s, cols=n, heads=h, head=d, masked=False, seed=8)
+    q, k, v, bias, dout = (t.to(DEV) for t in (q, k, v, bias, dout))
+    per_b, st = s * n * h * d, (n * h * d, d, h * d)
+    table, lse = [], s * h * n
+    for b in range(2):
+        qs = (b * per_b, *st)
+        biased = dict(bias=(h * n * n, 0, n * n, n), dbias=(0, 0, n * n, n), bias_mode=_lib.BIAS_SHARED) if b else {}
+        table += _core.table_row(groups=s, len_q=n, len_k=n, q=qs, k=qs, v=qs, lse_off=b * lse, **biased)
+    scale = d**-0.5
+    out, lo, l = _core._forward_impl(q, k, v, None, bias, table, h, scale, 2 * lse, True)
+    dq, dk, dv, db = _core._backward_impl(dout, q, k, v, None, bias, out, lo, l, table, h, scale, h * n * n,
+                                         [True] * 4)
+    for b in range(2):
+        leaves = [t[b : b + 1].clone().requires_grad_(True) for t in ((q, k, v, bias) if b else (q, k, v))]
+        ref = triangle_attention(*leaves[:3], None, leaves[3] if b else None)
+        grads = torch.autograd.grad(ref, leaves, dout[b : b + 1])
+        tol = dict(rtol=1e-4, atol=1e-4) if dtype == torch.float32 else dict(rtol=2e-2, atol=2e-2)
+        for x, y in zip((out, dq, dk, dv), (ref, *grads)):
+            torch.testing.assert_close(x[b : b + 1], y, **tol)
+        if b:
+            torch.testing.assert_close(db.view(h, n, n), grads[3].view(h, n, n).float(), **tol)
