@@ -437,6 +437,8 @@ def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_we
     att5, single_rows, weight = _operands(att_qhd, single, gate_weight, dtype)
     # (a subclass in the place of any operand goes through its own dispatch)
     traced = needs_custom_op(att5) or any(type(t) not in _PLAIN for t in (single, gate_weight, output_weight))
+    if not traced:  # raw pointers cannot observe a lazy negation
+        att5, single_rows, weight = att5.resolve_neg(), single_rows.resolve_neg(), weight.resolve_neg()
     shape = att_qhd.shape[:-2]
     # (a tangent of the output weight is the projection's to carry: the stage's kernels would drop it)
     stage = not traced and not forward_mode_active(output_weight)
@@ -463,8 +465,6 @@ def _gate_output(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, output_we
 def _operands(att_qhd: Tensor, single: Tensor, gate_weight: Tensor, dtype: torch.dtype):
     """The kernels' operands: attention (B, S, Q, H, D), single rows and gate weight with unit-stride channels."""
 
-    # (raw pointers cannot observe a lazy negation)
-    att_qhd, single, gate_weight = (t.resolve_neg() if t.is_neg() else t for t in (att_qhd, single, gate_weight))
     single = single if single.dtype == dtype else single.to(dtype)
     weight = gate_weight if gate_weight.dtype == dtype else gate_weight.to(dtype)
     att5 = att_qhd if att_qhd.dim() == 5 else att_qhd.unsqueeze(0)
