@@ -17,7 +17,9 @@
 // At 196608 rows of 256 channels in bf16, against the separate launches (projection kernel, gate kernels,
 // library GEMMs, chunked weight gradients): forward 108 us for 149, backward 1 142 us for 205, backward 2
 // 85 us for 119, the stage forward and backward 484 -> 306 us.  Few rows gain from the launches: 128 rows
-// forward 50 -> 18 us, forward and backward 256 -> 183 us, so there is no lower limit on the rows.  The
+// forward 50 -> 18 us, forward and backward 256 -> 183 us, so there is no lower limit on the rows (replayed
+// from a graph, 384 channels: forward and backward 36 us at 8 rows for 29 of separate launches, 37 for 35 at 64, 38
+// for 41 at 128; those launches clear a GEMM workspace with a memset, which does not belong in a graph).  The
 // upper limits are the register file's: both 256-wide weights fit beside the forward's accumulators, a 384-wide
 // one beside the gradients' (with a few spilled registers).
 //
@@ -41,10 +43,14 @@ constexpr int kStageRows = 64;   // rows per tile (row_grad_kernel)
 constexpr int kStageWgs = 256;   // workgroups: one per CU
 constexpr int kWideCols = 384;   // the largest C, H*D and O
 // Past 256 channels the forward streams its weights for every 32 rows, which is right for few rows only: forward
-// / forward and backward at 384 channels, eager, against the separate launches: 384 rows 23 / 128 us for 65 / 239,
-// 16384 rows 42 / 120 us for 72 / 304 (replayed from a graph, without host time: 32 / 55 for 26 / 46 and 46 /
-// 116 for 41 / 155).  Further up the streamed weights cost more than the launches save.
+// / forward and backward at 384 channels, replayed from a graph, against the separate launches: 384 rows 11 / 40 us
+// for 12 / 41, 2048 rows 11 / 49 for 15 / 68, 16384 rows 23 / 89 us for 35 / 147 (eager, where the host's time is
+// most of it: 18 / 175 for 55 / 288 and 22 / 172 for 55 / 328).
 constexpr int64_t kWideRows = 16384;
+// From 129 to 256 channels the streaming forward serves one tile per CU: one short workgroup each beats the
+// prologue of the kernel that keeps the weights (replayed at 256 channels: 8.0 us for 12.1 at 384 rows, 9.2 for 12.9
+// at 8192 rows), which walks more rows than that (16.1 for 16384 rows).
+constexpr int64_t kStreamRows = kStageWgs * 32;
 
 struct StageArgs {
   const void* x;       // forward: single [rows][kx]; gradients: X [rows][kx]
@@ -255,60 +261,83 @@ __global__ __launch_bounds__(512, 2) void gate_stage_forward_kernel(StageArgs a)
 
 constexpr int kWideThreads = kWideCols / 32 * 64;
 
-// The forward for up to 384 channels and few rows (the single representation): one 32-row tile per workgroup,
-// the weights' fragments straight from L2 (they do not fit in a workgroup's registers beside each other).  One
-// wave per 32 channels, all of its fragments in flight at once.
+// All but the last N vector-memory operations of this wave are done (no LDS read moves above it)
+template <int N>
+__device__ __forceinline__ void own_loads_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// The forward for 129 to 384 channels and few rows (the single representation): one 32-row tile per workgroup, one
+// wave per 32 channels.  The weights do not fit in a workgroup's registers or LDS, so each wave streams its own 32
+// rows of either in blocks of 64 columns through two LDS slots of its own (direct-to-LDS loads of whole 128-byte
+// lines, the next block in flight; no barrier).  That stream bounds it: 590 KB per workgroup.  Fragments loaded
+// straight from the rows touch 32 lines per load and made it 19 us at 384 rows of 384 channels for 10.8 now.
 template <typename T, bool LOGITS>
 __global__ __launch_bounds__(kWideThreads, 3) void gate_stage_wide_kernel(StageArgs a) {
   using E = Elem<T>;
   using Frag = typename E::Frag;
-  constexpr int RT = 32, P = kWideCols, KS = P / 16;
+  constexpr int RT = 32, P = kWideCols, BLK = 32 * 64;  // BLK: elements of a weight block
   __shared__ __attribute__((aligned(16))) T x_lds[RT * P];
   __shared__ __attribute__((aligned(16))) T y_lds[RT * P];  // attention -> gated
+  __shared__ __attribute__((aligned(16))) T w_lds[kWideThreads / 64][2][BLK];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 31, g2 = lane >> 5;
   const int64_t r0 = (int64_t)blockIdx.x * RT;
   const int nrows = (int)(a.rows - r0 < RT ? a.rows - r0 : RT);
-  auto load_block = [&](const void* w, int64_t w_row, int rows, int k_end, Frag (&f)[KS]) {
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(w, (uint32_t)(((rows - 1) * w_row + k_end) * 2));
-    const int c = 32 * wave + lq;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int k = 16 * ks + 8 * g2;
-      f[ks] = __builtin_bit_cast(Frag, buffer_load16(rs, c < rows && k < k_end ? (uint32_t)((c * w_row + k) * 2) : kOut));
-    }
-  };
-  Frag wf[KS];
-  load_block(a.w, a.w_row, a.n, a.kx, wf);
   {
-    const __amdgpu_buffer_rsrc_t xs =
-        make_rsrc(static_cast<const T*>(a.x) + r0 * a.x_row, (uint32_t)(((nrows - 1) * a.x_row + a.kx) * 2));
-    const __amdgpu_buffer_rsrc_t ys = make_rsrc(a.y, a.a_bytes);
+    const u32x4 xs = rsrc_words(static_cast<const T*>(a.x) + r0 * a.x_row, (uint32_t)(((nrows - 1) * a.x_row + a.kx) * 2));
+    const u32x4 ys = rsrc_words(a.y, a.a_bytes);
 #pragma unroll
     for (int j = 0; j < RT * P / 8 / kWideThreads; ++j) {
-      const int id = tid + kWideThreads * j, r = id / (P / 8), c = (id % (P / 8)) * 8;
-      const bool ok = r < nrows;
-      const uint4 xv = buffer_load16(xs, ok && c < a.kx ? (uint32_t)((r * a.x_row + c) * 2) : kOut);
-      const uint4 yv = buffer_load16(
-          ys, ok && c < a.n ? att_row_bytes(a, (uint32_t)r0 + r) + 2 * ((uint32_t)(c / a.width) * a.a_sh + (uint32_t)(c % a.width))
-                            : kOut);
-      *reinterpret_cast<uint4*>(&x_lds[panel_off<RT>(r, c)]) = xv;
-      *reinterpret_cast<uint4*>(&y_lds[panel_off<RT>(r, c)]) = yv;
+      const int at = (wave * 2 + j) * 64;
+      const Slot<RT> s(at + lane);
+      const bool ok = s.row < nrows;
+      dma16_asm(xs, x_lds + at * 8, ok && s.col < a.kx ? (uint32_t)((s.row * a.x_row + s.col) * 2) : kOut, 0);
+      dma16_asm(ys, y_lds + at * 8,
+                ok && s.col < a.n ? att_row_bytes(a, (uint32_t)r0 + s.row) +
+                                        2 * ((uint32_t)(s.col / a.width) * a.a_sh + (uint32_t)(s.col % a.width))
+                                  : kOut, 0);
     }
   }
-  __syncthreads();
-
-  auto product = [&](const T* tile, const Frag (&f)[KS], uint4& lo, uint4& hi) {
-    f32x16 acc = f32x16{};
+  // block t of the wave's stream: Wg's k blocks, then Wo's (past the last one: zeros, no memory traffic)
+  const int t1 = (a.kx + 63) >> 6, t_end = t1 + ((a.n + 63) >> 6);
+  auto request = [&](int t) {
+    const bool first = t < t1;
+    const int rows = first ? a.n : a.o, cols = first ? a.kx : t < t_end ? a.n : 0, k0 = (first ? t : t - t1) * 64;
+    const int64_t w_row = first ? a.w_row : a.w_out_row;
+    const u32x4 ws = rsrc_words(first ? a.w : a.w_out, (uint32_t)(((rows - 1) * w_row + (first ? a.kx : a.n)) * 2));
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) acc = E::mma(f[ks], lds_frag<T>(tile + panel_off<RT>(lq, 16 * ks + 8 * g2)), acc);
+    for (int j = 0; j < BLK / 512; ++j) {
+      const Slot<32> s(j * 64 + lane);
+      const int c = 32 * wave + s.row, k = k0 + s.col;
+      dma16_asm(ws, &w_lds[wave][t & 1][j * 512], c < rows && k < cols ? (uint32_t)((c * w_row + k) * 2) : kOut, 0);
+    }
+  };
+  constexpr int LOADS = BLK / 512;
+  request(0);
+  request(1);
+  own_loads_wait<2 * LOADS>();
+  lds_barrier();  // single and attention rows written
+
+  auto product = [&](const T* tile, int t, int end, uint4& lo, uint4& hi) {
+    f32x16 acc = f32x16{};
+    for (int k0 = 0; t < end; ++t, k0 += 64) {
+      own_loads_wait<LOADS>();  // (the next block may be in flight; stores in between only make this stricter)
+      const T* wb = w_lds[wave][t & 1];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        acc = E::mma(lds_frag<T>(wb + panel_off<32>(lq, 16 * ks + 8 * g2)),
+                     lds_frag<T>(tile + panel_off<RT>(lq, k0 + 16 * ks + 8 * g2)), acc);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block has been read
+      request(t + 2);
+    }
     round_run<T>(acc, lo, hi);
   };
   uint4 lo, hi;
+  const int c0 = 32 * wave + 16 * g2;
+  product(x_lds, 0, t1, lo, hi);
   if (32 * wave < a.n) {
-    product(x_lds, wf, lo, hi);
-    const int c0 = 32 * wave + 16 * g2;
     if constexpr (LOGITS) {
       const __amdgpu_buffer_rsrc_t lr = make_rsrc(static_cast<T*>(a.e) + r0 * a.n, (uint32_t)(nrows * a.n * 2));
       const uint32_t off = (uint32_t)((lq * a.n + c0) * 2);
@@ -321,16 +350,15 @@ __global__ __launch_bounds__(kWideThreads, 3) void gate_stage_wide_kernel(StageA
     *p0 = c0 < a.n ? gate_product<T>(lo, *p0) : make_uint4(0, 0, 0, 0);
     *p1 = c0 + 8 < a.n ? gate_product<T>(hi, *p1) : make_uint4(0, 0, 0, 0);
   }
-  load_block(a.w_out, a.w_out_row, a.o, a.n, wf);
-  __syncthreads();  // gated rows written
+  lds_barrier();  // gated rows written
+  product(y_lds, t1, t_end, lo, hi);
   if (32 * wave < a.o) {
-    product(y_lds, wf, lo, hi);
-    const int c0 = 32 * wave + 16 * g2;
     const __amdgpu_buffer_rsrc_t orr = make_rsrc(static_cast<T*>(a.d) + r0 * a.o, (uint32_t)(nrows * a.o * 2));
     const uint32_t off = (uint32_t)((lq * a.o + c0) * 2);
     buffer_store16(orr, lq < nrows && c0 < a.o ? off : kOut, lo);
     buffer_store16(orr, lq < nrows && c0 + 8 < a.o ? off + 16 : kOut, hi);
   }
+  vmem_wait_all();  // the last requests land before the LDS is given back
 }
 
 // ------------------------------------------------------------------ gradients
@@ -601,7 +629,7 @@ hipError_t launch_gate_stage_forward(const oops_gate_geometry& g, int64_t out_ch
   a.x_row = g.s_row, a.w_row = g.w_row, a.w_out_row = wo_row;
   a.kx = g.channels, a.n = g.heads * g.width, a.o = (int)out_channels;
   const int most = std::max({a.kx, a.n, a.o});
-  if (most > 256) {
+  if (most > 256 || (most > 128 && g.rows <= kStreamRows)) {
     return by_half(g.dtype, [&](auto tag) -> hipError_t {
       using T = decltype(tag);
       const dim3 grid((unsigned)((g.rows + 31) / 32));

@@ -281,3 +281,44 @@ def test_far_apart_rows():
 
     for a, b in zip(run(single), run(single.detach().contiguous().requires_grad_())):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("c", [136, 256])
+def test_rows_around_the_streaming_forward(c):
+    """The last row count of the streaming forward and the first of the one that keeps its weights: the same sums
+    in the same order, so the same bits."""
+
+    att, single, wg, wo = (t.detach() for t in _inputs(torch.bfloat16, (1,), c // 8, 8193, 8, c, c))
+    more = oops_amd.gate_attention_output(att, single, wg, wo)
+    fewer = oops_amd.gate_attention_output(att[:, :, :8192], single[:, :8192], wg, wo)
+    assert torch.equal(more[:, :8192], fewer)
+
+
+@pytest.mark.parametrize("rows", [48, 300])
+def test_captured_training_step(rows):
+    """Replays on new inputs, with eager work between them: the bits of eager calls."""
+
+    static = _inputs(torch.bfloat16, (1,), 16, rows, 24, 384, 384)
+    grad = torch.randn(1, rows, 384, device="cuda").to(torch.bfloat16)
+
+    def step(x):
+        out = oops_amd.gate_attention_output(*x)
+        return (out, *torch.autograd.grad(out, x, grad))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step(static)
+    for seed in range(1, 4):
+        fresh = _inputs(torch.bfloat16, (1,), 16, rows, 24, 384, 384, seed=seed)
+        with torch.no_grad():
+            for a, b in zip(static, fresh):
+                a.copy_(b)
+        graph.replay()
+        got = [t.clone() for t in captured]
+        for a, b in zip(got, step(fresh)):
+            assert torch.equal(a, b)
