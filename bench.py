@@ -535,6 +535,8 @@ def trimul_stage(device, n=512, c=128, h=128, dtype="bf16"):
         "ms_fwd_bwd": round(ms, 4),
         "ms_fwd": round(ms_fwd, 4),
         "tflops_fwd_bwd": round(flops / ms / 1e9, 2),
+        "factor_kernel_note": "factor_kernel_bwd, timed through the C ABI, is the separate factor backward of calls "
+        "with a mask gradient or other widths; the step above runs it fused with its products",
         "factor_kernel_fwd": kern(k_fwd, fwd_bytes),
         "factor_kernel_bwd": kern(k_bwd, bwd_bytes),
         "roofline_bound": "hbm" if dtype == "bf16" else "mfma (float32)",
@@ -656,6 +658,8 @@ def gate_stage(device):
     return {
         "workload": "gate_attention_output fwd+bwd, rows 512x384, H=8, D=32, C=256, O=256, bf16",
         "ms_fwd_bwd": round(step_ms, 4),
+        "kernel_note": "the two kernels below, timed alone, are those of traced calls and of wider operands; the step "
+        "above runs one pass forward and two backward",
         "projection_kernel": {
             "ms": round(fwd_ms, 4),
             "bound": "hbm",

@@ -893,9 +893,9 @@ void by_dp(const Plan& plan, F&& f) {
 // residues, 4 heads of 32, shared bias, ending node (generic -> here):
 // forward 112 -> 73 us, dK/dV 251 -> 126, dQ + delta + dBias 441 -> 140 (dQ
 // and dBias in separate kernels: 105 + 116); forward + backward 808 -> 335 us.
-// Matrix cores busy 43% (forward), 50% (dK/dV) there, 60% and 70% at 256
-// residues: 193 leaves 1544 workgroups on 256 CUs, and a CU's seventh runs
-// alone.
+// Matrix cores busy 41% (forward), 50% (dK/dV) and 34% (dQ + dBias) there, 60%
+// and 70% (forward, dK/dV) at 256 residues: 193 leaves 1544 workgroups on 256
+// CUs, and a CU's seventh runs alone.
 bool attn_f32_ok(const oops_attn_geometry& geo, const Plan& plan) {
   return geo.force_generic != 1 && geo.dtype == OOPS_F32 && plan.dp <= 64 && geo.head_size % 4 == 0 &&
          geo.vec_ok != 0 && !plan.any_pair_mask && !plan.any_bare && plan.offsets_32bit && plan.q_offsets_32bit && plan.max_len_k <= 32 * kF32MaxTiles;

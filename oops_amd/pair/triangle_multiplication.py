@@ -340,7 +340,7 @@ _F32_TINY = torch.finfo(torch.float32).tiny
 def _padded_side(n: int, grouped: Tensor, hidden: int) -> int:
     """The side on which an ``n x n`` 16-bit pair is worked: ``n`` rounded up to a multiple of 8, so that
     factor rows, contraction operands and norm tiles are 16-byte aligned, where the kernels that know both
-    sides serve the widths; else ``n``."""
+    sides serve the widths (and one pair: they find a row's cell from its index in one grid); else ``n``."""
 
     c = grouped.shape[2]
     if (n % 8 == 0 or n < PAD_MIN_SIDE or grouped.shape[0] != 1 or grouped.dtype not in _KERNEL_DTYPES or c % 8
