@@ -101,8 +101,6 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
       vf[r][s] = __builtin_bit_cast(Frag, buffer_load16(v_rsrc, ok ? (uint32_t)((key * (int)S.v_si + col) * 2) : kOut));
     }
   }
-  const ExactBias<T> xb(a.scale);
-  constexpr bool LAST = XB && ExactBias<T>::kLast;
   Frag ident[2];
   identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
 
@@ -192,7 +190,7 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
     }
   };
 
-  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
+  const float c1 = a.scale * kLog2e;
   f32x16 dk[R][NDT], dv[R][NDT];
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -215,26 +213,26 @@ __global__ __launch_bounds__(256, OOPS_DKV_OCC) void attn_dkv_fast_kernel(BwdArg
         // (XB: from zero, the LSE comes off x)
         const float* nlse = &nlse_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16];
         f32x16 sacc = XB ? f32x16{} : *reinterpret_cast<const f32x16*>(nlse);
-        auto add_bias = [&] {
+        if constexpr (HAS_BIAS) {
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][0]), ident[0], sacc);
           sacc = E::mma(__builtin_bit_cast(Frag, bias[qr][1]), ident[1], sacc);
-        };
-        if constexpr (HAS_BIAS && !LAST) add_bias();
-        if constexpr (XB && !LAST) xb.scale_first(sacc);
+        }
+        f32x16 log_bias;  // XB: log2 e b
+        if constexpr (XB) {
+          log_bias = ExactBias<T>::log2_bias(sacc);
+          sacc = f32x16{};
+        }
         f32x16 pacc = *reinterpret_cast<const f32x16*>(&ndlt_lds[(buf * R + r) * 64 + 32 * qr + g2 * 16]);
 #pragma unroll
         for (int s = 0; s < NQF; ++s) {
           sacc = E::mma(lds_frag<T>(qt + swz_off<DP>(32 * qr + lq, s * 16 + g2 * 8)), kf[r][s], sacc);
           pacc = E::mma(lds_frag<T>(dt + swz_off<DP>(32 * qr + lq, s * 16 + g2 * 8)), vf[r][s], pacc);
         }
-        if constexpr (LAST) {
-          xb.scale_first(sacc);
-          add_bias();
-        }
+        if constexpr (XB) ExactBias<T>::finish(sacc, c1, log_bias);
         float p[16], ds[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          p[j] = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, nlse[j]) : sacc[j] * c1);
+          p[j] = __builtin_amdgcn_exp2f(XB ? sacc[j] + nlse[j] : sacc[j] * c1);
           if (wave_masked[r]) p[j] = kvalid[r] ? p[j] : 0.0f;
           ds[j] = p[j] * pacc[j];
         }
@@ -343,7 +341,6 @@ template <typename T, int DP, bool HAS_BIAS, bool MASKED_TILES, bool FULL_DBIAS,
 __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ? 4 : OOPS_DQ_OCC)) void attn_dq_fast_kernel(
     BwdArgsT<T, T> a) {
   constexpr bool LEAN = kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD>;
-  constexpr bool LAST = XB && ExactBias<T>::kLast;
   static_assert(!FOLD || (MASKED_TILES && HAS_BIAS && sizeof(T) == 2), "fold: masked bf16 tiles with a bias");
   using E = Elem<T>;
   using Frag = typename E::Frag;
@@ -507,7 +504,6 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     }
     ndelta = -dl;
   }
-  const ExactBias<T> xb(a.scale);
   // the pack of the fused dK/dV + dBias kernel: per (g, h) row, -LSE / c (XB: -LSE) of
   // the Lq queries (lanes 0..31), then -delta (lanes 32..63)
   if (a.ld_pack != nullptr && qv) {
@@ -634,7 +630,7 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     return t;
   };
 
-  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
+  const float c1 = a.scale * kLog2e;
   f32x16 nd_tile;  // LEAN: the dP accumulator's starting value
 #pragma unroll
   for (int j = 0; j < 16; ++j) nd_tile[j] = LEAN ? ndelta : 0.0f;
@@ -652,29 +648,31 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
     const uint4* fm = reinterpret_cast<const uint4*>(&fold_lds[FOLD ? (t * 2 + g2) * 16 : 0]);
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      f32x16 sacc = f32x16{};
-      auto add_bias = [&] {
+      f32x16 sacc;
+      if constexpr (HAS_BIAS) {
         const uint4 b0 = FOLD ? fold_bias(bf[t2][0], fm[t2 * 2]) : bf[t2][0];
         const uint4 b1 = FOLD ? fold_bias(bf[t2][1], fm[t2 * 2 + 1]) : bf[t2][1];
-        sacc = E::mma(ident[0], __builtin_bit_cast(Frag, b0), sacc);
+        sacc = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
         sacc = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc);
-      };
-      if constexpr (HAS_BIAS && !LAST) add_bias();
-      if constexpr (XB && !LAST) xb.scale_first(sacc);
+      } else {
+        sacc = f32x16{};
+      }
+      f32x16 log_bias;  // XB: log2 e b
+      if constexpr (XB) {
+        log_bias = ExactBias<T>::log2_bias(sacc);
+        sacc = f32x16{};
+      }
       f32x16 pacc = LEAN ? nd_tile : f32x16{};
 #pragma unroll
       for (int s = 0; s < NQF; ++s) {
         sacc = E::mma(lds_frag<T>(kt + (32 * t2 + lq) * LD + s * 16 + g2 * 8), qf[s], sacc);
         pacc = E::mma(lds_frag<T>(vt + (32 * t2 + lq) * LD + s * 16 + g2 * 8), df[s], pacc);
       }
-      if constexpr (LAST) {
-        xb.scale_first(sacc);
-        add_bias();
-      }
+      if constexpr (XB) ExactBias<T>::finish(sacc, c1, log_bias);
       float ds[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        float p = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, neg_lse) : __builtin_fmaf(sacc[j], c1, neg_lse));
+        float p = __builtin_amdgcn_exp2f(XB ? sacc[j] + neg_lse : __builtin_fmaf(sacc[j], c1, neg_lse));
         if constexpr (MASKED) {
           const int kk = 32 * t2 + ((j >> 2) << 3) + (j & 3);
           p = ((lb >> kk) & 1) ? p : 0.0f;
@@ -763,9 +761,7 @@ __global__ __launch_bounds__(256, (kLeanDq<DP, MASKED_TILES, FULL_DBIAS, FOLD> ?
 // dS block accumulates in registers (no atomics).  Partial sums per part are
 // added by attn_dbias_reduce_kernel.
 // Reference: _backward_shared_bias (oops/attention/triangle/triton/kernel.py:721-873).
-// MASKED_TILES, XB: as in attn_dq_fast_kernel; with XB the logits are the
-// generic kernels' x = scale log2 e Q.K + log2 e b, the second term being what
-// the block keeps.
+// MASKED_TILES, XB: as in attn_dq_fast_kernel.
 template <typename T, int DP, bool MASKED_TILES, bool XB = false>
 __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(BwdArgsT<T, T> a) {
   using E = Elem<T>;
@@ -830,7 +826,7 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
   f32x16 bacc[2];
   {
     Frag ident[2];
-    identity_frags<T>(ident, XB ? ExactBias<T>::kBlockWeight : 1.0f / a.scale, lane);
+    identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
     // (from the fragment-major copy, or from the aligned bias rows when there is none)
     const T* brow = a.bias + S.b_off + h * S.b_sh + (int64_t)q_lane * S.b_si;
     const int qt = qb * 4 + wave;
@@ -852,10 +848,7 @@ __global__ __launch_bounds__(256, OOPS_DBIAS_OCC) void attn_dbias_fast_kernel(Bw
         }
         bacc[t2] = E::mma(ident[c], __builtin_bit_cast(Frag, u), bacc[t2]);
       }
-      if constexpr (XB) {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) bacc[t2][j] = ExactBias<T>::log2_bias(bacc[t2][j]);
-      }
+      if constexpr (XB) bacc[t2] = ExactBias<T>::log2_bias(bacc[t2]);
     }
   }
   f32x16 acc[2];

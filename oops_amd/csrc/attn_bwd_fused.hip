@@ -190,9 +190,7 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
   const int g_end = __builtin_amdgcn_readfirstlane((int)(G * (part + 1) / P));
   const int D = a.head_size;
   const int nqt = (Lq + 31) >> 5;  // <= NS * 4 (the launch picks NS for the longest sample)
-  const ExactBias<T> xb(a.scale);
-  constexpr bool LAST = XB && ExactBias<T>::kLast;
-  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
+  const float c1 = a.scale * kLog2e;
   const int key = kb * 32 + lq;  // this lane's key
   const bool has_mask = MASKED && a.mask != nullptr && S.m_off >= 0;
 
@@ -493,22 +491,27 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
       const T* dt_ = reinterpret_cast<const T*>(cur.d);
       // (XB: from zero, the LSE comes off x)
       f32x16 sacc = XB ? f32x16{} : *reinterpret_cast<const f32x16*>(&cur.ld[g2 * 16]);
-      auto add_bias = [&] {
+      {
         const T* bq = bias_lds + (i * kRowWaves + wq) * 2 * 64 * 8 + lane * 8;
         sacc = E::mma(lds_frag<T>(bq), ident[0], sacc);
         sacc = E::mma(lds_frag<T>(bq + 64 * 8), ident[1], sacc);
-      };
-      if constexpr (!LAST) add_bias();
-      if constexpr (XB && !LAST) xb.scale_first(sacc);
+      }
+      f32x16 log_bias;  // XB: log2 e b
+      if constexpr (XB) {
+        log_bias = ExactBias<T>::log2_bias(sacc);
+        sacc = f32x16{};
+      }
+      if constexpr (XB) {  // (x before dP: the registers hold three accumulators at a time, not four)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) sacc = E::mma(lds_frag<T>(qt_ + swz_off<32>(lq, s * 16 + g2 * 8)), kf[s], sacc);
+        ExactBias<T>::finish(sacc, c1, log_bias);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       f32x16 pacc = *reinterpret_cast<const f32x16*>(&cur.ld[32 + g2 * 16]);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        sacc = E::mma(lds_frag<T>(qt_ + swz_off<32>(lq, s * 16 + g2 * 8)), kf[s], sacc);
+        if constexpr (!XB) sacc = E::mma(lds_frag<T>(qt_ + swz_off<32>(lq, s * 16 + g2 * 8)), kf[s], sacc);
         pacc = E::mma(lds_frag<T>(dt_ + swz_off<32>(lq, s * 16 + g2 * 8)), vf[s], pacc);
-      }
-      if constexpr (LAST) {
-        xb.scale_first(sacc);
-        add_bias();
       }
       // two halves of 8 scores: each half's P and dS feed their MFMAs at once
 #pragma unroll
@@ -517,7 +520,7 @@ __global__ __launch_bounds__(512, 1) void attn_dkvb_fast_kernel(BwdArgsT<T, T> a
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int j = 8 * m + e;
-          p[e] = __builtin_amdgcn_exp2f(XB ? xb.log2_less(sacc[j], c1, cur.ld[g2 * 16 + j]) : sacc[j] * c1);
+          p[e] = __builtin_amdgcn_exp2f(XB ? sacc[j] + cur.ld[g2 * 16 + j] : sacc[j] * c1);
           if (MASKED && wave_masked) p[e] = kvalid ? p[e] : 0.0f;
           ds[e] = p[e] * pacc[j];
           region[i][j] += ds[e];

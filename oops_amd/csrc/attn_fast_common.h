@@ -143,46 +143,31 @@ __device__ __forceinline__ uint4 marked16(uint4 u) {
 }
 
 // The float32 bias of the routes that replace the generic kernels (bias rows
-// that are not 16-byte aligned).  Those compute x = scale log2 e Q.K +
-// log2 e b in float32; a weight 1/scale rounded to 16 bits would change b by
-// up to 2^-9 of itself.  So the identity MFMA's weight is exact here, and the
-// vector unit scales one of the two terms by a float32 factor (one
-// multiplication per score, two in float16).  b is the element, or the mark of
-// one that is not finite (marked1): a mark has to make the logit infinite, a
-// finite element only where it does in the generic kernels.
-//   bfloat16: kWeight b + (kWeight scale) Q.K, Q.K first.  kWeight b overflows
-//     for exactly the elements whose log2 e b does, the marks among them
-//     (b / scale would for smaller ones).
-//   float16: b / scale + Q.K, b first: the MFMA's 2 (b / 2) is at most 65504, a
-//     mark's 131008; of these only the mark is infinite times 2^112.
-// x is rounded before the maximum or the LSE is taken off it, as in the
-// generic kernels: a fused multiply-add would leave the product's rounding,
-// which is more than exp2 can take where every logit of a row is large (a row
-// of -1e9, or of half the lowest bfloat16).
+// that are not 16-byte aligned): their logits, bit for bit,
+//   x = fma(Q.K, scale log2 e, log2 e b),
+// of which P = exp2(x - max) or exp2(x - LSE), each difference rounded by
+// itself.  Anything else is another function of large logits (a weight 1/scale
+// rounded to 16 bits changes b by up to 2^-9 of itself, a sum in other units
+// rounds or overflows elsewhere), and a forward and a backward that run on
+// different kernels would not meet.  The identity MFMA brings b, with weight
+// 1, into accumulator order (a mark stays one, see marked1): three vector
+// operations per score for one.  float16: the MFMA's 2 (b / 2) is at most
+// 65504, a mark's 131008; of these only the mark is infinite times 2^112, and
+// a power of two changes no other rounding.
 template <typename T>
 struct ExactBias {
   static constexpr bool kBf = std::is_same_v<T, __bf16>;
-  static constexpr bool kLast = kBf;  // the bias is added after Q.K
-  static constexpr float kWeight = kBf ? 1.4453125f : 2.0f;
-  float scale;
-  __device__ __forceinline__ explicit ExactBias(float s) : scale(s) {}
-  // the first term, before the second is added to it
-  __device__ __forceinline__ void scale_first(f32x16& s) const {
-    const float r = kBf ? kWeight * scale : 0x1p-112f / scale;
+  static constexpr float kWeight = kBf ? 1.0f : 2.0f;
+  // log2 e b from the MFMA's output (marks: infinite)
+  static __device__ __forceinline__ f32x16 log2_bias(f32x16 b) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) s[j] = kBf ? s[j] * r : (s[j] * 0x1p112f) * r;
+    for (int j = 0; j < 16; ++j) b[j] = kBf ? b[j] * kLog2e : (b[j] * 0x1p112f) * (kLog2e * 0x1p-112f);
+    return b;
   }
-  // log2 units per unit of the sum
-  __device__ __forceinline__ float unit() const { return kBf ? kLog2e / kWeight : scale * kLog2e; }
-  // x (the sum s in log2 units, rounded) + c
-  static __device__ __forceinline__ float log2_less(float s, float unit, float c) {
-#pragma clang fp contract(off)
-    return s * unit + c;
-  }
-  // log2 e b of an identity MFMA with weight kBlockWeight alone (marks: infinite)
-  static constexpr float kBlockWeight = kBf ? 1.0f : 2.0f;
-  static __device__ __forceinline__ float log2_bias(float b) {
-    return kBf ? b * kLog2e : (b * 0x1p112f) * (kLog2e * 0x1p-112f);
+  // Q.K to x
+  static __device__ __forceinline__ void finish(f32x16& qk, float c1, const f32x16& lb) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) qk[j] = __builtin_fmaf(qk[j], c1, lb[j]);
   }
 };
 

@@ -142,7 +142,6 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
   }
   // identity A-fragments carrying the bias weight (1/scale; see ExactBias otherwise): MFMA c adds bias keys
   // 16c..16c+15
-  const ExactBias<T> xb(a.scale);
   Frag ident[2];
   identity_frags<T>(ident, XB ? ExactBias<T>::kWeight : 1.0f / a.scale, lane);
 
@@ -243,16 +242,8 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
 #pragma unroll
       for (int c = 0; c < 2; ++c) bf[t2][c] = buffer_load16_s(b_rsrc, t < ntiles ? b_off[t2][c] + s : kOut, 0);
   };
-  // S^T of a tile (bias by identity MFMA and Q K^T) from LDS buffer buf
-  constexpr bool LAST = XB && ExactBias<T>::kLast;
-  auto qk_tile = [&](auto bc, int t2, const f32x16& from, f32x16& acc) {
-#pragma unroll
-    for (int s = 0; s < NQF; ++s) {
-      const Frag kf = __builtin_bit_cast(
-          Frag, *reinterpret_cast<const uint4*>(kbuf(bc) + swz_off<DP>(32 * t2 + lq, s * 16 + g2 * 8)));
-      acc = E::mma(kf, qf[s], s == 0 ? from : acc);
-    }
-  };
+  // S^T of a tile (bias by identity MFMA, then Q K^T; XB: x) from LDS buffer buf
+  const float c1 = a.scale * kLog2e;
   auto scores = [&](auto bc, int t, const uint4 (&bf)[2][2], f32x16 (&sacc)[2]) {
     const uint4* fm = reinterpret_cast<const uint4*>(&fold_lds[FOLD ? (t * 2 + g2) * 16 : 0]);
 #pragma unroll
@@ -263,17 +254,23 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
         const uint4 r1 = use_bf ? bf[t2][1] : finite16<T>(bf[t2][1]);
         const uint4 b0 = FOLD ? fold_bias(r0, fm[t2 * 2]) : r0;
         const uint4 b1 = FOLD ? fold_bias(r1, fm[t2 * 2 + 1]) : r1;
-        if constexpr (LAST) {
-          qk_tile(bc, t2, f32x16{}, sacc[t2]);
-          xb.scale_first(sacc[t2]);
-        }
-        sacc[t2] = E::mma(ident[0], __builtin_bit_cast(Frag, b0), LAST ? sacc[t2] : f32x16{});
+        sacc[t2] = E::mma(ident[0], __builtin_bit_cast(Frag, b0), f32x16{});
         sacc[t2] = E::mma(ident[1], __builtin_bit_cast(Frag, b1), sacc[t2]);
-        if constexpr (XB && !LAST) xb.scale_first(sacc[t2]);
       } else {
         sacc[t2] = f32x16{};
       }
-      if constexpr (!LAST) qk_tile(bc, t2, sacc[t2], sacc[t2]);
+      f32x16 log_bias;  // XB: log2 e b
+      if constexpr (XB) {
+        log_bias = ExactBias<T>::log2_bias(sacc[t2]);
+        sacc[t2] = f32x16{};
+      }
+#pragma unroll
+      for (int s = 0; s < NQF; ++s) {
+        const Frag kf = __builtin_bit_cast(
+            Frag, *reinterpret_cast<const uint4*>(kbuf(bc) + swz_off<DP>(32 * t2 + lq, s * 16 + g2 * 8)));
+        sacc[t2] = E::mma(kf, qf[s], sacc[t2]);
+      }
+      if constexpr (XB) ExactBias<T>::finish(sacc[t2], c1, log_bias);
     }
   };
 
@@ -288,7 +285,6 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
     return t;
   };
 
-  const float c1 = XB ? xb.unit() : a.scale * kLog2e;
   float m_run = kNegInf;  // reference max (log2 units), raised lazily
   float neg_m = 0.0f;     // -m_run (0 while no key has been seen)
   float l_run = 0.0f;     // this lane's partial row sum
@@ -322,7 +318,7 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
       for (int j = 3; j < 15; j += 2) x = fmaxf(fmaxf(x, sacc[t2][j]), sacc[t2][j + 1]);
       mc[t2] = fmaxf(x, sacc[t2][15]);
     }
-    float mx = max_halves(fmaxf(mc[0], mc[1])) * c1;
+    float mx = max_halves(fmaxf(mc[0], mc[1])) * (XB ? 1.0f : c1);
     const bool grow = mx > m_run + a.lazy;
     if (__any(grow)) {
       const float m_new = grow ? mx : m_run;
@@ -337,7 +333,7 @@ __global__ __launch_bounds__(256, OOPS_FWD_OCC) void attn_fwd_fast_kernel(FwdArg
     // the row sum: one v_dot2 chain into l_run (the exponentials between its
     // links hide their latency; no chain registers to clear or add up)
     float psum = 0.0f;  // XB: the tile's sum before the rounding of P
-    auto less_max = [&](float s) { return XB ? xb.log2_less(s, c1, neg_m) : __builtin_fmaf(s, c1, neg_m); };
+    auto less_max = [&](float s) { return XB ? s + neg_m : __builtin_fmaf(s, c1, neg_m); };
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
@@ -458,15 +454,12 @@ bool fold_masks_ok(const Plan& plan) { return plan.max_len_k <= 64 * kFoldTiles;
 // Bias rows that are not 16-byte aligned (an odd number of keys) reach the
 // fast kernels only through the fragment-major copy, so every sample's bias
 // must be shared by its rows.  The generic kernels served these calls before,
-// and what they compute stays: the kernels add such a bias in float32 and
-// treat its non-finite elements the same way (ExactBias), which holds for
-// scales of this range.  Measured at 331 residues, 4 heads of 32, masked, bf16,
-// forward and backward: generic kernels 2363 us, this route 352 us (329 us with the bias weight and the row sum in 16 bits); at 127 MSA
-// rows x 277 tokens, 8 heads, float16, forward: 237 and 56 us (54).
-static bool unaligned_bias_ok(const oops_attn_geometry& geo, const Plan& plan) {
-  return plan.all_shared && geo.scale >= 0x1p-14f && geo.scale <= 1.0f;
-}
-
+// and what they compute stays: the kernels form their logits from such a bias
+// and treat its non-finite elements the same way (ExactBias).  Measured at 331
+// residues, 4 heads of 32, masked, bf16, forward and backward: generic kernels
+// 2363 us, this route 344 us (331 us with the bias weight and the row sum in
+// 16 bits); at 127 MSA rows x 277 tokens, 8 heads, float16, forward: 237 and
+// 56 us (55).
 bool exact_bias(const oops_attn_geometry& geo) { return bias_unaligned(geo); }
 
 bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan) {
@@ -475,7 +468,7 @@ bool fast_geometry_ok(const oops_attn_geometry& geo, const Plan& plan) {
       plan.any_bare || !geo.vec_ok || geo.head_size % 8 != 0 || !plan.offsets_32bit)
     return false;
   if (geo.has_bias && geo.bias_dtype != geo.dtype) return false;
-  return !bias_unaligned(geo) || unaligned_bias_ok(geo, plan);
+  return !bias_unaligned(geo) || plan.all_shared;
 }
 
 bool fast_path_ok(const oops_attn_geometry& geo, const Plan& plan) {

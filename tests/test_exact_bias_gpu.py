@@ -16,10 +16,10 @@ DEV = "cuda"
 NAMES = ("out", "dq", "dk", "dv", "dbias")
 
 
-def _run(case, shift=False):
+def _run(case, shift=False, scale=None):
     q, k, v, mask, bias, dout = case
     leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v, bias)]
-    out = triangle_attention(*leaves[:3], None if mask is None else mask.to(DEV), leaves[3])
+    out = triangle_attention(*leaves[:3], None if mask is None else mask.to(DEV), leaves[3], scale=scale)
     g = dout.to(DEV)
     if shift:  # dO off the 16-byte boundary
         flat = torch.empty(g.numel() + 1, dtype=g.dtype, device=DEV)[1:]
@@ -28,9 +28,9 @@ def _run(case, shift=False):
     return (out.detach(), *torch.autograd.grad(out, leaves, g))
 
 
-def _generic(case):
+def _generic(case, scale=None):
     with _core.force_generic():
-        return _run(case)
+        return _run(case, scale=scale)
 
 
 def _finite(tensors):
@@ -60,6 +60,23 @@ def test_finite_bias_of_any_size(dtype, rows, shift):
     _finite(got)
     # (the rows' logits have lost Q.K to float32's rounding of the bias: an equal weight for every key, and P = 1 in
     # the backward, whose LSE has lost the logarithm of their number)
+    torch.testing.assert_close(got[0], want[0], rtol=2e-2, atol=2e-2)
+    for name, a, b in zip(NAMES[1:], got[1:], want[1:]):
+        assert (a - b).float().norm() <= 1e-2 * b.float().norm(), name
+
+
+@pytest.mark.parametrize("rows,shift", [(3, False), (3, True), (400, False), (400, True)])
+@pytest.mark.parametrize("level", [0.3, -0.3, 0.49, -0.49, 0.69, -0.69])
+def test_passes_meet_at_large_logits(rows, shift, level):
+    """Whole rows at a level of the largest bfloat16: a unit in the last place of such a logit is more than exp2 can
+    take, so P = exp2(logit - LSE) needs the forward's and the backward's logits to have the same bits, whichever
+    kernels they come from."""
+
+    case = make_case(torch.bfloat16, prefix=(1,), rows=rows, cols=133, head=32, masked=True, seed=12)
+    case[4][0, 0, 0, 3:9] = torch.finfo(torch.bfloat16).max * level
+    got, want = _run(case, shift), _generic(case)
+    _finite(want)
+    _finite(got)
     torch.testing.assert_close(got[0], want[0], rtol=2e-2, atol=2e-2)
     for name, a, b in zip(NAMES[1:], got[1:], want[1:]):
         assert (a - b).float().norm() <= 1e-2 * b.float().norm(), name
@@ -118,3 +135,12 @@ def test_error_is_the_generic_kernels(dtype, head, spread):
         err, ref = ((t.double().cpu() - w).norm() / w.norm() for t in (a, g))
         print(f"{name}: {err:.3e}, generic {ref:.3e}")
         assert err <= 1.05 * ref, f"{name}: {err:.3e}, generic {ref:.3e}"
+
+
+@pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-6, 1.0, 2.5])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_any_scale(dtype, scale):
+    case = make_case(dtype, prefix=(1,), rows=200, cols=143, head=40, masked=True, seed=13)
+    got, want = _run(case, scale=scale), _generic(case, scale)
+    for name, a, b in zip(NAMES, got, want):  # (scale 0: dQ and dK are zeros)
+        assert (a - b).float().norm() <= 4 * torch.finfo(dtype).eps * b.float().norm(), name
