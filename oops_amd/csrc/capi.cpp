@@ -311,9 +311,9 @@ size_t workspace_bytes(const oops::Plan& plan) {
 // the bias copied by a launch of its own, which a small call does not repay:
 // the generic kernel walks a 32-key tile in about 3.3 us, so up to nine of
 // them (with up to three workgroups per CU at a time) end before the host has
-// enqueued the next call.  Measured back to back, generic against fast: 23.8
-// and 27.7 us at 127 residues, 27.0 and 27.4 at 32 MSA rows x 201 tokens, but
-// 40.1 and 27.7 at 151 residues, 41.7 and 27.7 at 385 single tokens.
+// enqueued the next call.  Measured back to back, generic against fast: 24.2
+// and 29.1 us at 127 residues, 27.3 and 28.5 at 32 MSA rows x 201 tokens, but
+// 40.1 and 28.6 at 151 residues, 41.7 and 28.7 at 385 single tokens.
 int make_forward_plan(const oops_attn_geometry* geo, oops::Plan& plan) {
   if (int rc = make_plan(geo, plan)) return rc;
   if (oops::bias_unaligned(*geo) && cdiv(plan.max_len_k, 32) * cdiv(plan.fwd_tiles, 768) <= 9) {
