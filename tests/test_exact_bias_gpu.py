@@ -144,3 +144,23 @@ def test_any_scale(dtype, scale):
     got, want = _run(case, scale=scale), _generic(case, scale)
     for name, a, b in zip(NAMES, got, want):  # (scale 0: dQ and dK are zeros)
         assert (a - b).float().norm() <= 4 * torch.finfo(dtype).eps * b.float().norm(), name
+
+
+@pytest.mark.parametrize("rows,shift", [(3, False), (400, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_nonfinite_bias_across_kernels(dtype, rows, shift):
+    """A generic forward before a fast backward and the other way round: the same elements are finite, with the
+    same values, as with generic kernels alone."""
+
+    case = make_case(dtype, prefix=(1,), rows=rows, cols=133, head=32, masked=True, seed=14)
+    bias, inf = case[4], float("inf")
+    bias[0, 0, 0, 3, ::2] = -inf
+    bias[0, 0, 0, 5] = -inf
+    bias[0, 0, 1, 6, 7] = inf
+    bias[0, 0, 1, 7, 0] = float("nan")
+    got, want = _run(case, shift), _generic(case)
+    for name, a, b in zip(NAMES, got, want):
+        assert torch.equal(a.isfinite(), b.isfinite()), name
+        kept = b.isfinite()
+        a, b = a.float()[kept], b.float()[kept]
+        assert (a - b).norm() <= 4 * torch.finfo(dtype).eps * b.norm(), name
